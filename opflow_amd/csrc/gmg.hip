@@ -782,32 +782,43 @@ __global__ __launch_bounds__(256) void k_pjacobi(GOp<T> o, const T* __restrict__
     xo[t] = yc + w * (b[t] - ay) / D;
 }
 
-// x = Cinv b in FP64 for the coarsest level: 16 lanes per row, each summing every 16th
-// column, the partial sums combined in a fixed order, so a row's reads are coalesced
-// and every thread of the block works (bv(c): b at column c)
+// rows row0 .. row1 - 1 of x = Cinv b in FP64 for the coarsest level: 16 lanes per row, each
+// summing every 16th column, the partial sums combined in a fixed order, so a row's reads are
+// coalesced and every thread of the block works (bv(c): b at column c)
 template <typename T, typename BV>
-__device__ __forceinline__ void dense_apply(const double* __restrict__ cinv, int n, BV bv, T* x) {
+__device__ __forceinline__ void dense_apply(const double* __restrict__ cinv, int n, int row0, int row1, BV bv, T* x) {
     const int lane = threadIdx.x & 15, groups = blockDim.x >> 4;
-    for (int row = threadIdx.x >> 4; row < n; row += groups) {  // the 16 lanes of a group share the row
+    for (int row = row0 + (threadIdx.x >> 4); row < row1; row += groups) {  // the 16 lanes of a group share the row
         const double* a = cinv + (long long)row * n;
         double s = 0;
-        for (int c = lane; c < n; c += 16) s += a[c] * bv(c);
+        int c = lane;
+        for (; c + 112 < n; c += 128) {  // eight loads in flight, summed in the loop's order
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = a[c + 16 * u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u] * bv(c + 16 * u);
+        }
+        for (; c < n; c += 16) s += a[c] * bv(c);
         for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 16);
         if (lane == 0) x[row] = (T)s;
     }
 }
 
-// coarsest level: x = Cinv b (FP64 inverse), one block per slot
+// coarsest level: x = Cinv b (FP64 inverse), 16 rows per block: the inverse of a level of 1000
+// cells is 8 MB, which one workgroup per slot took 987 us to read and 63 of them take 7 us
+constexpr int DENSE_ROWS = 16;
 template <typename T>
 __global__ __launch_bounds__(256) void k_dense(const double* __restrict__ cinv, int n, const T* __restrict__ b,
                                                T* __restrict__ x, Bat bt) {
     __shared__ double sb[1024];
     BAT_SLOT(bt);
+    const int row0 = blockIdx.x * DENSE_ROWS;
     b += (long long)slot * n;
     x += (long long)slot * n;
     for (int q = threadIdx.x; q < n; q += blockDim.x) sb[q] = (double)b[q];
     __syncthreads();
-    dense_apply<T>(cinv, n, [&](int c) { return sb[c]; }, x);
+    dense_apply<T>(cinv, n, row0, min(n, row0 + DENSE_ROWS), [&](int c) { return sb[c]; }, x);
 }
 
 
@@ -1253,7 +1264,7 @@ __global__ __launch_bounds__(GMG_TAIL_NT) void k_vtail(TailArgs<T> ta, Bat bt) {
     {  // coarsest: x = Cinv b in FP64
         const TailLevel<T>& L = ta.lv[ta.nl - 1];
         const T* bl = Bv(L);
-        dense_apply<T>(ta.cinv, ta.cN, [&](int c) { return (double)bl[c]; }, X(L));
+        dense_apply<T>(ta.cinv, ta.cN, 0, ta.cN, [&](int c) { return (double)bl[c]; }, X(L));
         __syncthreads();
     }
     for (int l = ta.nl - 2; l >= 0; --l) {  // up: prolongation, post-smoothing
@@ -1639,73 +1650,6 @@ static long long face_count(const int n[3], int d) {
     return (long long)(n[0] + (d == 0)) * (n[1] + (d == 1)) * (n[2] + (d == 2));
 }
 
-// dense operator of a level (host, FP64), for the coarsest solve
-static void dense_matrix(const Hierarchy& H, const GLevelHost& L, std::vector<double>& A) {
-    int n0 = L.n[0], n1 = L.n[1], n2 = L.n[2];
-    long long N = L.N;
-    A.assign(N * N, 0.0);
-    for (long long c = 0; c < N; ++c) {
-        int i = (int)(c % n0), j = (int)((c / n0) % n1), k = (int)(c / ((long long)n0 * n1));
-        int cc[3] = {i, j, k};
-        double D = L.var ? L.sg[c] : L.sigma;
-        for (int d = 0; d < H.dim; ++d) {
-            for (int s = 0; s < 2; ++s) {
-                int fc[3] = {i, j, k};
-                if (s == 1) fc[d] += 1;
-                double a = L.var ? L.af[d][face_index(d, fc[0], fc[1], fc[2], n0, n1)] : L.a[d];
-                int q[3] = {i, j, k};
-                q[d] += s == 0 ? -1 : 1;
-                bool inside = q[d] >= 0 && q[d] < L.n[d];
-                if (!inside && H.per[d]) {
-                    q[d] = q[d] < 0 ? L.n[d] - 1 : 0;
-                    inside = true;
-                }
-                if (inside) {
-                    D += a;
-                    long long nb = q[0] + (long long)n0 * (q[1] + (long long)n1 * q[2]);
-                    A[c * N + nb] -= a;
-                } else {
-                    D += a * (1.0 - H.alpha[d][s]);
-                }
-            }
-        }
-        (void)cc;
-        A[c * N + c] += D;
-    }
-}
-
-// Gauss-Jordan inverse with partial pivoting (small dense matrices)
-static bool invert(std::vector<double>& A, int n, std::vector<double>& inv) {
-    inv.assign((size_t)n * n, 0.0);
-    for (int i = 0; i < n; ++i) inv[(size_t)i * n + i] = 1.0;
-    for (int c = 0; c < n; ++c) {
-        int p = c;
-        for (int r = c + 1; r < n; ++r)
-            if (std::fabs(A[(size_t)r * n + c]) > std::fabs(A[(size_t)p * n + c])) p = r;
-        if (A[(size_t)p * n + c] == 0.0) return false;
-        if (p != c)
-            for (int k = 0; k < n; ++k) {
-                std::swap(A[(size_t)p * n + k], A[(size_t)c * n + k]);
-                std::swap(inv[(size_t)p * n + k], inv[(size_t)c * n + k]);
-            }
-        double d = 1.0 / A[(size_t)c * n + c];
-        for (int k = 0; k < n; ++k) {
-            A[(size_t)c * n + k] *= d;
-            inv[(size_t)c * n + k] *= d;
-        }
-        for (int r = 0; r < n; ++r) {
-            if (r == c) continue;
-            double f = A[(size_t)r * n + c];
-            if (f == 0.0) continue;
-            for (int k = 0; k < n; ++k) {
-                A[(size_t)r * n + k] -= f * A[(size_t)c * n + k];
-                inv[(size_t)r * n + k] -= f * inv[(size_t)c * n + k];
-            }
-        }
-    }
-    return true;
-}
-
 // the next coarser level's shape and constant-mode coefficients; its variable-mode
 // arrays too when `arrays` (host master copy)
 static void coarsen(const Hierarchy& H, const GLevelHost& F, GLevelHost& C, bool arrays = true) {
@@ -1796,27 +1740,6 @@ static int hier_levels(Hierarchy& H, const GLevelHost& fine, const int per[3], c
     return OPF_OK;
 }
 
-// dense inverse of the coarsest level (its arrays on the host in variable mode)
-// into H.cinv (allocated on first use)
-static int hier_coarsest(Hierarchy& H) {
-    const GLevelHost& Lc = H.host.back();
-    std::vector<double> A, inv;
-    dense_matrix(H, Lc, A);
-    if (H.singular) {
-        double dm = 0;
-        for (long long c = 0; c < Lc.N; ++c) dm += A[c * Lc.N + c];
-        dm /= (double)Lc.N * Lc.N;
-        for (auto& v : A) v += dm;
-    }
-    OPF_CHECK(invert(A, (int)Lc.N, inv), OPF_ERR_ARG, "gmg: singular coarsest operator");
-    if (!H.cinv) {
-        H.cN = (int)Lc.N;
-        OPF_TRY(alloc<double>((void**)&H.cinv, (long long)H.cN * H.cN, H.bytes));
-    }
-    OPF_HIP(hipMemcpy(H.cinv, inv.data(), sizeof(double) * inv.size(), hipMemcpyHostToDevice));
-    return OPF_OK;
-}
-
 // work vectors of every level (x, b below the finest, t), the Krylov vectors and
 // the scalars of the B slots
 static int hier_vectors(Hierarchy& H) {
@@ -1861,7 +1784,6 @@ int gmg_build(opf_ctx* ctx, Hierarchy& H, const GLevelHost& fine, const int per[
         for (double v : fine.sg) shift |= v != 0.0;
     OPF_TRY(hier_levels(H, fine, per, alpha, precision, slots, shift, true));
     H.bytes = 0;
-    OPF_TRY(hier_coarsest(H));
     // device levels
     H.dev.assign(H.host.size(), GLevelDev{});
     const bool mixed = precision == OPF_PREC_MIXED;
@@ -1894,9 +1816,8 @@ int gmg_build(opf_ctx* ctx, Hierarchy& H, const GLevelHost& fine, const int per[
             }
         }
     }
-    OPF_TRY(hier_vectors(H));
-    (void)ctx;
-    return OPF_OK;
+    OPF_TRY(coarse_inverse_dev(ctx->stream, H));
+    return hier_vectors(H);
 }
 
 int gmg_build_dev(opf_ctx* ctx, Hierarchy& H, const DevLevel& fine, const int per[3], const double alpha[3][2],
@@ -1975,19 +1896,7 @@ int gmg_build_dev(opf_ctx* ctx, Hierarchy& H, const DevLevel& fine, const int pe
             to_f32_dev(st, D.N, D.sg64, D.sg32);
         }
     OPF_HIP(hipGetLastError());
-    GLevelHost& Lc = H.host.back();
-    const GLevelDev& Dc = H.dev.back();
-    for (int d = 0; d < H.dim; ++d) {
-        Lc.af[d].resize(face_count(Lc.n, d));
-        OPF_HIP(hipMemcpyAsync(Lc.af[d].data(), Dc.af64[d], sizeof(double) * Lc.af[d].size(), hipMemcpyDeviceToHost, st));
-    }
-    Lc.sg.resize(Lc.N);
-    OPF_HIP(hipMemcpyAsync(Lc.sg.data(), Dc.sg64, sizeof(double) * Lc.N, hipMemcpyDeviceToHost, st));
-    OPF_HIP(hipStreamSynchronize(st));
-    int rc = hier_coarsest(H);
-    for (int d = 0; d < 3; ++d) std::vector<double>().swap(Lc.af[d]);
-    std::vector<double>().swap(Lc.sg);
-    return rc;
+    return coarse_inverse_dev(st, H);
 }
 
 void gmg_free(Hierarchy& H) {
@@ -2003,7 +1912,7 @@ void gmg_free(Hierarchy& H) {
         if (D.t) hipFree(D.t);
     }
     H.dev.clear();
-    void* ptrs[] = {H.cinv, H.r, H.z, H.p[0], H.p[1], H.q, H.e, H.r64, H.part, H.scal};
+    void* ptrs[] = {H.cinv, H.cwork, H.r, H.z, H.p[0], H.p[1], H.q, H.e, H.r64, H.part, H.scal};
     for (void* p : ptrs)
         if (p) hipFree(p);
     if (H.hscal) hipHostFree(H.hscal);
@@ -2013,7 +1922,7 @@ void gmg_free(Hierarchy& H) {
     H.iter_exec = nullptr;
     H.iter_graph = nullptr;
     H.mk = nullptr;
-    H.cinv = nullptr;
+    H.cinv = H.cwork = nullptr;
     H.r = H.z = H.p[0] = H.p[1] = H.q = H.e = nullptr;
     H.r64 = H.part = H.scal = H.hscal = nullptr;
 }
@@ -2133,7 +2042,8 @@ void ph_vcycle(const Hierarchy& H, hipStream_t st, const int* mask, int l, const
     const long long N = L.N;
     const unsigned B = (unsigned)H.B;
     if (l == (int)H.dev.size() - 1) {
-        hipLaunchKernelGGL(k_dense<T>, dim3(1, B), dim3(256), 0, st, H.cinv, H.cN, rhs, out, bat(H, mask, N));
+        hipLaunchKernelGGL(k_dense<T>, dim3((unsigned)((H.cN + DENSE_ROWS - 1) / DENSE_ROWS), B), dim3(256), 0, st, H.cinv,
+                           H.cN, rhs, out, bat(H, mask, N));
         if (dot_q)  // a one-level hierarchy: the dot products follow the dense solve
             hipLaunchKernelGGL(k_dot3<T>, dim3(red_count<T>(H), B), dim3(256), 0, st, N, rhs, (const T*)out, dot_q,
                                H.part, bat(H, mask, N));

@@ -89,8 +89,9 @@ struct Hierarchy {
     int pre = 2, post = 2;
     std::vector<GLevelHost> host;
     std::vector<GLevelDev> dev;
-    // coarsest dense inverse (FP64)
+    // coarsest dense inverse (FP64) and the scratch of its computation
     double* cinv = nullptr;
+    double* cwork = nullptr;
     int cN = 0;
     // Krylov vectors at level 0 (precision of the inner solve) and FP64 outer vectors
     void* r = nullptr;
@@ -143,6 +144,9 @@ void dev_level_free(DevLevel& L);
 void coarsen_dev(hipStream_t st, int dim, const int fn[3], const double* const faf[3], const double* fsg,
                  const int cn[3], double* const caf[3], double* csg);
 void to_f32_dev(hipStream_t st, long long n, const double* src, float* dst);
+// H.cinv = the dense inverse of the coarsest level from its device coefficients
+// (coarse.hip); ends with a wait for st
+int coarse_inverse_dev(hipStream_t st, Hierarchy& H);
 int read_scal(const Hierarchy& H, hipStream_t st);
 // Krylov solve with reliable updates, batched over the slots of H (vectors slot-major).
 // The Krylov vectors and the V-cycle are in precision T; x64 / b64 are the FP64
