@@ -1,27 +1,20 @@
 // FTCS heat update fast path:  u = u + coef * (d2x(u) + d2y(u) [+ d2z(u)])
 // (examples/FTCS2D/FTCS-OMP.cpp:26, D2SecondOrderCentered.hpp:160-171,
-//  FieldAssigner.hpp:26-86). One launch per step reads u^n (interior + ghosts)
-// and writes u^{n+1} together with the ghost values updatePadding would give
-// it, so the field is complete after every launch. On a uniform mesh the
-// reference's dx_l = dx_r = dx_c = h exactly, so D2 = ((r-c)/h - (c-l)/h)/h;
-// when h is a power of two the divisions are replaced by exact multiplications
-// by 1/h (same bits).
+//  FieldAssigner.hpp:26-86). A launch reads u^n and writes u^{n+k}; the field is
+// complete, its ghosts as updatePadding leaves them, after the call. On a uniform
+// mesh the reference's dx_l = dx_r = dx_c = h exactly, so D2 = ((r-c)/h - (c-l)/h)/h;
+// the divisions are replaced by cheaper operations that give the same bits (below).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
 
+#include "constdiv.hpp"
 #include "fastdiv.hpp"
 #include "opf_internal.hpp"
 
 using namespace opf;
 
 namespace {
-
-// storage index of cell q (interior origin 0, one ghost layer); z is padded only in 3-D
-template <int DIM>
-__host__ __device__ __forceinline__ long long ftcs_index(int e0, int e1, const int q[3]) {
-    return (q[0] + 1) + (long long)e0 * ((DIM >= 2 ? q[1] + 1 : 0) + (long long)e1 * (DIM == 3 ? q[2] + 1 : 0));
-}
 
 template <typename T>
 struct FtcsArgs {
@@ -31,9 +24,16 @@ struct FtcsArgs {
     T coefh;        // coef / h^2 (FTCS_FACTORED: exact, h a power of two)
     T hh[3];        // 1/h (FTCS_MUL, FTCS_FACTORED) or h (FTCS_DIV)
     int per[3];
-    int rtype[3][2];  // ghost rule per dim/side: 1 dirichlet, 2 neumann
+    int rtype[3][2];  // ghost rule per dim/side: RULE_*
     T rc1[3][2], rc2[3][2], rc3[3][2];
+    ConstDivisor cd[3];     // FTCS_CDIV: the spacings
+    ConstDivisor gd[3][2];  // RULE_CDIV: the divisors of the ghost rules
+    int gform;              // RULE_MUL when no side needs a division, else RULE_DIV
 };
+// v -> (rc1 v - rc2) / rc3 (Dirichlet) by division, by the multiplication with rc3's exact
+// reciprocal (rc3 a power of two: the same real number rounded once), or by const_div;
+// v + rc1 (Neumann)
+enum { RULE_NONE = 0, RULE_DIV = 1, RULE_ADD = 2, RULE_MUL = 3, RULE_CDIV = 4 };
 
 // Arithmetic modes of the update (all give the reference's bits):
 //  FTCS_DIV      D2 = ((r-c)/h - (c-l)/h)/h per dimension, as D2SecondOrderCentered computes it;
@@ -44,7 +44,18 @@ struct FtcsArgs {
 //                over dimensions keeps the common factor k^2, and coef * (k^2 S) =
 //                (coef k^2) * S with coef k^2 exact: u + coefh * (Dx + Dy [+ Dz]) with
 //                D = (r-c) - (c-l) -- 10 operations per 3-D cell instead of 19.
-enum { FTCS_DIV = 0, FTCS_MUL = 1, FTCS_FACTORED = 2 };
+//  FTCS_CDIV     any h: the divisions by h through its reciprocal (constdiv.hpp), where every
+//                value is in the range that needs; elsewhere FTCS_DIV's divisions.
+enum { FTCS_DIV = 0, FTCS_MUL = 1, FTCS_FACTORED = 2, FTCS_CDIV = 3 };
+
+// x / h of dim d in an arithmetic mode
+template <typename T, int MODE>
+__device__ __forceinline__ T over_h(T x, const FtcsArgs<T>& a, int d) {
+    if constexpr (MODE == FTCS_FACTORED) return x;
+    else if constexpr (MODE == FTCS_MUL) return x * a.hh[d];
+    else if constexpr (MODE == FTCS_CDIV) return const_div(x, a.cd[d]);
+    else return x / a.hh[d];
+}
 
 template <typename T, int MODE>
 __device__ __forceinline__ T d2(T l, T c, T r, T hh) {
@@ -52,12 +63,7 @@ __device__ __forceinline__ T d2(T l, T c, T r, T hh) {
     else return ((r - c) / hh - (c - l) / hh) / hh;
 }
 
-// u^{n+1} at one cell from its value and its x / y (/ z) neighbours
-template <typename T, int MODE>
-__device__ __forceinline__ T ftcs2(T c, T xl, T xr, T yl, T yr, const FtcsArgs<T>& a) {
-    if constexpr (MODE == FTCS_FACTORED) return c + a.coefh * (((xr - c) - (c - xl)) + ((yr - c) - (c - yl)));
-    else return c + a.coef * (d2<T, MODE>(xl, c, xr, a.hh[0]) + d2<T, MODE>(yl, c, yr, a.hh[1]));
-}
+// u^{n+1} at one cell of a 3-D field from its value and its x / y / z neighbours
 template <typename T, int MODE>
 __device__ __forceinline__ T ftcs3(T c, T xl, T xr, T yl, T yr, T zl, T zr, const FtcsArgs<T>& a) {
     if constexpr (MODE == FTCS_FACTORED) {
@@ -73,155 +79,314 @@ __device__ __forceinline__ T ftcs3(T c, T xl, T xr, T yl, T yr, T zl, T zr, cons
 
 template <typename T>
 __device__ __forceinline__ T rule(const FtcsArgs<T>& a, int d, int s, T v) {
-    int t = a.rtype[d][s];
-    if (t == 1) return (a.rc1[d][s] * v - a.rc2[d][s]) / a.rc3[d][s];
-    if (t == 2) return v + a.rc1[d][s];
-    return v;
+    const int t = a.rtype[d][s];
+    if (t == RULE_ADD) return v + a.rc1[d][s];
+    if (t == RULE_NONE) return v;
+    const T x = a.rc1[d][s] * v - a.rc2[d][s];
+    if (t == RULE_MUL) return x * a.rc3[d][s];
+    return x / a.rc3[d][s];
 }
 
-// Write the ghost images whose source is interior cell p (value v), in the
-// closed form of updatePaddingImpl_final for one ghost layer.
-template <typename T, int DIM>
-__device__ __forceinline__ void write_images(T* __restrict__ out, const FtcsArgs<T>& a, const int p[3], T v) {
-    int lo[3], hi[3];  // is p the source of the lower / upper ghost of dim d
-    bool any = false;
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        if (a.per[d]) {
-            lo[d] = p[d] == a.n[d] - 1;
-            hi[d] = p[d] == 0;
-        } else {
-            lo[d] = p[d] == 0;
-            hi[d] = p[d] == a.n[d] - 1;
-        }
-        any |= lo[d] | hi[d];
-    }
-    if (!any) return;
-    constexpr int NC = DIM == 1 ? 3 : DIM == 2 ? 9 : 27;
-    for (int c = 1; c < NC; ++c) {
-        int ch[3] = {c % 3, (c / 3) % 3, c / 9};
-        int q[3] = {p[0], p[1], p[2]};
-        T w = v;
-        bool ok = true;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            if (ch[d] == 0) continue;
-            int s = ch[d] - 1;
-            if (!(s == 0 ? lo[d] : hi[d])) { ok = false; break; }
-            q[d] = s == 0 ? -1 : a.n[d];
-            if (!a.per[d]) w = rule(a, d, s, w);
-        }
-        if (!ok) continue;
-        out[ftcs_index<DIM>(a.e0, a.e1, q)] = w;
-    }
-}
-
-// 2-D: one cell per thread, block 64 x 4.
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) void ftcs2d_kernel(const T* __restrict__ in, T* __restrict__ out, FtcsArgs<T> a) {
-    int i = blockIdx.x * 64 + threadIdx.x;
-    int j = blockIdx.y * 4 + threadIdx.y;
-    if (i >= a.n[0] || j >= a.n[1]) return;
-    long long l = (i + 1) + (long long)a.e0 * (j + 1);
-    T c = in[l];
-    T v = ftcs2<T, MODE>(c, in[l - 1], in[l + 1], in[l - a.e0], in[l + a.e0], a);
-    out[l] = v;
-    int p[3] = {i, j, 0};
-    write_images<T, 2>(out, a, p, v);
-}
-
-
-// 2-D temporal blocking: one workgroup advances a TS x TS output tile by `nt`
-// (<= TB) steps inside LDS, from a region padded by TB cells per side (clamped
-// to the ghost layer on non-periodic sides, wrapped on periodic ones). Every
-// step recomputes all region cells whose stencil lies inside the region; the
-// values at distance < s from an open region edge go stale, which never reaches
-// the tile. Ghost cells inside the region are refilled from the fresh interior
-// with the BC rules, x first then y (the corner composition of updatePadding).
-// Same arithmetic per cell and step as ftcs2d_kernel, so the bits are equal.
-template <int TS, int TB>
-struct Ftcs2dTile {
-    static constexpr int W = TS + 2 * TB;
+// The ghost rules of a launch in one form, (c1 v - c2) over c3 with c1 = c3 = 1 where the rule only
+// adds (both exact): over c3 a multiplication by its exact reciprocal, a const_div or a division.
+// One straight line for every side, so that the lanes of a wave take theirs together.
+template <typename T>
+struct SideRule {
+    T c1, c2, c3;
+    ConstDivisor cd;
 };
+template <typename T>
+__device__ __forceinline__ SideRule<T> side_rule(const FtcsArgs<T>& a, int d, int s) {
+    const int t = a.rtype[d][s];
+    SideRule<T> r{T(1), T(0), T(1), {}};
+    if (t == RULE_ADD) r.c2 = -a.rc1[d][s];
+    if (t == RULE_DIV || t == RULE_MUL || t == RULE_CDIV) r.c1 = a.rc1[d][s], r.c2 = a.rc2[d][s], r.c3 = a.rc3[d][s];
+    if (t == RULE_CDIV) r.cd = a.gd[d][s];
+    return r;
+}
+// again: RULE_CDIV met a value outside const_div's range
+template <int FORM, typename T>
+__device__ __forceinline__ T ghost_value(T c1, T c2, T c3, double h, double y, T v, bool& again) {
+    const T x = c1 * v - c2;
+    if constexpr (FORM == RULE_MUL) return x * c3;
+    else if constexpr (FORM == RULE_DIV) return x / c3;
+    else {
+        const T q = const_div(x, ConstDivisor{h, y});
+        if constexpr (sizeof(T) == 4) again |= div_subnormal(q);
+        else again |= div_key(v) < kDivLow;
+        return c3 < T(0) ? -q : q;  // h = |c3|
+    }
+}
 
-template <typename T, int MODE, int TS, int TB>
-__global__ __launch_bounds__(256) void ftcs2d_tb_kernel(const T* __restrict__ in, T* __restrict__ out, FtcsArgs<T> a,
-                                                        int nt) {
-    constexpr int W = Ftcs2dTile<TS, TB>::W;
-    __shared__ T buf[2][W][W];
-    const int tilesx = (a.n[0] + TS - 1) / TS;
+// the value of the next / previous lane of the wave (0 in the last / first lane)
+template <int CTRL>
+__device__ __forceinline__ int dpp32(int v) {
+    return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL, typename T>
+__device__ __forceinline__ T dpp(T v) {
+    if constexpr (sizeof(T) == 4) return __int_as_float(dpp32<CTRL>(__float_as_int(v)));
+    else return __hiloint2double(dpp32<CTRL>(__double2hiint(v)), dpp32<CTRL>(__double2loint(v)));
+}
+// c ? x : y of two loaded values (a conditional between array elements would pick an address and
+// put the array in memory)
+template <typename T>
+__device__ __forceinline__ T pick(bool c, T x, T y) {
+    return c ? x : y;
+}
+template <typename T>
+__device__ __forceinline__ T lane_next(T v) { return dpp<0x130>(v); }
+template <typename T>
+__device__ __forceinline__ T lane_prev(T v) { return dpp<0x138>(v); }
+
+// 2-D steps in registers. A workgroup holds a region of 64 XW x NW RW cells: lane l of a wave
+// the XW neighbouring cells l XW .. in x, wave w the RW rows w RW .., so that y neighbours are
+// registers, x neighbours are registers or one lane away (DPP, no LDS), and only the first and
+// last row of each wave pass through LDS, with one barrier a step. It advances the region nt
+// steps and writes the tx x ty tile in its middle; the values at distance < s from an open region
+// edge are stale after s steps, which never reaches the tile. A difference of neighbours, and its
+// quotient by h, is formed once and serves both cells. On a non-periodic side the region starts
+// at, or contains, the ghost layer, which is refilled after every step from the fresh cells with
+// the BC rules, x first, then y (the corner composition of updatePadding); the rows are placed so
+// that a y ghost and its source cell belong to one wave. Periodic sides read wrapped cells. The
+// tile's ghost images are written with it, so the output field is complete.
+// Per cell and step the operations and their order are those of D2 in the reference, so the bits
+// are too. FP64 issue bounds the large grids (7 operations and 2 lane moves a cell and step, 19 and
+// 2 with const_div, over the share of the region that is tile), the barrier and the launch the
+// small ones. Against LDS tiles of the values (32 x 32, 4 steps; 8 x 8, 5 steps): 256^2 Dirichlet
+// 1.61 -> 0.75 us a step, 1500 x 1100 with const_div 12.3 -> 4.5 (0.13 -> 0.37 T cell-updates/s),
+// 4096^2 periodic 42 -> 10.1 (0.40 -> 1.66 T/s).
+template <typename T, int MODE, int XW, int RW, int NW>
+__global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restrict__ in, T* __restrict__ out,
+                                                               FtcsArgs<T> a, int nt, int tx, int ty) {
+    static_assert(XW <= 2, "the ghost columns are a lane's first or second");
+    constexpr int WX = 64 * XW, WY = RW * NW;
+    __shared__ T edge[2][NW][2][XW][64];  // first and last row of every wave, double-buffered
+    const int n0 = a.n[0], n1 = a.n[1];
+    const int tilesx = (n0 + tx - 1) / tx;
     const int tb = (int)xcd_block(blockIdx.x, gridDim.x);  // x-neighbouring tiles share an XCD's L2
-    const int x0 = (tb % tilesx) * TS, y0 = (tb / tilesx) * TS;
-    // region origin in global cell coordinates; non-periodic sides clamp to the ghost layer
-    int lo[2], hi[2];
-    const int org[2] = {x0, y0};
-    for (int d = 0; d < 2; ++d) {
-        lo[d] = org[d] - TB;
-        hi[d] = org[d] + TS + TB;
-        if (!a.per[d]) {
-            lo[d] = max(lo[d], -1);
-            hi[d] = min(hi[d], a.n[d] + 1);
+    const int x0 = (tb % tilesx) * tx, y0 = (tb / tilesx) * ty;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // region origin; non-periodic sides: x from the ghost column on, y from the ghost row or up to it
+    int lox = x0 - nt, loy = y0 - nt;
+    if (!a.per[0]) lox = max(lox, -1);
+    if (!a.per[1]) {
+        loy = max(loy, -1);
+        if (loy + WY > n1 + 1) {
+            loy = n1 + 1 - WY;  // the upper ghost row is the last of the last wave
+            if (loy < -1) loy = (n1 + 1) % RW == 0 ? -2 : -1;  // both ghost rows inside
         }
     }
-    const int wx = hi[0] - lo[0], wy = hi[1] - lo[1];
-    auto gidx = [&](int gx, int gy) -> long long {
-        if (a.per[0]) gx = ((gx % a.n[0]) + a.n[0]) % a.n[0];
-        if (a.per[1]) gy = ((gy % a.n[1]) + a.n[1]) % a.n[1];
-        return (gx + 1) + (long long)a.e0 * (gy + 1);
+    const int gx0 = lox + lane * XW, gy0 = loy + w * RW;
+    T u[RW][XW];
+    {
+        int ox[XW];
+#pragma unroll
+        for (int k = 0; k < XW; ++k) {
+            int gx = gx0 + k;
+            if (a.per[0]) gx = ((gx % n0) + n0) % n0;
+            ox[k] = min(max(gx, -1), n0) + 1;
+        }
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            int gy = gy0 + r;
+            if (a.per[1]) gy = ((gy % n1) + n1) % n1;
+            const T* row = in + (long long)a.e0 * (min(max(gy, -1), n1) + 1);
+#pragma unroll
+            for (int k = 0; k < XW; ++k) u[r][k] = row[ox[k]];
+        }
+    }
+    // the ghosts of this wave: columns (uniform over the workgroup), rows (of this wave)
+    const bool xlo = !a.per[0] && lox <= -1, xhi = !a.per[0] && lox + WX > n0;
+    const int rlo = a.per[1] ? -1 : -1 - gy0, rhi = a.per[1] ? -1 : n1 - gy0;
+    const bool ylo = rlo >= 0 && rlo < RW, yhi = rhi >= 0 && rhi < RW;
+    const bool ghosts = xlo || xhi || ylo || yhi;
+    constexpr int FORM = MODE == FTCS_CDIV ? RULE_CDIV : MODE == FTCS_DIV ? RULE_DIV : RULE_MUL;
+    // x rule of this lane's column (a lane holds at most one ghost column of each side)
+    const bool hilane = gx0 + XW > n0;
+    const SideRule<T> rl = side_rule(a, 0, 0), rh = side_rule(a, 0, 1), ryl = side_rule(a, 1, 0), ryh = side_rule(a, 1, 1);
+    const T xc1 = hilane ? rh.c1 : rl.c1, xc2 = hilane ? rh.c2 : rl.c2, xc3 = hilane ? rh.c3 : rl.c3;
+    const double xh = hilane ? rh.cd.h : rl.cd.h, xy = hilane ? rh.cd.y : rl.cd.y;
+    // refills the ghosts of v; true when RULE_CDIV met a value out of its range (v is unchanged then)
+    auto refill = [&](auto F, T(&v)[RW][XW]) __attribute__((always_inline)) -> bool {
+        constexpr int FM = decltype(F)::value;
+        bool again = false;
+        if (xlo || xhi) {
+            // the lower ghost is a lane's first column, its source the next one; the upper ghost's
+            // source the previous column
+            T g[RW][XW];
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                const T nx = XW > 1 ? v[r][XW > 1 ? 1 : 0] : lane_next(v[r][0]);
+                const T pv = lane_prev(v[r][XW - 1]);
+                g[r][0] = ghost_value<FM>(xc1, xc2, xc3, xh, xy, hilane ? pv : nx, again);
+                if constexpr (XW > 1) g[r][1] = ghost_value<FM>(xc1, xc2, xc3, xh, xy, v[r][0], again);
+            }
+            if (FM == RULE_CDIV && __any(again)) return true;
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                v[r][0] = pick(gx0 == -1 || gx0 == n0, g[r][0], v[r][0]);
+                if constexpr (XW > 1) v[r][1] = pick(gx0 + 1 == n0, g[r][1], v[r][1]);
+            }
+        }
+        if (ylo) {
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                T src = v[1][k];
+#pragma unroll
+                for (int r = 1; r + 1 < RW; ++r) src = pick(r == rlo, v[r + 1][k], src);
+                T g = ghost_value<FM>(ryl.c1, ryl.c2, ryl.c3, ryl.cd.h, ryl.cd.y, src, again);
+                if (FM == RULE_CDIV && __any(again)) g = ghost_value<RULE_DIV>(ryl.c1, ryl.c2, ryl.c3, 1., 1., src, again);
+#pragma unroll
+                for (int r = 0; r + 1 < RW; ++r) v[r][k] = pick(r == rlo, g, v[r][k]);
+            }
+        }
+        if (yhi) {
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                T src = v[0][k];
+#pragma unroll
+                for (int r = 2; r < RW; ++r) src = pick(r == rhi, v[r - 1][k], src);
+                T g = ghost_value<FM>(ryh.c1, ryh.c2, ryh.c3, ryh.cd.h, ryh.cd.y, src, again);
+                if (FM == RULE_CDIV && __any(again)) g = ghost_value<RULE_DIV>(ryh.c1, ryh.c2, ryh.c3, 1., 1., src, again);
+#pragma unroll
+                for (int r = 1; r < RW; ++r) v[r][k] = pick(r == rhi, g, v[r][k]);
+            }
+        }
+        return false;
     };
-    // positions walk the full W x W square (a compile-time divisor); clamped regions skip the rest
-    for (int t = threadIdx.x; t < W * W; t += blockDim.x) {
-        const int lx = t % W, ly = t / W;
-        if (lx >= wx || ly >= wy) continue;
-        buf[0][ly][lx] = in[gidx(lo[0] + lx, lo[1] + ly)];
+    bool slow = false;  // FTCS_CDIV, FP64: a value outside the range for the whole launch
+    if constexpr (MODE == FTCS_CDIV && sizeof(T) == 8) {
+        bool bad = false;
+#pragma unroll
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+            for (int k = 0; k < XW; ++k) bad |= div_unsafe(u[r][k]);
+        slow = __syncthreads_or(bad);
     }
-    __syncthreads();
-    int cur = 0;
     for (int s = 0; s < nt; ++s) {
-        const int nxt = 1 - cur;
-        // interior cells with all four neighbours inside the region
-        for (int t = threadIdx.x; t < W * W; t += blockDim.x) {
-            const int lx = t % W, ly = t / W;
-            if (lx >= wx || ly >= wy) continue;
-            int gx = lo[0] + lx, gy = lo[1] + ly;
-            bool inx = a.per[0] || (gx >= 0 && gx < a.n[0]);
-            bool iny = a.per[1] || (gy >= 0 && gy < a.n[1]);
-            if (!inx || !iny || lx == 0 || ly == 0 || lx == wx - 1 || ly == wy - 1) continue;
-            T c = buf[cur][ly][lx];
-            T v = ftcs2<T, MODE>(c, buf[cur][ly][lx - 1], buf[cur][ly][lx + 1], buf[cur][ly - 1][lx],
-                                 buf[cur][ly + 1][lx], a);
-            buf[nxt][ly][lx] = v;
-        }
-        __syncthreads();
-        // ghosts of non-periodic x sides (rows inside the y interior), then y sides (all
-        // columns); only tiles whose region reaches a non-periodic side have any (a
-        // condition uniform over the workgroup, so the barriers stay uniform)
-        if (!a.per[0] && (lo[0] == -1 || hi[0] == a.n[0] + 1)) {
-            for (int ly = threadIdx.x; ly < wy; ly += blockDim.x) {
-                int gy = lo[1] + ly;
-                if (!a.per[1] && (gy < 0 || gy >= a.n[1])) continue;
-                if (lo[0] == -1) buf[nxt][ly][0] = rule(a, 0, 0, buf[nxt][ly][1]);
-                if (hi[0] == a.n[0] + 1) buf[nxt][ly][wx - 1] = rule(a, 0, 1, buf[nxt][ly][wx - 2]);
+        auto& e = edge[s & 1];
+        if constexpr (NW > 1) {
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                e[w][0][k][lane] = u[0][k];
+                e[w][1][k][lane] = u[RW - 1][k];
             }
-            __syncthreads();
         }
-        if (!a.per[1] && (lo[1] == -1 || hi[1] == a.n[1] + 1)) {
-            for (int lx = threadIdx.x; lx < wx; lx += blockDim.x) {
-                if (lo[1] == -1) buf[nxt][0][lx] = rule(a, 1, 0, buf[nxt][1][lx]);
-                if (hi[1] == a.n[1] + 1) buf[nxt][wy - 1][lx] = rule(a, 1, 1, buf[nxt][wy - 2][lx]);
+        T v[RW][XW];  // the second x differences, then the new values
+        // returns whether a float quotient was subnormal
+        auto xpart = [&](auto M) __attribute__((always_inline)) -> bool {
+            constexpr int MD = decltype(M)::value;
+            bool sub = false;
+            auto quo = [&](T x) __attribute__((always_inline)) -> T {
+                const T q = over_h<T, MD>(x, a, 0);
+                if constexpr (MD == FTCS_CDIV && sizeof(T) == 4) sub |= div_subnormal(q);
+                return q;
+            };
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                T qx[XW];
+#pragma unroll
+                for (int k = 0; k < XW; ++k) {
+                    const T right = k + 1 < XW ? u[r][k + 1 < XW ? k + 1 : 0] : lane_next(u[r][0]);
+                    qx[k] = quo(right - u[r][k]);
+                }
+                const T left = lane_prev(qx[XW - 1]);
+#pragma unroll
+                for (int k = 0; k < XW; ++k) v[r][k] = quo(qx[k] - (k > 0 ? qx[k > 0 ? k - 1 : 0] : left));
             }
+            return sub;
+        };
+        T dn[XW], up[XW];  // the rows before the first and after the last
+        auto ypart = [&](auto M) __attribute__((always_inline)) -> bool {
+            constexpr int MD = decltype(M)::value;
+            bool sub = false;
+            auto quo = [&](T x) __attribute__((always_inline)) -> T {
+                const T q = over_h<T, MD>(x, a, 1);
+                if constexpr (MD == FTCS_CDIV && sizeof(T) == 4) sub |= div_subnormal(q);
+                return q;
+            };
+            T qy[XW];
+#pragma unroll
+            for (int k = 0; k < XW; ++k) qy[k] = quo(u[0][k] - dn[k]);
+#pragma unroll
+            for (int r = 0; r < RW; ++r)
+#pragma unroll
+                for (int k = 0; k < XW; ++k) {
+                    const T qn = quo((r + 1 < RW ? u[r + 1 < RW ? r + 1 : 0][k] : up[k]) - u[r][k]);
+                    const T dy = quo(qn - qy[k]);
+                    qy[k] = qn;
+                    v[r][k] = u[r][k] + (MD == FTCS_FACTORED ? a.coefh : a.coef) * (v[r][k] + dy);
+                }
+            return sub;
+        };
+        bool sub = xpart(std::integral_constant<int, MODE>{});  // needs no other wave: while the rows are on their way
+        if constexpr (NW > 1) {
             __syncthreads();
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                dn[k] = e[max(w - 1, 0)][1][k][lane];
+                up[k] = e[min(w + 1, NW - 1)][0][k][lane];
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < XW; ++k) dn[k] = u[0][k], up[k] = u[RW - 1][k];
         }
-        cur = nxt;
+        bool again = slow;
+        if constexpr (MODE == FTCS_CDIV && sizeof(T) == 8) {
+            unsigned m = 0xffffffffu;
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                m = min(m, min(div_key(dn[k]), div_key(up[k])));
+#pragma unroll
+                for (int r = 0; r < RW; ++r) m = min(m, div_key(u[r][k]));
+            }
+            again |= __any(m < kDivLow);
+        }
+        if (!again) sub |= ypart(std::integral_constant<int, MODE>{});
+        if constexpr (MODE == FTCS_CDIV) {
+            if (sizeof(T) == 4) again = __any(sub);
+            if (again) {
+                xpart(std::integral_constant<int, FTCS_DIV>{});
+                ypart(std::integral_constant<int, FTCS_DIV>{});
+            }
+        }
+        if (ghosts) {
+            bool done = false;
+            if (FORM == RULE_MUL && a.gform == RULE_MUL) done = !refill(std::integral_constant<int, RULE_MUL>{}, v);
+            else if (FORM == RULE_CDIV && !again) done = !refill(std::integral_constant<int, RULE_CDIV>{}, v);
+            if (!done) refill(std::integral_constant<int, RULE_DIV>{}, v);
+        }
+#pragma unroll
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+            for (int k = 0; k < XW; ++k) u[r][k] = v[r][k];
     }
-    // write the tile and the ghost images it is the source of
-    for (int t = threadIdx.x; t < TS * TS; t += blockDim.x) {
-        int i = x0 + t % TS, j = y0 + t / TS;
-        if (i >= a.n[0] || j >= a.n[1]) continue;
-        T v = buf[cur][j - lo[1]][i - lo[0]];
-        int p[3] = {i, j, 0};
-        out[ftcs_index<2>(a.e0, a.e1, p)] = v;
-        write_images<T, 2>(out, a, p, v);
+    // the tile with the ghost positions beyond it: its own columns and, on non-periodic sides, the
+    // ghost columns; periodic images of the first and last column and row
+    const int x1 = min(x0 + tx, n0), y1 = min(y0 + ty, n1);
+    const int xa = !a.per[0] && x0 == 0 ? -1 : x0, xb = !a.per[0] && x1 == n0 ? n0 + 1 : x1;
+    const int ya = !a.per[1] && y0 == 0 ? -1 : y0, yb = !a.per[1] && y1 == n1 ? n1 + 1 : y1;
+    const bool imlo = a.per[0] && x1 == n0, imhi = a.per[0] && x0 == 0;  // images at -1 and at n
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        const int gy = gy0 + r;
+        if (gy < ya || gy >= yb) continue;
+        auto put = [&](int y) __attribute__((always_inline)) {
+            T* row = out + (long long)a.e0 * (y + 1) + 1;
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                const int gx = gx0 + k;
+                if (gx >= xa && gx < xb) row[gx] = u[r][k];
+                if (imlo && gx == n0 - 1) row[-1] = u[r][k];
+                if (imhi && gx == 0) row[n0] = u[r][k];
+            }
+        };
+        put(gy);
+        if (a.per[1]) {
+            if (gy == n1 - 1) put(-1);
+            if (gy == 0) put(n1);
+        }
     }
 }
 
@@ -473,18 +638,52 @@ __global__ __launch_bounds__(NT) void ftcs3d_tb_kernel(const T* __restrict__ in,
     }
 }
 
-// launch shapes: 2-D tiles of FT_TS2^2 cells advanced FT_TB2 steps per launch
-// (swept at 1024^2..4096^2: 32x32 with 4 steps beat 2, 3, 5, 6, 8 and 10 steps
-// and 16..64-cell tiles; 4096^2 FP64 288 -> 390 G cell-updates/s against 8 steps);
-// grids with fewer than 512 such tiles use FT_TS2S^2 tiles and FT_TB2S steps, so
-// that every CU gets several workgroups (256^2 FP64 x 1000 steps: 16x16/8 2.06 ms,
-// 8x8/5 1.73 ms; 8x8 with 3..7 steps and 4x4 / 12x12 tiles were slower)
-constexpr int FT_TS2 = 32, FT_TB2 = 4, FT_TS2S = 8, FT_TB2S = 5;
+// Launches of the 2-D kernel: the region (cells in x per lane, rows per wave, waves), the steps per
+// launch and the tile that is left of the region. Per step a launch costs
+//   S2_LAUNCH / nt + max(alone, tiles / CUs * shared)
+// with the measured time of one step of one workgroup when it has a CU to itself (alone: the
+// barrier and the waves' latency) and when several share one (shared: instruction issue), about
+// 1.8 times that with const_div. More steps a launch save launches and lose tile. FP64, us per
+// step: 256^2 periodic 64 x 32 region with 12 steps 0.65 (64 x 64, 24 steps: 0.71); 700^2 64 x 64,
+// 10 steps 2.0 (64 x 32, 6: 2.1); 4096^2 128 x 64, 10 steps 10.1 (64 x 64: 14.0, 64 x 32: 19.8).
+// With const_div the 128 x 64 region holds too few waves (117 registers): 2000^2 7.7 against 7.3.
+constexpr int S2_XW[3] = {1, 1, 2}, S2_RW[3] = {4, 8, 8}, S2_NW[3] = {8, 8, 8};
+constexpr double S2_ALONE[3] = {0.33, 0.55, 1.3}, S2_SHARED[3] = {0.31, 0.49, 0.74}, S2_LAUNCH = 4.2;
+constexpr int S2_MOST = 128;  // steps a launch takes at most (the range const_div is given, div_range)
+struct Strip2d {
+    int cfg = 0;
+    int nt = 1, tx = 1, ty = 1;  // steps, tile
+};
 
-// steps per launch of the 2-D blocked kernel for an n[0] x n[1] grid
-inline int tb2_steps(const int n[3]) {
-    const int tiles = ((n[0] + FT_TS2 - 1) / FT_TS2) * ((n[1] + FT_TS2 - 1) / FT_TS2);
-    return tiles < 512 ? FT_TB2S : FT_TB2;
+Strip2d strip_plan(const int n[3], const int per[3], int nsteps, int tblock, bool div, int cus) {
+    Strip2d best;
+    double cost = 0;
+    for (int c = 0; c < (div ? 2 : 3); ++c) {
+        const int wx = 64 * S2_XW[c], wy = S2_RW[c] * S2_NW[c];
+        const bool allx = !per[0] && n[0] + 2 <= wx, ally = !per[1] && n[1] + 3 <= wy;  // no halo in that dim
+        const int most = std::min(nsteps, allx && ally ? S2_MOST : (ally ? wx : allx ? wy : std::min(wx, wy)) / 2 - 2);
+        // 1 (when asked for), else 2, 3 .. 12, 24, .. and the most
+        for (int nt = tblock == 1 ? 1 : std::min(2, most);;) {
+            const int tx = allx ? n[0] : wx - 2 * nt, ty = ally ? n[1] : wy - 2 * nt;
+            const double tiles = (double)((n[0] + tx - 1) / tx) * ((n[1] + ty - 1) / ty);
+            const double t = S2_LAUNCH / nt +
+                             (div ? 1.8 : 1.0) * std::max(S2_ALONE[c], tiles / cus * S2_SHARED[c]);
+            if (cost == 0 || t < cost) {
+                cost = t;
+                best.cfg = c;
+                best.nt = nt;
+            }
+            if (tblock == 1 || nt >= most) break;
+            nt = std::min(most, nt < 12 ? nt + 1 : 2 * nt);
+        }
+    }
+    // the steps spread evenly over that many launches
+    const int launches = (nsteps + best.nt - 1) / best.nt;
+    best.nt = (nsteps + launches - 1) / launches;
+    const int wx = 64 * S2_XW[best.cfg], wy = S2_RW[best.cfg] * S2_NW[best.cfg];
+    best.tx = !per[0] && n[0] + 2 <= wx ? n[0] : wx - 2 * best.nt;
+    best.ty = !per[1] && n[1] + 3 <= wy ? n[1] : wy - 2 * best.nt;
+    return best;
 }
 
 // 3-D blocked launch shape per precision (swept at 512^3 on MI355X): TX x TY
@@ -504,19 +703,10 @@ struct Ftcs3dCfg<float> {
     static constexpr bool XCD = true;
 };
 
-// Steps the next launch advances: the launch plan shared by the sweep and
-// opf_ftcs_plan. tblock = 1 forces single steps.
-int launch_steps(int dim, int dtype, const int n[3], const int per[3], long long plane, int remaining, int tblock) {
-    if (tblock == 1) return 1;
-    if (dim == 2) {
-        const int tb = tb2_steps(n);
-        if (remaining >= 2 && n[0] >= tb && n[1] >= tb) return std::min(tb, remaining);
-        return 1;
-    }
+// Steps the next launch of a 3-D field advances. tblock = 1 forces single steps.
+int launch_steps3(int dtype, long long plane, int remaining, int tblock) {
     const int k3 = dtype == OPF_F64 ? Ftcs3dCfg<double>::K : Ftcs3dCfg<float>::K;
-    (void)per;
-    if (dim == 3 && plane < (1LL << 31) && remaining >= 2) return std::min(k3, remaining);
-    return 1;
+    return tblock != 1 && plane < (1LL << 31) && remaining >= 2 ? std::min(k3, remaining) : 1;
 }
 
 bool is_pow2(double h) {
@@ -557,7 +747,7 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
             OPF_CHECK(t == OPF_BC_DIRC || t == OPF_BC_NEUM || t == OPF_BC_PERIODIC, OPF_ERR_UNSUPPORTED,
                       "ftcs: bc %d unsupported", t);
             const GhostRule& r = gi.rule[q][s][0];
-            a.rtype[q][s] = r.type;
+            a.rtype[q][s] = r.type == 1 ? RULE_DIV : r.type == 2 ? RULE_ADD : RULE_NONE;
             a.rc1[q][s] = (T)r.c1;
             a.rc2[q][s] = (T)r.c2;
             a.rc3[q][s] = (T)r.c3;
@@ -569,7 +759,41 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
     }
     bool same = true;
     for (int q = 1; q < d.dim; ++q) same &= m->h[q] == m->h[0];
-    const int mode = !pow2 ? FTCS_DIV : same ? FTCS_FACTORED : FTCS_MUL;
+    int mode = !pow2 ? FTCS_DIV : same ? FTCS_FACTORED : FTCS_MUL;
+    if (mode == FTCS_DIV && d.dim == 2) {
+        bool ok = std::is_same<T, float>::value || div_range(m->h, d.dim, coef, S2_MOST);
+        for (int q = 0; q < d.dim; ++q) {
+            a.cd[q].h = (double)a.hh[q];
+            a.cd[q].y = 1.0 / a.cd[q].h;
+            for (int s = 0; s < 2; ++s) {  // a boundary's constant is 0 or well inside the range
+                const GhostRule& r = gi.rule[q][s][0];
+                const double c = std::fabs(r.type == 1 ? r.c2 / r.c3 : r.type == 2 ? r.c1 : 0.0);
+                ok &= c == 0.0 || (c >= 0x1p-400 && c <= 0x1p400);
+            }
+        }
+        if (ok) mode = FTCS_CDIV;
+    }
+    // the Dirichlet rules' divisors, in the form the arithmetic mode takes: reciprocals when every
+    // one of them is a power of two
+    bool rpow2 = mode != FTCS_CDIV;
+    for (int q = 0; q < d.dim; ++q)
+        for (int s = 0; s < 2; ++s) {
+            const double c3 = std::fabs((double)a.rc3[q][s]);
+            if (a.rtype[q][s] == RULE_DIV) rpow2 &= is_pow2(c3) && c3 >= 0x1p-100 && c3 <= 0x1p100;
+        }
+    a.gform = rpow2 ? RULE_MUL : RULE_DIV;
+    for (int q = 0; q < d.dim; ++q)
+        for (int s = 0; s < 2; ++s) {
+            if (a.rtype[q][s] != RULE_DIV) continue;
+            if (rpow2) {
+                a.rtype[q][s] = RULE_MUL;
+                a.rc3[q][s] = T(1) / a.rc3[q][s];
+            } else if (mode == FTCS_CDIV) {
+                a.rtype[q][s] = RULE_CDIV;
+                a.gd[q][s].h = std::fabs((double)a.rc3[q][s]);
+                a.gd[q][s].y = 1.0 / a.gd[q][s].h;
+            }
+        }
     if (pow2) {
         for (int q = 0; q < d.dim; ++q) a.hh[q] = (T)(1.0 / m->h[q]);
         const T k2 = a.hh[0] * a.hh[0];  // exact: a power of two
@@ -593,11 +817,13 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
         }
         nxt = f->spare;
     }
+    const Strip2d p2 = d.dim == 2 ? strip_plan(a.n, a.per, nsteps, tblock, !pow2, f->ctx->cus) : Strip2d{};
     bool ghosts_stale = false;  // the 3-D blocked kernel writes interior cells only
     for (int it = 0; it < nsteps;) {
         const T* in = (const T*)cur;
         T* out = (T*)nxt;
-        const int k = launch_steps(d.dim, d.dtype, a.n, a.per, (long long)a.e0 * a.e1, nsteps - it, tblock);
+        const int k = d.dim == 2 ? std::min(p2.nt, nsteps - it)
+                                 : launch_steps3(d.dtype, (long long)a.e0 * a.e1, nsteps - it, tblock);
         if (ghosts_stale && !(d.dim == 3 && k > 1 && a.per[0] && a.per[1] && a.per[2])) {
             OPF_TRY(launch_ghost_fill(f, cur));
             ghosts_stale = false;
@@ -608,27 +834,21 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
             else if (mode == FTCS_MUL) launch(std::integral_constant<int, FTCS_MUL>{});
             else launch(std::integral_constant<int, FTCS_DIV>{});
         };
-        if (d.dim == 2 && k > 1) {
-            // nt = k <= the kernel's TB steps (a remainder runs the same tile shape)
-            int tiles = ((a.n[0] + FT_TS2 - 1) / FT_TS2) * ((a.n[1] + FT_TS2 - 1) / FT_TS2);
-            if (tb2_steps(a.n) == FT_TB2S) {
-                // small grids: small tiles so that every CU gets several workgroups
-                int ts = ((a.n[0] + FT_TS2S - 1) / FT_TS2S) * ((a.n[1] + FT_TS2S - 1) / FT_TS2S);
-                by_mode([&](auto M) {
-                    hipLaunchKernelGGL((ftcs2d_tb_kernel<T, decltype(M)::value, FT_TS2S, FT_TB2S>), dim3(ts), dim3(256),
-                                       0, st, in, out, a, k);
-                });
-            } else {
-                by_mode([&](auto M) {
-                    hipLaunchKernelGGL((ftcs2d_tb_kernel<T, decltype(M)::value, FT_TS2, FT_TB2>), dim3(tiles), dim3(256),
-                                       0, st, in, out, a, k);
-                });
-            }
-        } else if (d.dim == 2) {
-            dim3 grid((a.n[0] + 63) / 64, (a.n[1] + 3) / 4);
-            by_mode([&](auto M) {
-                hipLaunchKernelGGL((ftcs2d_kernel<T, decltype(M)::value>), grid, dim3(64, 4), 0, st, in, out, a);
-            });
+        if (d.dim == 2) {
+            const unsigned tiles = (unsigned)(((a.n[0] + p2.tx - 1) / p2.tx) * ((a.n[1] + p2.ty - 1) / p2.ty));
+            auto launch2 = [&](auto M) {
+                constexpr int MD = decltype(M)::value;
+                auto with = [&](auto C) {
+                    constexpr int c = decltype(C)::value;
+                    hipLaunchKernelGGL((ftcs2d_strip_kernel<T, MD, S2_XW[c], S2_RW[c], S2_NW[c]>), dim3(tiles),
+                                       dim3(64 * S2_NW[c]), 0, st, in, out, a, k, p2.tx, p2.ty);
+                };
+                if (p2.cfg == 0) with(std::integral_constant<int, 0>{});
+                else if (p2.cfg == 1) with(std::integral_constant<int, 1>{});
+                else if constexpr (MD != FTCS_CDIV && MD != FTCS_DIV) with(std::integral_constant<int, 2>{});
+            };
+            if (mode == FTCS_CDIV) launch2(std::integral_constant<int, FTCS_CDIV>{});
+            else by_mode(launch2);
         } else if (d.dim == 3 && k > 1) {
             using C3 = Ftcs3dCfg<T>;
             const bool allper = a.per[0] && a.per[1] && a.per[2];
@@ -715,8 +935,12 @@ extern "C" int opf_ftcs_plan(const opf_field* u, int nsteps, int tblock, int* la
     }
     *launches = 0;
     *max_steps = 0;
+    bool pow2 = true;
+    for (int q = 0; q < d.dim; ++q) pow2 &= is_pow2(u->mesh->h[q]);
+    const int nt = d.dim == 2 && nsteps > 0 ? strip_plan(n, per, nsteps, tblock, !pow2, u->ctx->cus).nt : 0;
     for (int it = 0; it < nsteps;) {
-        int k = launch_steps(d.dim, d.dtype, n, per, (long long)d.extent[0] * d.extent[1], nsteps - it, tblock);
+        const int k = d.dim == 2 ? std::min(nt, nsteps - it)
+                                 : launch_steps3(d.dtype, (long long)d.extent[0] * d.extent[1], nsteps - it, tblock);
         ++*launches;
         *max_steps = std::max(*max_steps, k);
         it += k;

@@ -22,3 +22,7 @@ def test_ghost_index_math(tmp_path):
 
 def test_fastdiv_matches_hardware_divide(tmp_path):
     assert "passed" in _build_run("fastdiv_check", tmp_path)
+
+
+def test_const_div_is_the_ieee_quotient(tmp_path):
+    assert "passed" in _build_run("constdiv_check", tmp_path)
