@@ -367,7 +367,7 @@ def main():
                      "step_equivalent_frac": alg_bytes * args.steps / (ms / 1e3) / 1e9 / HBM_PEAK_GBS,
                      "traffic_GBps": traffic / per_launch_s / 1e9 if traffic else None,
                      "traffic_frac": traffic / per_launch_s / 1e9 / HBM_PEAK_GBS if traffic else None,
-                     "kernel": "ftcs3d_tb_kernel" if steps_per_launch > 1 else "ftcs3d_lds_kernel",
+                     "kernel": "ftcs3d_strip_kernel",
                      "steps_per_launch": steps_per_launch, "launches": launches},
         "cpu_baseline": cpu,
         "wall_s_timed_region": wall,

@@ -12,8 +12,8 @@
 // FP32: the quotient of two 24-bit numbers is at least 2^-49 (relative) away from every midpoint
 // of neighbouring floats it is not equal to, and x RN64(1 / h) in FP64 is within 2^-52 of it, so
 // rounding that product to float gives the IEEE quotient. It can equal a midpoint only where the
-// result is subnormal; such a quotient is reported (div_subnormal) and divided by the caller
-// again. Infinities, NaN, zeros and overflow come out as in the division.
+// result is subnormal, which the callers' range keeps out. Infinities, NaN, zeros and overflow come
+// out as in the division.
 #pragma once
 
 #include <cmath>
@@ -38,37 +38,58 @@ OPF_CD_HD double const_div(double x, const ConstDivisor& c) {
 }
 OPF_CD_HD float const_div(float x, const ConstDivisor& c) { return (float)((double)x * c.y); }
 
-// FP64 heat steps of a field whose values are all 0 or in [2^-500, 2^600): a difference of two is
-// 0 or at least 2^-552, its quotient by h <= 2^50 at least 2^-602, a difference of two quotients 0
-// or at least 2^-654 -- far above the 2^-969 below which the residual would not be exact -- and
-// with |coef| >= 2^-100 the new value is 0 or at least 2^-908, so its magnitude shows in the high
-// word, where the next step's test looks for it. div_key orders the high words so that 0 is the
-// largest: a minimum over cells below kDivLow means a nonzero value under 2^-500.
+// The range of a field's values for its heat steps: every value 0 or at least 2^-T in magnitude,
+// and in FP64 under 2^600.
+//   FP64, T = 500: a difference of two values is 0 or at least 2^-552, its quotient by h <= 2^50 at
+//   least 2^-602, a difference of two quotients 0 or at least 2^-654 -- far above the 2^-969 below
+//   which the residual would not be exact -- and with |coef| >= 2^-100 the new value is 0 or at least
+//   2^-908, so its magnitude shows in the high word, where the next step's test looks for it.
+//   FP32, T = min(100, 103 + l, 80 + 2 l) for spacings up to 2^-l: a difference is 0 or at least
+//   2^-(T + 23), so its quotient at least 2^-126; a difference of two quotients is 0 or at least
+//   2^-(T + 46) / h, and its quotient at least 2^-126 again: nothing is subnormal.
+// div_key orders the magnitudes (the high words, in FP64) so that 0 is the largest: a minimum over
+// cells below the key of 2^-T means that a nonzero value is smaller.
 constexpr unsigned kDivLow = ((1023u - 500u) << 21) - 1u;
 constexpr unsigned kDivHigh = (1023u + 400u) << 21;  // at the launch's start; the steps then add at most 2^200
 
 #if defined(__HIPCC__)
-__device__ __forceinline__ unsigned div_key(double v) {  // 2 hi - 1 (the compiler takes three instructions)
+// 2 bits - 1 in one instruction (the compiler takes three)
+__device__ __forceinline__ unsigned div_key_bits(int bits) {
     unsigned k;
-    asm("v_lshl_add_u32 %0, %1, 1, -1" : "=v"(k) : "v"(__double2hiint(v)));
+    asm("v_lshl_add_u32 %0, %1, 1, -1" : "=v"(k) : "v"(bits));
     return k;
 }
+__device__ __forceinline__ unsigned div_key(double v) { return div_key_bits(__double2hiint(v)); }
+__device__ __forceinline__ unsigned div_key(float v) { return div_key_bits(__float_as_int(v)); }
 // outside the range at the launch's start: subnormal, below 2^-500, 2^400 or more, infinite, NaN
 __device__ __forceinline__ bool div_unsafe(double v) {
     const unsigned m = (unsigned)__double2hiint(v) << 1;
     return (m - kDivLow >= kDivHigh - kDivLow) && v != 0.0;
 }
-__device__ __forceinline__ bool div_subnormal(float q) { return __builtin_isfpclass(q, 0x90); }  // +-subnormal
 #endif
 
+// the least key of a value in the range of spacings h[0 .. dim - 1]
+inline unsigned div_low(const double* h, int dim, bool f64) {
+    if (f64) return kDivLow;
+    int l = 1000, e;
+    for (int d = 0; d < dim; ++d) {
+        std::frexp(h[d], &e);  // h < 2^e
+        if (-e < l) l = -e;
+    }
+    int t = 100;
+    if (103 + l < t) t = 103 + l;
+    if (80 + 2 * l < t) t = 80 + 2 * l;
+    return t < -100 ? 0xffffffffu : ((unsigned)(127 - t) << 24) - 1u;
+}
+
 // the host's side of the range: spacing, coefficient and growth of `steps` steps in `dim` dims
-inline bool div_range(const double* h, int dim, double coef, int steps) {
+inline bool div_range(const double* h, int dim, double coef, int steps, bool f64) {
     double g = 0;
     for (int d = 0; d < dim; ++d) {
-        if (!(h[d] >= 0x1p-100 && h[d] <= 0x1p50)) return false;
+        if (!(f64 ? h[d] >= 0x1p-100 && h[d] <= 0x1p50 : h[d] >= 0x1p-60 && h[d] <= 0x1p20)) return false;
         g += 4.0 * std::fabs(coef) / (h[d] * h[d]);
     }
-    return std::fabs(coef) >= 0x1p-100 && std::fabs(coef) <= 0x1p200 && steps * std::log2(1.0 + g) <= 200.0;
+    return !f64 || (std::fabs(coef) >= 0x1p-100 && std::fabs(coef) <= 0x1p200 && steps * std::log2(1.0 + g) <= 200.0);
 }
 
 }  // namespace opf

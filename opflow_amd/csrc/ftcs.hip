@@ -29,6 +29,9 @@ struct FtcsArgs {
     ConstDivisor cd[3];     // FTCS_CDIV: the spacings
     ConstDivisor gd[3][2];  // RULE_CDIV: the divisors of the ghost rules
     int gform;              // RULE_MUL when no side needs a division, else RULE_DIV
+    int divide;             // FTCS_CDIV: every division by h as a division
+    unsigned low;           // FTCS_CDIV: the least div_key of a value in the range
+    int stale;              // 3-D: the input's ghosts are not filled
 };
 // v -> (rc1 v - rc2) / rc3 (Dirichlet) by division, by the multiplication with rc3's exact
 // reciprocal (rc3 a power of two: the same real number rounded once), or by const_div;
@@ -44,8 +47,8 @@ enum { RULE_NONE = 0, RULE_DIV = 1, RULE_ADD = 2, RULE_MUL = 3, RULE_CDIV = 4 };
 //                over dimensions keeps the common factor k^2, and coef * (k^2 S) =
 //                (coef k^2) * S with coef k^2 exact: u + coefh * (Dx + Dy [+ Dz]) with
 //                D = (r-c) - (c-l) -- 10 operations per 3-D cell instead of 19.
-//  FTCS_CDIV     any h: the divisions by h through its reciprocal (constdiv.hpp), where every
-//                value is in the range that needs; elsewhere FTCS_DIV's divisions.
+//  FTCS_CDIV     any h: FTCS_DIV's divisions through the reciprocal of h (constdiv.hpp) where the
+//                values are in the range that needs, as divisions elsewhere (FtcsArgs::divide: all).
 enum { FTCS_DIV = 0, FTCS_MUL = 1, FTCS_FACTORED = 2, FTCS_CDIV = 3 };
 
 // x / h of dim d in an arithmetic mode
@@ -57,64 +60,33 @@ __device__ __forceinline__ T over_h(T x, const FtcsArgs<T>& a, int d) {
     else return x / a.hh[d];
 }
 
-template <typename T, int MODE>
-__device__ __forceinline__ T d2(T l, T c, T r, T hh) {
-    if constexpr (MODE != FTCS_DIV) return ((r - c) * hh - (c - l) * hh) * hh;
-    else return ((r - c) / hh - (c - l) / hh) / hh;
-}
-
-// u^{n+1} at one cell of a 3-D field from its value and its x / y / z neighbours
-template <typename T, int MODE>
-__device__ __forceinline__ T ftcs3(T c, T xl, T xr, T yl, T yr, T zl, T zr, const FtcsArgs<T>& a) {
-    if constexpr (MODE == FTCS_FACTORED) {
-        T s = ((xr - c) - (c - xl)) + ((yr - c) - (c - yl));
-        s = s + ((zr - c) - (c - zl));
-        return c + a.coefh * s;
-    } else {
-        T s = d2<T, MODE>(xl, c, xr, a.hh[0]) + d2<T, MODE>(yl, c, yr, a.hh[1]);
-        s = s + d2<T, MODE>(zl, c, zr, a.hh[2]);
-        return c + a.coef * s;
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ T rule(const FtcsArgs<T>& a, int d, int s, T v) {
-    const int t = a.rtype[d][s];
-    if (t == RULE_ADD) return v + a.rc1[d][s];
-    if (t == RULE_NONE) return v;
-    const T x = a.rc1[d][s] * v - a.rc2[d][s];
-    if (t == RULE_MUL) return x * a.rc3[d][s];
-    return x / a.rc3[d][s];
-}
-
 // The ghost rules of a launch in one form, (c1 v - c2) over c3 with c1 = c3 = 1 where the rule only
 // adds (both exact): over c3 a multiplication by its exact reciprocal, a const_div or a division.
 // One straight line for every side, so that the lanes of a wave take theirs together.
 template <typename T>
 struct SideRule {
     T c1, c2, c3;
-    ConstDivisor cd;
+    double h, y;  // |c3| and its reciprocal (RULE_CDIV)
 };
 template <typename T>
 __device__ __forceinline__ SideRule<T> side_rule(const FtcsArgs<T>& a, int d, int s) {
     const int t = a.rtype[d][s];
-    SideRule<T> r{T(1), T(0), T(1), {}};
+    SideRule<T> r{T(1), T(0), T(1), 1.0, 1.0};
     if (t == RULE_ADD) r.c2 = -a.rc1[d][s];
     if (t == RULE_DIV || t == RULE_MUL || t == RULE_CDIV) r.c1 = a.rc1[d][s], r.c2 = a.rc2[d][s], r.c3 = a.rc3[d][s];
-    if (t == RULE_CDIV) r.cd = a.gd[d][s];
+    if (t == RULE_CDIV) r.h = a.gd[d][s].h, r.y = a.gd[d][s].y;
     return r;
 }
 // again: RULE_CDIV met a value outside const_div's range
 template <int FORM, typename T>
-__device__ __forceinline__ T ghost_value(T c1, T c2, T c3, double h, double y, T v, bool& again) {
-    const T x = c1 * v - c2;
-    if constexpr (FORM == RULE_MUL) return x * c3;
-    else if constexpr (FORM == RULE_DIV) return x / c3;
+__device__ __forceinline__ T ghost_value(const SideRule<T>& s, T v, unsigned low, bool& again) {
+    const T x = s.c1 * v - s.c2;
+    if constexpr (FORM == RULE_MUL) return x * s.c3;
+    else if constexpr (FORM == RULE_DIV) return x / s.c3;
     else {
-        const T q = const_div(x, ConstDivisor{h, y});
-        if constexpr (sizeof(T) == 4) again |= div_subnormal(q);
-        else again |= div_key(v) < kDivLow;
-        return c3 < T(0) ? -q : q;  // h = |c3|
+        const T q = const_div(x, ConstDivisor{s.h, s.y});
+        again |= div_key(v) < low;
+        return s.c3 < T(0) ? -q : q;  // h = |c3|
     }
 }
 
@@ -139,6 +111,143 @@ __device__ __forceinline__ T lane_next(T v) { return dpp<0x130>(v); }
 template <typename T>
 __device__ __forceinline__ T lane_prev(T v) { return dpp<0x138>(v); }
 
+// a wave-uniform value in scalar registers
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+__device__ __forceinline__ double uniform(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+template <bool HOIST, typename T>
+__device__ __forceinline__ SideRule<T> uniform_side(const SideRule<T>* s) {
+    int here = 0;
+    if constexpr (!HOIST) asm volatile("" : "+s"(here));  // read at each use, see stage_sides
+    s += here;
+    return {uniform(s->c1), uniform(s->c2), uniform(s->c3), uniform(s->h), uniform(s->y)};
+}
+
+// the rules of a field's sides in LDS, x lower, x upper, y lower, ..: in 3-D read where a workgroup
+// has ghosts to refill, they would otherwise hold 40 scalar registers through every loop; 2-D has
+// the registers (HOIST)
+template <typename T>
+__device__ __forceinline__ void stage_sides(const FtcsArgs<T>& a, SideRule<T>* side, int dim) {
+    if ((int)threadIdx.x < 2 * dim) side[threadIdx.x] = side_rule(a, threadIdx.x >> 1, threadIdx.x & 1);
+    __syncthreads();
+}
+
+// The ghost cells of a wave's part of a region (XW cells a lane from column gx0, RW rows from row
+// gy0; the region spans width columns from lox) and their refill from fresh cells: x, then y.
+template <typename T, int XW, int RW, bool HOIST>
+struct StripGhosts {
+    static_assert(XW <= 2, "the ghost columns are a lane's first or second");
+    bool xlo, xhi, ylo, yhi, any;  // uniform over the wave
+    bool lo, hi0, hi1;             // this lane: its first column is the lower ghost; its first, second the upper
+    int rlo, rhi;                  // ghost rows
+    const SideRule<T>* side;       // x lower, x upper, y lower, y upper
+    unsigned low;                  // FtcsArgs::low
+
+    __device__ __forceinline__ StripGhosts(const FtcsArgs<T>& a, const SideRule<T>* sides, int lox, int width, int gx0,
+                                           int gy0)
+        : side(sides), low(a.low) {
+        const int n0 = a.n[0], n1 = a.n[1];
+        xlo = !a.per[0] && lox <= -1;
+        xhi = !a.per[0] && lox + width > n0;
+        rlo = a.per[1] ? -1 : -1 - gy0;
+        rhi = a.per[1] ? -1 : n1 - gy0;
+        ylo = rlo >= 0 && rlo < RW;
+        yhi = rhi >= 0 && rhi < RW;
+        any = xlo || xhi || ylo || yhi;
+        lo = gx0 == -1;
+        hi0 = gx0 == n0;
+        hi1 = gx0 + 1 == n0;
+    }
+    // true when RULE_CDIV met a value out of its range: the fill is then done again by division
+    template <int FM>
+    __device__ __forceinline__ bool refill(T (&v)[RW][XW]) const {
+        bool again = false;
+        if (xlo) {
+            const SideRule<T> s = uniform_side<HOIST>(side);
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                const T src = XW > 1 ? v[r][XW > 1 ? 1 : 0] : lane_next(v[r][0]);
+                v[r][0] = pick(lo, ghost_value<FM>(s, src, low, again), v[r][0]);
+            }
+        }
+        if (xhi) {
+            const SideRule<T> s = uniform_side<HOIST>(side + 1);
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                const T prev = lane_prev(v[r][XW - 1]);
+                if constexpr (XW > 1) v[r][1] = pick(hi1, ghost_value<FM>(s, v[r][0], low, again), v[r][1]);
+                v[r][0] = pick(hi0, ghost_value<FM>(s, prev, low, again), v[r][0]);
+            }
+        }
+        if (ylo) {
+            const SideRule<T> s = uniform_side<HOIST>(side + 2);
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                T src = v[1][k];
+#pragma unroll
+                for (int r = 1; r + 1 < RW; ++r) src = pick(r == rlo, v[r + 1][k], src);
+                const T g = ghost_value<FM>(s, src, low, again);
+#pragma unroll
+                for (int r = 0; r + 1 < RW; ++r) v[r][k] = pick(r == rlo, g, v[r][k]);
+            }
+        }
+        if (yhi) {
+            const SideRule<T> s = uniform_side<HOIST>(side + 3);
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                T src = v[0][k];
+#pragma unroll
+                for (int r = 2; r < RW; ++r) src = pick(r == rhi, v[r - 1][k], src);
+                const T g = ghost_value<FM>(s, src, low, again);
+#pragma unroll
+                for (int r = 1; r < RW; ++r) v[r][k] = pick(r == rhi, g, v[r][k]);
+            }
+        }
+        return FM == RULE_CDIV && __any(again);
+    }
+    // mul: every rule multiplies; slow: no const_div
+    template <int FORM>
+    __device__ __forceinline__ void fill(T (&v)[RW][XW], bool mul, bool slow) const {
+        if (FORM == RULE_MUL && mul) refill<RULE_MUL>(v);
+        else if (FORM != RULE_CDIV || slow || refill<RULE_CDIV>(v)) refill<RULE_DIV>(v);
+    }
+};
+
+// First row of a region of WY rows for the tile from row y0 with nt rows of halo, on a side that is
+// not periodic: from the ghost row on, or up to it as the last row of the last wave; both ghost rows
+// inside, each in one wave with the row beside it.
+template <int RW, int WY>
+__device__ __forceinline__ int strip_rows(int y0, int nt, int n1) {
+    int lo = max(y0 - nt, -1);
+    if (lo + WY > n1 + 1) {
+        lo = n1 + 1 - WY;
+        if (lo < -1) lo = (n1 + 1) % RW == 0 ? -2 : -1;
+    }
+    return lo;
+}
+
+// a ghost plane from the plane beside it
+template <int FORM, typename T, int RW, int XW>
+__device__ __forceinline__ void strip_ghost_plane(const SideRule<T>* side, const T (&src)[RW][XW], T (&dst)[RW][XW],
+                                                  bool mul, bool slow, unsigned low) {
+    const SideRule<T> r = uniform_side<false>(side);
+    auto fill = [&](auto F) __attribute__((always_inline)) -> bool {
+        constexpr int FM = decltype(F)::value;
+        bool again = false;
+#pragma unroll
+        for (int j = 0; j < RW; ++j)
+#pragma unroll
+            for (int k = 0; k < XW; ++k)
+                dst[j][k] = ghost_value<FM>(r, src[j][k], low, again);
+        return FM == RULE_CDIV && __any(again);
+    };
+    if (FORM == RULE_MUL && mul) fill(std::integral_constant<int, RULE_MUL>{});
+    else if (FORM != RULE_CDIV || slow || fill(std::integral_constant<int, RULE_CDIV>{}))
+        fill(std::integral_constant<int, RULE_DIV>{});
+}
+
 // 2-D steps in registers. A workgroup holds a region of 64 XW x NW RW cells: lane l of a wave
 // the XW neighbouring cells l XW .. in x, wave w the RW rows w RW .., so that y neighbours are
 // registers, x neighbours are registers or one lane away (DPP, no LDS), and only the first and
@@ -159,7 +268,6 @@ __device__ __forceinline__ T lane_prev(T v) { return dpp<0x138>(v); }
 template <typename T, int MODE, int XW, int RW, int NW>
 __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restrict__ in, T* __restrict__ out,
                                                                FtcsArgs<T> a, int nt, int tx, int ty) {
-    static_assert(XW <= 2, "the ghost columns are a lane's first or second");
     constexpr int WX = 64 * XW, WY = RW * NW;
     __shared__ T edge[2][NW][2][XW][64];  // first and last row of every wave, double-buffered
     const int n0 = a.n[0], n1 = a.n[1];
@@ -167,16 +275,8 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
     const int tb = (int)xcd_block(blockIdx.x, gridDim.x);  // x-neighbouring tiles share an XCD's L2
     const int x0 = (tb % tilesx) * tx, y0 = (tb / tilesx) * ty;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // region origin; non-periodic sides: x from the ghost column on, y from the ghost row or up to it
-    int lox = x0 - nt, loy = y0 - nt;
-    if (!a.per[0]) lox = max(lox, -1);
-    if (!a.per[1]) {
-        loy = max(loy, -1);
-        if (loy + WY > n1 + 1) {
-            loy = n1 + 1 - WY;  // the upper ghost row is the last of the last wave
-            if (loy < -1) loy = (n1 + 1) % RW == 0 ? -2 : -1;  // both ghost rows inside
-        }
-    }
+    const int lox = a.per[0] ? x0 - nt : max(x0 - nt, -1);
+    const int loy = a.per[1] ? y0 - nt : strip_rows<RW, WY>(y0, nt, n1);
     const int gx0 = lox + lane * XW, gy0 = loy + w * RW;
     T u[RW][XW];
     {
@@ -196,73 +296,18 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
             for (int k = 0; k < XW; ++k) u[r][k] = row[ox[k]];
         }
     }
-    // the ghosts of this wave: columns (uniform over the workgroup), rows (of this wave)
-    const bool xlo = !a.per[0] && lox <= -1, xhi = !a.per[0] && lox + WX > n0;
-    const int rlo = a.per[1] ? -1 : -1 - gy0, rhi = a.per[1] ? -1 : n1 - gy0;
-    const bool ylo = rlo >= 0 && rlo < RW, yhi = rhi >= 0 && rhi < RW;
-    const bool ghosts = xlo || xhi || ylo || yhi;
-    constexpr int FORM = MODE == FTCS_CDIV ? RULE_CDIV : MODE == FTCS_DIV ? RULE_DIV : RULE_MUL;
-    // x rule of this lane's column (a lane holds at most one ghost column of each side)
-    const bool hilane = gx0 + XW > n0;
-    const SideRule<T> rl = side_rule(a, 0, 0), rh = side_rule(a, 0, 1), ryl = side_rule(a, 1, 0), ryh = side_rule(a, 1, 1);
-    const T xc1 = hilane ? rh.c1 : rl.c1, xc2 = hilane ? rh.c2 : rl.c2, xc3 = hilane ? rh.c3 : rl.c3;
-    const double xh = hilane ? rh.cd.h : rl.cd.h, xy = hilane ? rh.cd.y : rl.cd.y;
-    // refills the ghosts of v; true when RULE_CDIV met a value out of its range (v is unchanged then)
-    auto refill = [&](auto F, T(&v)[RW][XW]) __attribute__((always_inline)) -> bool {
-        constexpr int FM = decltype(F)::value;
-        bool again = false;
-        if (xlo || xhi) {
-            // the lower ghost is a lane's first column, its source the next one; the upper ghost's
-            // source the previous column
-            T g[RW][XW];
-#pragma unroll
-            for (int r = 0; r < RW; ++r) {
-                const T nx = XW > 1 ? v[r][XW > 1 ? 1 : 0] : lane_next(v[r][0]);
-                const T pv = lane_prev(v[r][XW - 1]);
-                g[r][0] = ghost_value<FM>(xc1, xc2, xc3, xh, xy, hilane ? pv : nx, again);
-                if constexpr (XW > 1) g[r][1] = ghost_value<FM>(xc1, xc2, xc3, xh, xy, v[r][0], again);
-            }
-            if (FM == RULE_CDIV && __any(again)) return true;
-#pragma unroll
-            for (int r = 0; r < RW; ++r) {
-                v[r][0] = pick(gx0 == -1 || gx0 == n0, g[r][0], v[r][0]);
-                if constexpr (XW > 1) v[r][1] = pick(gx0 + 1 == n0, g[r][1], v[r][1]);
-            }
-        }
-        if (ylo) {
-#pragma unroll
-            for (int k = 0; k < XW; ++k) {
-                T src = v[1][k];
-#pragma unroll
-                for (int r = 1; r + 1 < RW; ++r) src = pick(r == rlo, v[r + 1][k], src);
-                T g = ghost_value<FM>(ryl.c1, ryl.c2, ryl.c3, ryl.cd.h, ryl.cd.y, src, again);
-                if (FM == RULE_CDIV && __any(again)) g = ghost_value<RULE_DIV>(ryl.c1, ryl.c2, ryl.c3, 1., 1., src, again);
-#pragma unroll
-                for (int r = 0; r + 1 < RW; ++r) v[r][k] = pick(r == rlo, g, v[r][k]);
-            }
-        }
-        if (yhi) {
-#pragma unroll
-            for (int k = 0; k < XW; ++k) {
-                T src = v[0][k];
-#pragma unroll
-                for (int r = 2; r < RW; ++r) src = pick(r == rhi, v[r - 1][k], src);
-                T g = ghost_value<FM>(ryh.c1, ryh.c2, ryh.c3, ryh.cd.h, ryh.cd.y, src, again);
-                if (FM == RULE_CDIV && __any(again)) g = ghost_value<RULE_DIV>(ryh.c1, ryh.c2, ryh.c3, 1., 1., src, again);
-#pragma unroll
-                for (int r = 1; r < RW; ++r) v[r][k] = pick(r == rhi, g, v[r][k]);
-            }
-        }
-        return false;
-    };
-    bool slow = false;  // FTCS_CDIV, FP64: a value outside the range for the whole launch
+    constexpr int FORM = MODE == FTCS_CDIV ? RULE_CDIV : RULE_MUL;
+    __shared__ SideRule<T> side[4];
+    stage_sides(a, side, 2);
+    const StripGhosts<T, XW, RW, true> gh(a, side, lox, WX, gx0, gy0);
+    bool slow = MODE == FTCS_CDIV && a.divide;  // FP64: or a value outside the range for the whole launch
     if constexpr (MODE == FTCS_CDIV && sizeof(T) == 8) {
         bool bad = false;
 #pragma unroll
         for (int r = 0; r < RW; ++r)
 #pragma unroll
             for (int k = 0; k < XW; ++k) bad |= div_unsafe(u[r][k]);
-        slow = __syncthreads_or(bad);
+        slow |= (bool)__syncthreads_or(bad);
     }
     for (int s = 0; s < nt; ++s) {
         auto& e = edge[s & 1];
@@ -274,15 +319,9 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
             }
         }
         T v[RW][XW];  // the second x differences, then the new values
-        // returns whether a float quotient was subnormal
-        auto xpart = [&](auto M) __attribute__((always_inline)) -> bool {
+        auto xpart = [&](auto M) __attribute__((always_inline)) {
             constexpr int MD = decltype(M)::value;
-            bool sub = false;
-            auto quo = [&](T x) __attribute__((always_inline)) -> T {
-                const T q = over_h<T, MD>(x, a, 0);
-                if constexpr (MD == FTCS_CDIV && sizeof(T) == 4) sub |= div_subnormal(q);
-                return q;
-            };
+            auto quo = [&](T x) __attribute__((always_inline)) -> T { return over_h<T, MD>(x, a, 0); };
 #pragma unroll
             for (int r = 0; r < RW; ++r) {
                 T qx[XW];
@@ -295,17 +334,11 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
 #pragma unroll
                 for (int k = 0; k < XW; ++k) v[r][k] = quo(qx[k] - (k > 0 ? qx[k > 0 ? k - 1 : 0] : left));
             }
-            return sub;
         };
         T dn[XW], up[XW];  // the rows before the first and after the last
-        auto ypart = [&](auto M) __attribute__((always_inline)) -> bool {
+        auto ypart = [&](auto M) __attribute__((always_inline)) {
             constexpr int MD = decltype(M)::value;
-            bool sub = false;
-            auto quo = [&](T x) __attribute__((always_inline)) -> T {
-                const T q = over_h<T, MD>(x, a, 1);
-                if constexpr (MD == FTCS_CDIV && sizeof(T) == 4) sub |= div_subnormal(q);
-                return q;
-            };
+            auto quo = [&](T x) __attribute__((always_inline)) -> T { return over_h<T, MD>(x, a, 1); };
             T qy[XW];
 #pragma unroll
             for (int k = 0; k < XW; ++k) qy[k] = quo(u[0][k] - dn[k]);
@@ -318,9 +351,8 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
                     qy[k] = qn;
                     v[r][k] = u[r][k] + (MD == FTCS_FACTORED ? a.coefh : a.coef) * (v[r][k] + dy);
                 }
-            return sub;
         };
-        bool sub = xpart(std::integral_constant<int, MODE>{});  // needs no other wave: while the rows are on their way
+        xpart(std::integral_constant<int, MODE>{});  // needs no other wave: while the rows are on their way
         if constexpr (NW > 1) {
             __syncthreads();
 #pragma unroll
@@ -333,7 +365,7 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
             for (int k = 0; k < XW; ++k) dn[k] = u[0][k], up[k] = u[RW - 1][k];
         }
         bool again = slow;
-        if constexpr (MODE == FTCS_CDIV && sizeof(T) == 8) {
+        if constexpr (MODE == FTCS_CDIV) {
             unsigned m = 0xffffffffu;
 #pragma unroll
             for (int k = 0; k < XW; ++k) {
@@ -341,22 +373,16 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
 #pragma unroll
                 for (int r = 0; r < RW; ++r) m = min(m, div_key(u[r][k]));
             }
-            again |= __any(m < kDivLow);
+            again |= __any(m < a.low);
         }
-        if (!again) sub |= ypart(std::integral_constant<int, MODE>{});
+        if (!again) ypart(std::integral_constant<int, MODE>{});
         if constexpr (MODE == FTCS_CDIV) {
-            if (sizeof(T) == 4) again = __any(sub);
             if (again) {
                 xpart(std::integral_constant<int, FTCS_DIV>{});
                 ypart(std::integral_constant<int, FTCS_DIV>{});
             }
         }
-        if (ghosts) {
-            bool done = false;
-            if (FORM == RULE_MUL && a.gform == RULE_MUL) done = !refill(std::integral_constant<int, RULE_MUL>{}, v);
-            else if (FORM == RULE_CDIV && !again) done = !refill(std::integral_constant<int, RULE_CDIV>{}, v);
-            if (!done) refill(std::integral_constant<int, RULE_DIV>{}, v);
-        }
+        if (gh.any) gh.template fill<FORM>(v, a.gform == RULE_MUL, again);
 #pragma unroll
         for (int r = 0; r < RW; ++r)
 #pragma unroll
@@ -390,250 +416,228 @@ __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restri
     }
 }
 
-// 3-D single step, LDS-tiled: a 64 x NTY workgroup owns a 64 x (NTY * RY) x-y
-// tile (each thread RY rows) and marches ZC planes in z. The current plane of
-// the tile and its one-cell x/y halo sit in LDS (double-buffered, one barrier
-// per plane); each thread keeps its cells' z-1 / z / z+1 values in registers
-// and loads plane k+2 while plane k is computed. The input's ghost layer
-// supplies the halo of boundary tiles, so loads never wrap; the kernel writes
-// interior cells only and the host loop refills the output's ghosts before
-// they are read. Per cell: d2x + d2y, then + d2z, then u + coef * s -- the
-// arithmetic every FTCS kernel here uses, so all give the same bits.
-// Launch shape swept at 512^3 on MI355X (64 x 8 threads, 2 rows each, 8 planes).
-constexpr int FT3_TX = 64, FT3_NTY = 8, FT3_RY = 2, FT3_TY = FT3_NTY * FT3_RY, FT3_ZC = 8;
-
-template <typename T, int MODE, int ZC, int NTY, int RY>
-__global__ __launch_bounds__(64 * NTY) void ftcs3d_lds_kernel(const T* __restrict__ in, T* __restrict__ out,
-                                                              FtcsArgs<T> a) {
-    constexpr int TY = NTY * RY;
-    static_assert(128 + 2 * TY <= 64 * NTY, "one halo element per thread at most");
-    __shared__ T lds[2][TY + 2][FT3_TX + 2];
-    const int tx = threadIdx.x, ty = threadIdx.y, t = ty * 64 + tx;
-    // tile of this block: the flat id through xcd_block, so that each XCD's L2 holds a
-    // contiguous slab whose x / y halo lines its own tiles share
-    const uint32_t L = xcd_block(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
-                                 gridDim.x * gridDim.y * gridDim.z);
-    const int x0 = (int)(L % gridDim.x) * FT3_TX, y0 = (int)((L / gridDim.x) % gridDim.y) * TY,
-              k0 = (int)(L / (gridDim.x * gridDim.y)) * ZC;
-    const int kend = min(k0 + ZC, a.n[2]);
-    const long long sy = a.e0, sz = (long long)a.e0 * a.e1;
-    const int i = x0 + tx;
-    // storage index of (x, y, k) (ghost layer at -1 and n)
-    auto at = [&](int x, int y, int k) { return (long long)(x + 1) + sy * (y + 1) + sz * (k + 1); };
-    // valid storage positions: interior and the ghost layer
-    auto ok = [&](int x, int y) { return x >= -1 && x <= a.n[0] && y >= -1 && y <= a.n[1]; };
-    // this thread's halo element: rows y0 - 1 and y0 + TY (threads 0..127), then the
-    // columns x0 - 1 and x0 + TX over the tile's rows; corners are not read
-    int hx = 0, hy = 0, hlx = 0, hly = 0;
-    if (t < 128) {
-        hx = x0 + (t & 63);
-        hy = t < 64 ? y0 - 1 : y0 + TY;
-        hlx = (t & 63) + 1;
-        hly = t < 64 ? 0 : TY + 1;
-    } else if (t < 128 + 2 * TY) {
-        const int q = t - 128, side = q / TY, r = q % TY;
-        hx = side == 0 ? x0 - 1 : x0 + FT3_TX;
-        hy = y0 + r;
-        hlx = side == 0 ? 0 : FT3_TX + 1;
-        hly = r + 1;
-    }
-    const bool hl = t < 128 + 2 * TY && ok(hx, hy);
-    bool own[RY];
-    T zm[RY], zc[RY], zp[RY], zq[RY];
-    T hp = T(0), hq = T(0);
-#pragma unroll
-    for (int r = 0; r < RY; ++r) {
-        const int j = y0 + ty * RY + r;
-        own[r] = ok(i, j);
-        zm[r] = own[r] ? in[at(i, j, k0 - 1)] : T(0);
-        zc[r] = own[r] ? in[at(i, j, k0)] : T(0);
-        zp[r] = own[r] ? in[at(i, j, k0 + 1)] : T(0);  // k0 + 1 <= n[2]: the ghost plane at most
-        lds[0][ty * RY + r + 1][tx + 1] = zc[r];
-    }
-    if (hl) {
-        lds[0][hly][hlx] = in[at(hx, hy, k0)];
-        hp = in[at(hx, hy, k0 + 1)];
-    }
-    __syncthreads();
-    int cur = 0;
-    for (int k = k0; k < kend; ++k) {
-        // plane k + 2 is loaded one step ahead of its use (only while a next step needs it)
-        if (k + 1 < kend) {
-#pragma unroll
-            for (int r = 0; r < RY; ++r) zq[r] = own[r] ? in[at(i, y0 + ty * RY + r, k + 2)] : T(0);
-            if (hl) hq = in[at(hx, hy, k + 2)];
-        }
-#pragma unroll
-        for (int r = 0; r < RY; ++r) {
-            const int ly = ty * RY + r + 1, j = y0 + ly - 1;
-            if (i >= a.n[0] || j >= a.n[1]) continue;
-            const T c = zc[r];
-            out[at(i, j, k)] = ftcs3<T, MODE>(c, lds[cur][ly][tx], lds[cur][ly][tx + 2], lds[cur][ly - 1][tx + 1],
-                                              lds[cur][ly + 1][tx + 1], zm[r], zp[r], a);
-        }
-        const int nxt = cur ^ 1;
-#pragma unroll
-        for (int r = 0; r < RY; ++r) {
-            lds[nxt][ty * RY + r + 1][tx + 1] = zp[r];
-            zm[r] = zc[r];
-            zc[r] = zp[r];
-            zp[r] = zq[r];
-        }
-        if (hl) lds[nxt][hly][hlx] = hp;
-        hp = hq;
-        __syncthreads();
-        cur = nxt;
-    }
-}
-
-// 3-D temporal blocking, K steps per launch. A workgroup owns a TX x TY column
-// of the x-y plane and the z chunk [z0, z0 + zc) and streams the planes of u^n
-// with a K-cell halo in x and y. Every thread owns fixed positions of the
-// (TX+2K) x (TY+2K) region and keeps, for each, the last three planes of
-// levels 0 .. K-1 (u^n .. u^{n+K-1}) in registers, so the centre and the z
-// neighbours never go through LDS; LDS holds only the current plane of each
-// level (double-buffered), read for the x and y neighbours. Step zz stores
-// level-0 plane zz and computes level L at plane zz - L (L = 1 .. K) on the
-// region shrunk by L cells; level K is exactly the tile and goes straight to
-// global memory. One barrier per step separates a step's LDS writes from the
-// next step's reads (levels read the plane the level below wrote one step
-// earlier). Level-0 planes are loaded three planes ahead; the unroll by 3 keeps
-// the history slots static; every load is unconditional so the compiler keeps
-// counted load waits.
-// Periodic dimensions wrap the halo to interior cells (the input's ghosts are
-// never read). Dirichlet / Neumann dimensions (ALLPER = false) clamp the halo to
-// the ghost layer: level 0 reads the input's ghosts (refilled by the host before
-// the launch), and the ghosts of the intermediate levels 1 .. K-1 are rebuilt
-// from the level's fresh boundary cells with the BC rules, as updatePadding
-// does after every step: x / y face ghosts in LDS at the start of the next step
-// (one extra barrier, only in workgroups whose region reaches such a side), z
-// ghost planes in the register history when the level computes plane 0 or
-// reaches plane n. The 7-point stencil reads face ghosts only, so edge and
-// corner ghosts are never needed; region cells beyond the ghost layer hold
-// values that never reach a valid cell. The output's ghosts are left stale and
-// refilled by the host loop before anything reads them. Per cell and step the
-// arithmetic is that of ftcs3d_lds_kernel, so the result has the same bits as K
-// single steps.
-template <typename T, int MODE, int TX, int TY, int NT, int K, bool XCD, bool ALLPER>
-__global__ __launch_bounds__(NT) void ftcs3d_tb_kernel(const T* __restrict__ in, T* __restrict__ out, FtcsArgs<T> a,
-                                                       int zc) {
-    static_assert(K >= 2, "one step per launch is ftcs3d_lds_kernel");
-    constexpr int RX = TX + 2 * K, RY = TY + 2 * K, RP = RX * RY;
-    constexpr int NL = (RP + NT - 1) / NT;
-    constexpr int PF = 3;
-    __shared__ T lds[K][2][NL * NT];  // current plane of levels 0 .. K-1
-    const int tilesx = (a.n[0] + TX - 1) / TX, tilesy = (a.n[1] + TY - 1) / TY;
-    int b = XCD ? (int)xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;  // neighbouring tiles share an XCD's L2
-    const int x0 = (b % tilesx) * TX;
+// 3-D steps in registers, K per launch: the 2-D kernel's region (64 XW x NW RW cells of a plane,
+// RW rows a wave) marching through the planes of a z chunk. Stage s of the pipeline takes the
+// planes of level s (u^{n+s}) as they appear and gives those of level s + 1 one plane later. Per
+// level a cell holds its value, the quotient of its last z difference and d2x + d2y, so that a new
+// plane costs one difference in z, and the update follows from registers alone:
+//   level s + 1 at plane p - 1 from level s at p - 1 (held) and at p (new), straight into stage
+//   s + 1 as its plane p - 1, and so on; level K goes to memory.
+// Then each wave's first and last rows of every level's new plane pass through LDS (one barrier a
+// plane), and d2x + d2y of those planes is formed for the next one. One plane
+// of level 0 is in flight. Periodic sides wrap the halo; on the others the region starts at, or contains, the
+// ghost layer: level 0 reads the input's ghosts, those of the other levels are refilled in
+// registers when a plane appears (x, then y), and the ghost planes in z are the rules of the planes
+// beside them. The output's ghosts are left stale: the host loop refills them before a launch that
+// reads them and at the end (a launch of three steps that refilled them itself would gain nothing,
+// 196 against 187 us a step at 512^3 FP64 Dirichlet: the workgroups at the sides are the last to
+// end); a single step refills its input in registers (128^3 17.9 -> 13.2 us). Per cell and step the
+// operations and their order are those of D2 in the reference.
+// A plane step takes 2.5 us of a workgroup that has its CU to itself, 1.4 of it FP64, lane moves and
+// LDS instructions of the three levels, the rest the waves' wait at the barrier and for the rows of
+// their neighbours. FP32 has the registers for two planes a round, which saves the moves of the held
+// planes (512^3 98 -> 86 us a step); FP64 spills with two. us a step, against LDS tiles of the values
+// that marched with one step (ghosts filled by a launch per step; periodic FACTORED: two steps):
+// 512^3 FP64 periodic 180 -> 152, Dirichlet 355 -> 187, 128^3 Dirichlet 30 -> 14.3, 300 x 260 x 220
+// FP32 Dirichlet 59 -> 23.
+template <typename T, int MODE, int XW, int RW, int NW, int K, bool ALLPER>
+__global__ __launch_bounds__(64 * NW) void ftcs3d_strip_kernel(const T* __restrict__ in, T* __restrict__ out,
+                                                               FtcsArgs<T> a, int tx, int ty, int zc) {
+    constexpr int WX = 64 * XW, WY = RW * NW;
+    constexpr bool D64 = sizeof(T) == 8;
+    constexpr int FORM = MODE == FTCS_CDIV ? RULE_CDIV : RULE_MUL;
+    __shared__ T edge[2][K][NW][2][XW][64];  // first and last row of every wave and level, double-buffered
+    __shared__ int wild;                     // FTCS_CDIV, FP64: a value outside the range has been read
+    const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2];
+    const int tilesx = (n0 + tx - 1) / tx, tilesy = (n1 + ty - 1) / ty;
+    int b = (int)xcd_block(blockIdx.x, gridDim.x);  // neighbouring tiles share an XCD's L2
+    const int x0 = (b % tilesx) * tx;
     b /= tilesx;
-    const int y0 = (b % tilesy) * TY;
-    const int z0 = (b / tilesy) * zc;
-    const int z1 = min(z0 + zc, a.n[2]);
+    const int y0 = (b % tilesy) * ty;
+    const int z0 = (b / tilesy) * zc, z1 = min(z0 + zc, n2);
+    const int lane = threadIdx.x & 63, w_ = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool xper = ALLPER || a.per[0], yper = ALLPER || a.per[1], zper = ALLPER || a.per[2];
+    const int lox = xper ? x0 - K : max(x0 - K, -1);
+    const int loy = yper ? y0 - K : strip_rows<RW, WY>(y0, K, n1);
+    const int gx0 = lox + lane * XW, gy0 = loy + w_ * RW;
+    __shared__ SideRule<T> side[6];
+    stage_sides(a, side, 3);
+    const StripGhosts<T, XW, RW, false> gh(a, side, lox, WX, gx0, gy0);
     const long long sz = (long long)a.e0 * a.e1;
-    const int tid = threadIdx.x;
-    // this thread's region positions: input offset, region coordinates, output offset;
-    // gh: 0 interior, 1 / 2 the low / high x face ghost, 3 / 4 the low / high y face ghost
-    int off[NL], lxm[NL], lym[NL], gh[NL];
-    bool valid[NL], inr[NL];
-    long long oo[NL];
+    const int st = K > 1 || ALLPER ? 0 : a.stale;  // read no ghosts
+    int ox[XW];  // storage offsets of this lane's columns and this wave's rows
+    long long oy[RW];
 #pragma unroll
-    for (int m = 0; m < NL; ++m) {
-        const int e = tid + m * NT;
-        valid[m] = e < RP;
-        const int ee = valid[m] ? e : 0;
-        const int lx = ee % RX, ly = ee / RX;
-        lxm[m] = lx;
-        lym[m] = ly;
-        int gx = x0 - K + lx, gy = y0 - K + ly;
-        gh[m] = 0;
-        if (ALLPER || a.per[0]) gx = (gx % a.n[0] + a.n[0]) % a.n[0];
-        if (ALLPER || a.per[1]) gy = (gy % a.n[1] + a.n[1]) % a.n[1];
-        if (!ALLPER) {
-            const bool inx = gx >= 0 && gx < a.n[0], iny = gy >= 0 && gy < a.n[1];
-            if (iny && (gx == -1 || gx == a.n[0])) gh[m] = gx < 0 ? 1 : 2;
-            if (inx && (gy == -1 || gy == a.n[1])) gh[m] = gy < 0 ? 3 : 4;
-            gx = min(max(gx, -1), a.n[0]);  // clamped: inside the storage
-            gy = min(max(gy, -1), a.n[1]);
-        }
-        off[m] = (gx + 1) + a.e0 * (gy + 1);
-        const int i = x0 + lx - K, j = y0 + ly - K;
-        inr[m] = i < a.n[0] && j < a.n[1];
-        oo[m] = (long long)(i + 1) + (long long)a.e0 * (j + 1);
+    for (int k = 0; k < XW; ++k) {
+        int gx = gx0 + k;
+        if (xper) gx = ((gx % n0) + n0) % n0;
+        ox[k] = min(max(gx, -1 + st), n0 - st) + 1;
     }
-    // position m takes part in level L (region shrunk by L cells)
-    auto at_level = [&](int m, int L) {
-        return valid[m] && lxm[m] >= L && lxm[m] <= RX - 1 - L && lym[m] >= L && lym[m] <= RY - 1 - L;
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        int gy = gy0 + r;
+        if (yper) gy = ((gy % n1) + n1) % n1;
+        oy[r] = (long long)a.e0 * (min(max(gy, -1 + st), n1 - st) + 1);
+    }
+    // planes of level 0 from ta; level K's plane t - K appears at t
+    const int ta = zper ? z0 - K : max(z0 - K, -1 + st), tb = z1 + K;
+    const int zw = zper ? ((ta % n2) + n2) % n2 : max(ta, -1 + st);
+    const T* from = in + sz * (zw + 1);  // the next plane to load
+    const T* const wrap = in + sz * (n2 + 1);
+    const T* const last = wrap - sz * st;
+    T pre[RW][XW], u[K][RW][XW], qz[K][RW][XW], sx[K][RW][XW];
+#pragma unroll
+    for (int s = 0; s < K; ++s)
+#pragma unroll
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+            for (int k = 0; k < XW; ++k) u[s][r][k] = qz[s][r][k] = sx[s][r][k] = T(0);
+    int odd[K] = {};  // FTCS_CDIV: bit q: plane t - s - q of this wave holds a value under the range
+    bool slow = MODE == FTCS_CDIV && a.divide;
+    if (MODE == FTCS_CDIV && D64) {
+        if (threadIdx.x == 0) wild = slow;
+        __syncthreads();
+    }
+    auto load = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+            for (int k = 0; k < XW; ++k) pre[r][k] = (from + oy[r])[ox[k]];
+        // periodic: plane 0 after plane n2 - 1; else the last plane (the ghost plane) again
+        from += sz;
+        if (zper && from == wrap) from = in + sz;
+        if (!zper && from > last) from = last;
     };
-    // the region reaches a non-periodic x / y side: face ghosts to rebuild (uniform over the block)
-    const bool edge = !ALLPER && ((!a.per[0] && (x0 - K < 0 || x0 + TX + K > a.n[0])) ||
-                                  (!a.per[1] && (y0 - K < 0 || y0 + TY + K > a.n[1])));
-    const bool zper = ALLPER || a.per[2];
-    const int zb = z0 - K, ze = z1 + K;  // level-0 planes zb .. ze - 1
-    T pre[PF][NL], hist[K][NL][3];       // history slot of plane p: (p - zb) % 3
-    auto load = [&](T(&r)[NL], int z) {
-        if (zper) z = (z % a.n[2] + a.n[2]) % a.n[2];
-        else z = min(max(z, -1), a.n[2]);
-        const T* p = in + sz * (z + 1);
+    load();
+    const T coef = MODE == FTCS_FACTORED ? a.coefh : a.coef;
+    auto plane = [&](int t) __attribute__((always_inline)) {
+        T w[RW][XW];  // the plane that appears
 #pragma unroll
-        for (int m = 0; m < NL; ++m) r[m] = p[off[m]];
-    };
+        for (int r = 0; r < RW; ++r)
 #pragma unroll
-    for (int u = 0; u < PF; ++u) load(pre[u], min(zb + u, ze - 1));
-    for (int zz0 = zb; zz0 < ze; zz0 += PF) {
+            for (int k = 0; k < XW; ++k) w[r][k] = pre[r][k];
+        load();
+        if constexpr (MODE == FTCS_CDIV && D64) {
+            bool bad = false;
 #pragma unroll
-        for (int u = 0; u < PF; ++u) {
-            const int zz = zz0 + u;  // (zz - zb) % 3 == u
-            if (zz >= ze) break;     // uniform over the block
-            __syncthreads();
-            T* w0 = lds[0][zz & 1];
+            for (int r = 0; r < RW; ++r)
 #pragma unroll
-            for (int m = 0; m < NL; ++m) {
-                hist[0][m][u] = pre[u][m];
-                w0[tid + m * NT] = pre[u][m];
+                for (int k = 0; k < XW; ++k) bad |= div_unsafe(w[r][k]);
+            if (__any(bad)) slow = true, wild = 1;
+        }
+        if (K == 1 && !ALLPER && st && gh.any) gh.template fill<FORM>(w, a.gform == RULE_MUL, slow);
+#pragma unroll
+        for (int s = 0; s < K; ++s) {
+            if (!zper && (s > 0 || (K == 1 && st))) {  // ghost planes of level s: n2 from the last plane, -1 before the first
+                if (t - s == n2) strip_ghost_plane<FORM>(side + 5, u[s], w, a.gform == RULE_MUL, slow, a.low);
+                if (t - s == 0) strip_ghost_plane<FORM>(side + 4, w, u[s], a.gform == RULE_MUL, slow, a.low);
             }
-            load(pre[u], min(zz + PF, ze - 1));
-            if (!ALLPER && edge) {
-                // face ghosts of the planes levels 1 .. K-1 wrote in the last step, from their
-                // boundary cells (read after the barrier above), before the next level reads them
+            T qn[RW][XW], v[RW][XW];
+            auto zpart = [&](auto M) __attribute__((always_inline)) {
+                constexpr int MD = decltype(M)::value;
 #pragma unroll
-                for (int L = 1; L < K; ++L) {
-                    if (zz - 1 < z0 - K + 2 * L) continue;  // level L had no plane yet (uniform)
-                    T* P = lds[L][(zz - 1 - L) & 1];
+                for (int r = 0; r < RW; ++r)
 #pragma unroll
-                    for (int m = 0; m < NL; ++m) {
-                        if (!gh[m] || !at_level(m, L)) continue;
-                        const int e = tid + m * NT;
-                        const int g = gh[m];
-                        const int nb = g == 1 ? e + 1 : g == 2 ? e - 1 : g == 3 ? e + RX : e - RX;
-                        P[e] = rule(a, g <= 2 ? 0 : 1, (g - 1) & 1, P[nb]);
+                    for (int k = 0; k < XW; ++k) {
+                        qn[r][k] = over_h<T, MD>(w[r][k] - u[s][r][k], a, 2);
+                        const T dz = over_h<T, MD>(qn[r][k] - qz[s][r][k], a, 2);
+                        v[r][k] = u[s][r][k] + coef * (sx[s][r][k] + dz);
+                    }
+            };
+            bool again = slow;
+            if constexpr (MODE == FTCS_CDIV) {
+                unsigned m = 0xffffffffu;
+#pragma unroll
+                for (int r = 0; r < RW; ++r)
+#pragma unroll
+                    for (int k = 0; k < XW; ++k) m = min(m, div_key(w[r][k]));
+                odd[s] = (odd[s] << 1 | (__any(m < a.low) ? 1 : 0)) & 7;
+                again |= odd[s] != 0;
+            }
+            if (!again) zpart(std::integral_constant<int, MODE>{});
+            if constexpr (MODE == FTCS_CDIV) {
+                if (again) zpart(std::integral_constant<int, FTCS_DIV>{});
+            }
+#pragma unroll
+            for (int r = 0; r < RW; ++r)
+#pragma unroll
+                for (int k = 0; k < XW; ++k) {
+                    u[s][r][k] = w[r][k];
+                    qz[s][r][k] = qn[r][k];
+                    w[r][k] = v[r][k];
+                }
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                edge[t & 1][s][w_][0][k][lane] = u[s][0][k];
+                edge[t & 1][s][w_][1][k][lane] = u[s][RW - 1][k];
+            }
+            if (!ALLPER && s + 1 < K && gh.any) gh.template fill<FORM>(w, a.gform == RULE_MUL, again);
+        }
+        if (t - K >= z0) {  // level K of plane t - K
+            T* to = out + sz * (t - K + 1);
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                const int gy = gy0 + r;
+                if (gy < y0 || gy >= min(y0 + ty, n1)) continue;
+#pragma unroll
+                for (int k = 0; k < XW; ++k) {
+                    const int gx = gx0 + k;
+                    if (gx >= x0 && gx < min(x0 + tx, n0)) (to + (long long)a.e0 * (gy + 1) + 1)[gx] = w[r][k];
+                }
+            }
+        }
+        __syncthreads();
+        if constexpr (MODE == FTCS_CDIV && D64) slow = __builtin_amdgcn_readfirstlane(wild) != 0;
+#pragma unroll
+        for (int s = 0; s < K; ++s) {
+            T dn[XW], up[XW];
+#pragma unroll
+            for (int k = 0; k < XW; ++k) {
+                dn[k] = edge[t & 1][s][max(w_ - 1, 0)][1][k][lane];
+                up[k] = edge[t & 1][s][min(w_ + 1, NW - 1)][0][k][lane];
+            }
+            auto xypart = [&](auto M) __attribute__((always_inline)) {
+                constexpr int MD = decltype(M)::value;
+                auto quo = [&](T x, int d) __attribute__((always_inline)) -> T { return over_h<T, MD>(x, a, d); };
+                T qy[XW];
+#pragma unroll
+                for (int k = 0; k < XW; ++k) qy[k] = quo(u[s][0][k] - dn[k], 1);
+#pragma unroll
+                for (int r = 0; r < RW; ++r) {
+                    T qx[XW];
+#pragma unroll
+                    for (int k = 0; k < XW; ++k) {
+                        const T right = k + 1 < XW ? u[s][r][k + 1 < XW ? k + 1 : 0] : lane_next(u[s][r][0]);
+                        qx[k] = quo(right - u[s][r][k], 0);
+                    }
+                    const T left = lane_prev(qx[XW - 1]);
+#pragma unroll
+                    for (int k = 0; k < XW; ++k) {
+                        const T qn = quo((r + 1 < RW ? u[s][r + 1 < RW ? r + 1 : 0][k] : up[k]) - u[s][r][k], 1);
+                        const T dx = quo(qx[k] - (k > 0 ? qx[k > 0 ? k - 1 : 0] : left), 0);
+                        sx[s][r][k] = dx + quo(qn - qy[k], 1);
+                        qy[k] = qn;
                     }
                 }
-                __syncthreads();
-            }
+            };
+            bool again = slow;
+            if constexpr (MODE == FTCS_CDIV) {
+                unsigned m = 0xffffffffu;
 #pragma unroll
-            for (int L = 1; L <= K; ++L) {
-                if (zz < z0 - K + 2 * L) break;  // plane zz - L of level L not computable yet (uniform)
-                // level L-1 planes zz-L+1, zz-L, zz-L-1 sit in slots sp, sc, sm
-                const int sp = ((u - L + 1) % 3 + 3) % 3, sc = ((u - L) % 3 + 3) % 3, sm = ((u - L - 1) % 3 + 3) % 3;
-                const T* P = lds[L - 1][(zz - L) & 1];
-                const int pz = zz - L;  // the plane level L computes
-#pragma unroll
-                for (int m = 0; m < NL; ++m) {
-                    if (L < K ? !at_level(m, L) : !(at_level(m, K) && inr[m])) continue;
-                    const int e = tid + m * NT;
-                    const T c = hist[L - 1][m][sc];
-                    T v = ftcs3<T, MODE>(c, P[e - 1], P[e + 1], P[e - RX], P[e + RX], hist[L - 1][m][sm],
-                                         hist[L - 1][m][sp], a);
-                    if (L < K) {
-                        if (!zper && pz == a.n[2]) v = rule(a, 2, 1, hist[L][m][sm]);  // ghost plane n
-                        hist[L][m][sc] = v;
-                        if (!zper && pz == 0) hist[L][m][sm] = rule(a, 2, 0, v);  // ghost plane -1
-                        lds[L][(zz - L) & 1][e] = v;
-                    } else {
-                        out[sz * (zz - K + 1) + oo[m]] = v;
-                    }
-                }
+                for (int k = 0; k < XW; ++k) m = min(m, min(div_key(dn[k]), div_key(up[k])));
+                again |= (odd[s] & 1) != 0 || __any(m < a.low);
             }
+            if (!again) xypart(std::integral_constant<int, MODE>{});
+            if constexpr (MODE == FTCS_CDIV) {
+                if (again) xypart(std::integral_constant<int, FTCS_DIV>{});
+            }
+        }
+    };
+    for (int t = ta; t < tb; ++t) {
+        plane(t);
+        if (!D64) {  // two planes a round: the held planes change registers by name, not by moves
+            if (++t >= tb) break;
+            plane(t);
         }
     }
 }
@@ -686,27 +690,34 @@ Strip2d strip_plan(const int n[3], const int per[3], int nsteps, int tblock, boo
     return best;
 }
 
-// 3-D blocked launch shape per precision (swept at 512^3 on MI355X): TX x TY
-// columns, NT threads, K steps per launch (a remainder of two steps takes one K = 2
-// launch of the same tile, one step the single-step kernel); the z chunk is chosen per
-// launch (ftcs_t)
-template <typename T>
-struct Ftcs3dCfg;
-template <>
-struct Ftcs3dCfg<double> {
-    static constexpr int TX = 64, TY = 32, NT = 1024, K = 3;
-    static constexpr bool XCD = true;
-};
-template <>
-struct Ftcs3dCfg<float> {
-    static constexpr int TX = 128, TY = 32, NT = 1024, K = 3;
-    static constexpr bool XCD = true;
-};
+// Launches of the 3-D kernel: 64 x 64 cells of a plane in 16 waves of 4 rows, three steps a launch
+// (a remainder of two or one takes a launch of its own). Swept at 512^3 FP64 periodic: 8 waves of 8
+// rows 151 us a step, 128 x 32 cells 202, against 146; four steps fit 64 x 48 cells (162: 130 tiles
+// fill the chip badly) and spill in 64 x 64.
+constexpr int S3_XW = 1, S3_RW = 4, S3_NW = 16, S3_K = 3;
+// Single steps take half the waves and two workgroups a CU while the field and its second buffer
+// stay in the 256 MB last-level cache, where a workgroup's latency bounds them: 128^3 FP64 Dirichlet
+// 14.9 -> 13.2 us, 64^3 9.4 -> 7.4; beyond, the larger region reads less halo (512^3 FP64 609 -> 485).
+constexpr size_t S3_CACHE = (size_t)256 << 20;
 
 // Steps the next launch of a 3-D field advances. tblock = 1 forces single steps.
-int launch_steps3(int dtype, long long plane, int remaining, int tblock) {
-    const int k3 = dtype == OPF_F64 ? Ftcs3dCfg<double>::K : Ftcs3dCfg<float>::K;
-    return tblock != 1 && plane < (1LL << 31) && remaining >= 2 ? std::min(k3, remaining) : 1;
+// The last four are two and two.
+int launch_steps3(int remaining, int tblock) { return tblock == 1 ? 1 : remaining == 4 ? 2 : std::min(S3_K, remaining); }
+
+// Planes per workgroup: a chunk of zc planes costs zc + 2 K plane steps and one workgroup fills a CU,
+// so the cost is that times the rounds the workgroups take; 512^3 FP64 periodic (81 tiles): 171
+// planes, one round of 243, 146 us a step; 128 planes, two rounds, 211; 86, two rounds, 170.
+int chunk_planes(int tiles, int n2, int k, int cus) {
+    int best = n2;
+    long long cost = 0;
+    for (int c = 1; c == 1 || n2 / c >= 2; ++c) {
+        const int zc = (n2 + c - 1) / c;
+        const long long wgs = (long long)tiles * ((n2 + zc - 1) / zc);
+        const long long t = ((wgs + cus - 1) / cus) * (zc + 2 * k);
+        if (c == 1 || t < cost) best = zc, cost = t;
+        if (wgs > 16LL * cus) break;
+    }
+    return best;
 }
 
 bool is_pow2(double h) {
@@ -759,19 +770,21 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
     }
     bool same = true;
     for (int q = 1; q < d.dim; ++q) same &= m->h[q] == m->h[0];
-    int mode = !pow2 ? FTCS_DIV : same ? FTCS_FACTORED : FTCS_MUL;
-    if (mode == FTCS_DIV && d.dim == 2) {
-        bool ok = std::is_same<T, float>::value || div_range(m->h, d.dim, coef, S2_MOST);
+    const int mode = !pow2 ? FTCS_CDIV : same ? FTCS_FACTORED : FTCS_MUL;
+    if (mode == FTCS_CDIV) {
+        constexpr bool f64 = std::is_same<T, double>::value;
+        bool ok = div_range(m->h, d.dim, coef, S2_MOST, f64);
+        a.low = div_low(m->h, d.dim, f64);
         for (int q = 0; q < d.dim; ++q) {
             a.cd[q].h = (double)a.hh[q];
             a.cd[q].y = 1.0 / a.cd[q].h;
             for (int s = 0; s < 2; ++s) {  // a boundary's constant is 0 or well inside the range
                 const GhostRule& r = gi.rule[q][s][0];
                 const double c = std::fabs(r.type == 1 ? r.c2 / r.c3 : r.type == 2 ? r.c1 : 0.0);
-                ok &= c == 0.0 || (c >= 0x1p-400 && c <= 0x1p400);
+                ok &= !f64 || c == 0.0 || (c >= 0x1p-400 && c <= 0x1p400);
             }
         }
-        if (ok) mode = FTCS_CDIV;
+        a.divide = !ok;
     }
     // the Dirichlet rules' divisors, in the form the arithmetic mode takes: reciprocals when every
     // one of them is a power of two
@@ -823,20 +836,17 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
         const T* in = (const T*)cur;
         T* out = (T*)nxt;
         const int k = d.dim == 2 ? std::min(p2.nt, nsteps - it)
-                                 : launch_steps3(d.dtype, (long long)a.e0 * a.e1, nsteps - it, tblock);
-        if (ghosts_stale && !(d.dim == 3 && k > 1 && a.per[0] && a.per[1] && a.per[2])) {
-            OPF_TRY(launch_ghost_fill(f, cur));
-            ghosts_stale = false;
-        }
+                                 : launch_steps3(nsteps - it, tblock);
+        const bool allper = a.per[0] && a.per[1] && a.per[2];
         // launches the kernel instantiated for the arithmetic mode
         auto by_mode = [&](auto launch) {
             if (mode == FTCS_FACTORED) launch(std::integral_constant<int, FTCS_FACTORED>{});
             else if (mode == FTCS_MUL) launch(std::integral_constant<int, FTCS_MUL>{});
-            else launch(std::integral_constant<int, FTCS_DIV>{});
+            else launch(std::integral_constant<int, FTCS_CDIV>{});
         };
         if (d.dim == 2) {
             const unsigned tiles = (unsigned)(((a.n[0] + p2.tx - 1) / p2.tx) * ((a.n[1] + p2.ty - 1) / p2.ty));
-            auto launch2 = [&](auto M) {
+            by_mode([&](auto M) {
                 constexpr int MD = decltype(M)::value;
                 auto with = [&](auto C) {
                     constexpr int c = decltype(C)::value;
@@ -845,46 +855,35 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
                 };
                 if (p2.cfg == 0) with(std::integral_constant<int, 0>{});
                 else if (p2.cfg == 1) with(std::integral_constant<int, 1>{});
-                else if constexpr (MD != FTCS_CDIV && MD != FTCS_DIV) with(std::integral_constant<int, 2>{});
-            };
-            if (mode == FTCS_CDIV) launch2(std::integral_constant<int, FTCS_CDIV>{});
-            else by_mode(launch2);
-        } else if (d.dim == 3 && k > 1) {
-            using C3 = Ftcs3dCfg<T>;
-            const bool allper = a.per[0] && a.per[1] && a.per[2];
-            // z chunk: periodic fields take the longest (each chunk recomputes 2K halo
-            // planes) that still gives every CU a workgroup (one 147 KB workgroup fills a
-            // CU). 512^3 FP64: 256 planes, 256 workgroups, one round: 750 -> 800 G
-            // cell-updates/s against 64-plane chunks (four rounds); FP32 (128-wide tiles)
-            // 128 planes: 1515 -> 1610. With Dirichlet / Neumann sides the workgroups that
-            // rebuild ghosts take longer, and 64-plane chunks (more workgroups than CUs,
-            // balanced by the dispatcher) stay faster (512^3 FP64: 376 vs 330 G/s)
-            const int tiles = ((a.n[0] + C3::TX - 1) / C3::TX) * ((a.n[1] + C3::TY - 1) / C3::TY);
-            int zc = allper ? 256 : 64;
-            while (zc > 16 && (long long)tiles * ((a.n[2] + zc - 1) / zc) < f->ctx->cus) zc /= 2;
-            const int nb = tiles * ((a.n[2] + zc - 1) / zc);
-            static_assert(C3::K == 3, "remainder launches assume K = 3");
+                else if constexpr (MD != FTCS_CDIV) with(std::integral_constant<int, 2>{});
+            });
+        } else if (d.dim == 3) {
+            const bool small = k == 1 && 2 * f->nbytes <= S3_CACHE;
+            const int wx = 64 * S3_XW, wy = S3_RW * (small ? S3_NW / 2 : S3_NW);
+            const int tx = !a.per[0] && a.n[0] + 2 <= wx ? a.n[0] : wx - 2 * k;
+            const int ty = !a.per[1] && a.n[1] + 3 <= wy ? a.n[1] : wy - 2 * k;
+            const int tiles = ((a.n[0] + tx - 1) / tx) * ((a.n[1] + ty - 1) / ty);
+            const int zc = chunk_planes(tiles, a.n[2], k, f->ctx->cus * (small ? 2 : 1));
+            const unsigned nb = (unsigned)tiles * ((a.n[2] + zc - 1) / zc);
+            if (k > 1 && ghosts_stale && !allper) OPF_TRY(launch_ghost_fill(f, cur));
+            a.stale = k == 1 && ghosts_stale && !allper;
             by_mode([&](auto M) {
                 constexpr int MD = decltype(M)::value;
-                if (k == C3::K && allper)
-                    hipLaunchKernelGGL((ftcs3d_tb_kernel<T, MD, C3::TX, C3::TY, C3::NT, C3::K, C3::XCD, true>),
-                                       dim3(nb), dim3(C3::NT), 0, st, in, out, a, zc);
-                else if (k == C3::K)
-                    hipLaunchKernelGGL((ftcs3d_tb_kernel<T, MD, C3::TX, C3::TY, C3::NT, C3::K, C3::XCD, false>),
-                                       dim3(nb), dim3(C3::NT), 0, st, in, out, a, zc);
-                else if (allper)
-                    hipLaunchKernelGGL((ftcs3d_tb_kernel<T, MD, C3::TX, C3::TY, C3::NT, 2, C3::XCD, true>),
-                                       dim3(nb), dim3(C3::NT), 0, st, in, out, a, zc);
-                else
-                    hipLaunchKernelGGL((ftcs3d_tb_kernel<T, MD, C3::TX, C3::TY, C3::NT, 2, C3::XCD, false>),
-                                       dim3(nb), dim3(C3::NT), 0, st, in, out, a, zc);
-            });
-            ghosts_stale = true;
-        } else if (d.dim == 3) {
-            dim3 grid((a.n[0] + FT3_TX - 1) / FT3_TX, (a.n[1] + FT3_TY - 1) / FT3_TY, (a.n[2] + FT3_ZC - 1) / FT3_ZC);
-            by_mode([&](auto M) {
-                hipLaunchKernelGGL((ftcs3d_lds_kernel<T, decltype(M)::value, FT3_ZC, FT3_NTY, FT3_RY>), grid,
-                                   dim3(64, FT3_NTY), 0, st, in, out, a);
+                auto with = [&](auto K_, auto W_) {
+                    constexpr int K = decltype(K_)::value, W = decltype(W_)::value;
+                    if (allper)
+                        hipLaunchKernelGGL((ftcs3d_strip_kernel<T, MD, S3_XW, S3_RW, W, K, true>), dim3(nb),
+                                           dim3(64 * W), 0, st, in, out, a, tx, ty, zc);
+                    else
+                        hipLaunchKernelGGL((ftcs3d_strip_kernel<T, MD, S3_XW, S3_RW, W, K, false>), dim3(nb),
+                                           dim3(64 * W), 0, st, in, out, a, tx, ty, zc);
+                };
+                static_assert(S3_K == 3, "a launch of each remainder");
+                using Whole = std::integral_constant<int, S3_NW>;
+                if (k == 3) with(std::integral_constant<int, 3>{}, Whole{});
+                else if (k == 2) with(std::integral_constant<int, 2>{}, Whole{});
+                else if (!small) with(std::integral_constant<int, 1>{}, Whole{});
+                else with(std::integral_constant<int, 1>{}, std::integral_constant<int, S3_NW / 2>{});
             });
             ghosts_stale = true;
         } else {
@@ -940,7 +939,7 @@ extern "C" int opf_ftcs_plan(const opf_field* u, int nsteps, int tblock, int* la
     const int nt = d.dim == 2 && nsteps > 0 ? strip_plan(n, per, nsteps, tblock, !pow2, u->ctx->cus).nt : 0;
     for (int it = 0; it < nsteps;) {
         const int k = d.dim == 2 ? std::min(nt, nsteps - it)
-                                 : launch_steps3(d.dtype, (long long)d.extent[0] * d.extent[1], nsteps - it, tblock);
+                                 : launch_steps3(nsteps - it, tblock);
         ++*launches;
         *max_steps = std::max(*max_steps, k);
         it += k;

@@ -72,8 +72,8 @@ int main() {
     }
     // the range test of the host
     const double h3[3] = {1. / 300, 1. / 260, 1. / 220}, bad[3] = {1e-40, 1., 1.};
-    if (!opf::div_range(h3, 3, 1e-6, 128) || opf::div_range(bad, 3, 1e-6, 3) || opf::div_range(h3, 3, 1e-50, 3) ||
-        opf::div_range(h3, 3, 1e30, 128))
+    if (!opf::div_range(h3, 3, 1e-6, 128, true) || opf::div_range(bad, 3, 1e-6, 3, true) ||
+        opf::div_range(h3, 3, 1e-50, 3, true) || opf::div_range(h3, 3, 1e30, 128, true))
         return std::printf("div_range\n"), 1;
     std::printf("passed %lld\n", n);
     return 0;
