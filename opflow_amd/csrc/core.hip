@@ -139,14 +139,19 @@ static uint64_t fnv1a(const void* p, size_t n) {
     return h ^ (uint64_t)n;
 }
 
-int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool evictable) {
+int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool evictable, ProgImage image, int* meta) {
     uint64_t h = fnv1a(bytes, n);
     for (auto& p : ctx->progs)
-        if (p.hash == h && p.bytes == n && p.evictable == evictable && std::memcmp(p.host.data(), bytes, n) == 0) {
+        if (p.hash == h && p.bytes == n && p.evictable == evictable && p.image == image &&
+            std::memcmp(p.host.data(), bytes, n) == 0) {
             p.used = ++ctx->prog_tick;
             *dev = p.dev;
+            if (meta) std::copy(p.meta, p.meta + 5, meta);
             return OPF_OK;
         }
+    std::vector<unsigned char> made;
+    int m[5] = {0, 0, 0, 0, 0};
+    if (image) image(bytes, n, made, m);
     if (evictable) {
         size_t ne = 0;
         for (auto& p : ctx->progs) ne += p.evictable;
@@ -161,11 +166,15 @@ int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool e
         }
     }
     void* d = nullptr;
-    OPF_HIP(hipMalloc(&d, n));
-    OPF_HIP(hipMemcpyAsync(d, bytes, n, hipMemcpyHostToDevice, ctx->stream));
+    OPF_HIP(hipMalloc(&d, image ? made.size() : n));
+    OPF_HIP(hipMemcpyAsync(d, image ? made.data() : bytes, image ? made.size() : n, hipMemcpyHostToDevice,
+                           ctx->stream));
     OPF_HIP(hipStreamSynchronize(ctx->stream));
     const unsigned char* b = (const unsigned char*)bytes;
     ctx->progs.push_back({h, d, n, ++ctx->prog_tick, evictable, std::vector<unsigned char>(b, b + n)});
+    ctx->progs.back().image = image;
+    std::copy(m, m + 5, ctx->progs.back().meta);
+    if (meta) std::copy(m, m + 5, meta);
     ++ctx->prog_uploads;
     *dev = d;
     return OPF_OK;

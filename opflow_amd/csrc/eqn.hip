@@ -294,6 +294,7 @@ struct opf_eqn {
     // unknown read from a zero field whose ghosts hold the boundary constants
     LoweredProgram Pb;
     void* progb = nullptr;
+    DagInfo dagb;
     void* zbuf = nullptr;
     opf_solve_params params{};
     int s[3], n[3];
@@ -374,7 +375,7 @@ static int eqn_eval_bias(opf_eqn* e) {
         OPF_TRY(lower_tree(e->all.data(), (int)e->all.size(), (int)e->all.size() - 1, fl.data(), nf + 1, t->mesh, nf,
                            &e->Pb, true));
         OPF_TRY(check_bounds(e->Pb, fl.data(), nf + 1, t->mesh, e->s, e->n));
-        OPF_TRY(upload_program(ctx, e->Pb.code.data(), e->Pb.code.size() * sizeof(Insn), &e->progb));
+        OPF_TRY(upload_sweep(ctx, e->Pb.code, false, &e->progb, &e->dagb));
     }
     OPF_TRY(launch_ghost_fill(t, e->zbuf));  // boundary constants (values may change between solves)
     SweepArgs a{};
@@ -400,7 +401,7 @@ static int eqn_eval_bias(opf_eqn* e) {
     a.code = e->progb;
     a.ncode = (int)e->Pb.code.size();
     (void)st;
-    return launch_sweep(ctx, OPF_F64, a, e->Pb);
+    return launch_sweep(ctx, OPF_F64, a, e->Pb, e->dagb);
 }
 
 // rows -> multigrid hierarchy of a single equation, on the device (the rows are

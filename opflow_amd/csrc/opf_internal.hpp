@@ -62,6 +62,9 @@ struct opf_ctx {
         uint64_t used;
         bool evictable;
         std::vector<unsigned char> host;
+        // how the device's copy was made from the bytes (null: it is them), what its maker says of it
+        void (*image)(const void*, size_t, std::vector<unsigned char>&, int[5]) = nullptr;
+        int meta[5] = {0, 0, 0, 0, 0};
     };
     static constexpr size_t kMaxPrograms = 1024;
     std::vector<ProgEntry> progs;
@@ -120,6 +123,10 @@ int gen_bumps_grid_dev(hipStream_t st, int dim, const int n[3], uint64_t seed, i
 // device program cache
 // evictable: the caller uses *dev only for launches enqueued right away (a sweep),
 // so the cache may free it later, after a drain of the context's stream
-int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool evictable = false);
+// image (optional) makes the device's form of the bytes, when they are uploaded, and what a launch
+// needs to know of it (meta)
+using ProgImage = void (*)(const void* bytes, size_t n, std::vector<unsigned char>& out, int meta[5]);
+int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool evictable = false,
+                   ProgImage image = nullptr, int* meta = nullptr);
 
 }  // namespace opf

@@ -7,12 +7,17 @@
 // spells out each operator's mesh arithmetic in the reference's operation
 // order, so FP64 results match OpFlow's evaluation bit for bit. The program
 // is a straight line of stack instructions; every lane runs the same
-// instruction stream (uniform control flow) and keeps the stack in LDS.
+// instruction stream (uniform control flow). The interpreter runs it as bundles of
+// independent operations on values in LDS (sweep_dag.hpp), programs with more values
+// than that form holds with their stack in LDS.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
+#include "fastdiv.hpp"
 #include "opf_internal.hpp"
 #include "sweep.hpp"
+#include "sweep_dag.hpp"
 
 using namespace opf;
 
@@ -615,6 +620,119 @@ __global__ __launch_bounds__(256) void sweep_kernel(SweepArgs a) {
     ((T*)a.out)[lo] = v;
 }
 
+// where a load of a bundled program reads: element ofs + i s0 + j s1 + k s2 + b of p
+struct DagSrc {
+    const void* p;
+    int s0, s1;
+    long long s2, b;
+};
+struct DagArgs {
+    DagSrc src[14];
+    DagInfo info;
+    FastDiv n0;
+};
+
+// The bundled program over consecutive cells of a plane, 64 a wave (no lane idles at the end of a
+// row). Bound by a wave's own latencies where a CU has few of them, by LDS and instruction issue
+// elsewhere. us per sweep with its ghost fill, stack program -> bundles: QUICK transport 96 x 80 cells
+// FP64 85 -> 29 (77 -> 20 the kernel), 24 x 20 85 -> 28, 500^2 163 -> 79, 1500^2 1005 -> 538; FTCS
+// 96 x 80 22 -> 16, 1500^2 208 -> 95; WENO 500^2 22 -> 19; u 2 + 1, 1500^2 28 -> 24 (FP32 19 -> 20).
+template <typename T>
+__global__ __launch_bounds__(256) void sweep_dag_kernel(SweepArgs a, DagArgs g) {
+    extern __shared__ __attribute__((aligned(16))) char dag_lds[];
+    const int lane = threadIdx.x & 63;
+    T* uni = (T*)dag_lds + (blockDim.x >> 6) * (g.info.nslot * 64);       // constants
+    T* val = (T*)dag_lds + (int)(threadIdx.x >> 6) * g.info.nslot * 64;   // val[slot * 64 + lane]
+    const unsigned cells = (unsigned)a.n[0] * (unsigned)a.n[1], t = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned c = min(t, cells - 1);  // lanes past the end walk the program on the last cell
+    const unsigned row = g.n0.div(c);
+    const int i = a.s[0] + (int)(c - row * g.n0.d), j = a.s[1] + (int)row;
+    const int k = a.s[2] + (int)blockIdx.z;
+    const DagBundle* __restrict__ code = (const DagBundle*)a.code;
+    const DagLoad* __restrict__ ld = (const DagLoad*)(code + g.info.nbundle + 1);
+    const DagUni* __restrict__ un = (const DagUni*)(ld + dag_loads(g.info.nload));
+    for (int q = threadIdx.x; q < g.info.nuni; q += blockDim.x) uni[q] = un[q].slot >= 0 ? (T)a.cst[un[q].slot] : (T)un[q].imm;
+    auto load = [&](int l, auto W_) __attribute__((always_inline)) {
+        constexpr int W = decltype(W_)::value;
+        T v[W];
+#pragma unroll
+        for (int q = 0; q < W; ++q) {
+            const DagSrc& s = g.src[ld[l + q].src];
+            const T* p = (const T*)s.p + (s.s2 * k + s.b + ld[l + q].ofs);
+            v[q] = p[(long long)i * s.s0 + (long long)j * s.s1];
+        }
+#pragma unroll
+        for (int q = 0; q < W; ++q) val[ld[l + q].d * 64 + lane] = v[q];
+    };
+    {
+        int l = 0;
+        for (; l + DAG_LOADS <= g.info.nload; l += DAG_LOADS) load(l, std::integral_constant<int, DAG_LOADS>{});
+        if (l + 8 <= g.info.nload) load(l, std::integral_constant<int, 8>{}), l += 8;
+        if (l + 4 < g.info.nload) load(l, std::integral_constant<int, 8>{}), l += 8;
+        else if (l + 1 < g.info.nload) load(l, std::integral_constant<int, 4>{}), l += 4;
+        else if (l < g.info.nload) load(l, std::integral_constant<int, 1>{});
+    }
+    __syncthreads();  // the constants were written by other lanes
+    auto at = [&](int w) __attribute__((always_inline)) -> T& {
+        return (w & 1) ? val[(w >> 1) * 64 + lane] : uni[w >> 1];
+    };
+    auto run = [&](const DagBundle& in, auto W_) __attribute__((always_inline)) {
+        constexpr int W = decltype(W_)::value;
+        T x[W], y[W], z[W];
+#pragma unroll
+        for (int q = 0; q < W; ++q) x[q] = at(in.a[q]), y[q] = at(in.b[q]);
+#define DAG_OP(E)                                              \
+    _Pragma("unroll") for (int q = 0; q < W; ++q) z[q] = (E); \
+    break
+        switch (in.op) {
+            case I_ADD: DAG_OP(x[q] + y[q]);
+            case I_SUB: DAG_OP(x[q] - y[q]);
+            case I_MUL: DAG_OP(x[q] * y[q]);
+            case I_DIV: DAG_OP(x[q] / y[q]);
+            case I_NEG: DAG_OP(-x[q]);
+            case I_MIN: DAG_OP(y[q] < x[q] ? y[q] : x[q]);
+            case I_MAX: DAG_OP(x[q] < y[q] ? y[q] : x[q]);
+            case I_ABS: DAG_OP(fabs(x[q]));
+            case I_GT: DAG_OP(x[q] > y[q] ? (T)1 : (T)0);
+            case I_LT: DAG_OP(x[q] < y[q] ? (T)1 : (T)0);
+            case I_GE: DAG_OP(x[q] >= y[q] ? (T)1 : (T)0);
+            case I_LE: DAG_OP(x[q] <= y[q] ? (T)1 : (T)0);
+            default:
+                if constexpr (W == 1) {
+                    if (in.op == I_SEL) z[0] = x[0] != (T)0 ? y[0] : at(in.a[1]);
+                    else if (in.op == I_FN1) z[0] = interp_fn1<T>(in.sub, x[0]);
+                    else if (in.op == I_FN2) z[0] = interp_fn2<T>(in.sub, x[0], y[0]);
+                    else
+                        z[0] = weno_kernel<T>(x[0], at(in.a[1]), at(in.a[2]), at(in.a[3]), y[0], at(in.b[1]),
+                                              at(in.b[2]), in.op == I_WENO_UP);
+                }
+        }
+#undef DAG_OP
+#pragma unroll
+        for (int q = W - 1; q >= 0; --q) val[(in.d[q] >> 1) * 64 + lane] = z[q];
+    };
+    DagBundle nx = code[0];
+    for (int pc = 0; pc < g.info.nbundle; ++pc) {
+        const DagBundle in = nx;
+        nx = code[pc + 1];
+        if (in.count == 1) run(in, std::integral_constant<int, 1>{});
+        else run(in, std::integral_constant<int, DAG_W>{});
+    }
+    if (t >= cells) return;
+    T v = at(g.info.result);
+    const long long lo = (i - a.oo[0]) + (long long)a.oe0 * ((j - a.oo[1]) + (long long)a.oe1 * (k - a.oo[2]));
+    if (a.op != OPF_OP_EQ) {
+        const T old = ((const T*)a.old)[lo];
+        switch (a.op) {
+            case OPF_OP_ADD: v = old + v; break;
+            case OPF_OP_MINUS: v = old - v; break;
+            case OPF_OP_MUL: v = old * v; break;
+            case OPF_OP_DIV: v = old / v; break;
+        }
+    }
+    ((T*)a.out)[lo] = v;
+}
+
 }  // namespace opf
 
 namespace opf {
@@ -642,7 +760,23 @@ void uniform_spacing(const opf_mesh* m, int dtype, SweepArgs& a) {
     }
 }
 
-int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProgram& P) {
+int upload_sweep(opf_ctx* ctx, const std::vector<Insn>& code, bool evictable, void** dev, DagInfo* dag) {
+    const ProgImage image = [](const void* bytes, size_t n, std::vector<unsigned char>& out, int meta[5]) {
+        DagInfo d;
+        const Insn* c = (const Insn*)bytes;
+        if (!DagBuilder().build(c, n / sizeof(Insn), out, d)) {
+            d = DagInfo{};
+            out.assign((const unsigned char*)bytes, (const unsigned char*)bytes + n);
+        }
+        meta[0] = d.nload, meta[1] = d.nuni, meta[2] = d.nbundle, meta[3] = d.nslot, meta[4] = d.result;
+    };
+    int m[5];
+    OPF_TRY(upload_program(ctx, code.data(), code.size() * sizeof(Insn), dev, evictable, image, m));
+    *dag = {m[0], m[1], m[2], m[3], m[4]};
+    return OPF_OK;
+}
+
+int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProgram& P, const DagInfo& dag) {
     hipStream_t st = ctx->stream;
     SweepArgs a = a0;
     OPF_CHECK(P.consts.size() <= (size_t)SWEEP_MAX_CONSTS, OPF_ERR_ARG, "sweep: %zu constant slots",
@@ -658,6 +792,30 @@ int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProg
         // runs the same program on the interpreter (same bits); argument errors stand
         if (rc != OPF_ERR_HIP) return rc;
         (void)hipGetLastError();
+    }
+    if (dag.nslot > 0 && (long long)a.n[0] * a.n[1] < (1LL << 31)) {
+        DagArgs g{};
+        g.n0 = FastDiv((uint32_t)a.n[0]);
+        for (int f = 0; f < SWEEP_MAX_FIELDS; ++f) {
+            const FieldArg& F = a.f[f];
+            const long long e1 = F.e1, e0 = F.e0;
+            g.src[f] = {F.ptr, 1, F.e0, e0 * e1, -(F.off0 + e0 * (F.off1 + e1 * F.off2))};
+        }
+        for (int d = 0; d < 3; ++d)
+            for (int q = 0; q < 2; ++q)
+                g.src[8 + 3 * q + d] = {q ? a.x[d] : a.dx[d], d == 0, d == 1, d == 2, -(long long)a.morg[d]};
+        g.info = dag;
+        // small programs of many cells take up to four waves a workgroup, where starting workgroups
+        // of one would bound them (u 2 + 1, 1500^2: 55 us with one); with fewer than four waves a CU
+        // they are spread over the CUs, and programs with many values would leave a CU one workgroup
+        int waves = 1;
+        while (waves < 4 && cells >= 4LL * 64 * ctx->cus * waves && dag.nslot * waves <= DAG_MAX_SLOTS / 2) waves *= 2;
+        const dim3 gd((unsigned)(((long long)a.n[0] * a.n[1] + 64 * waves - 1) / (64 * waves)), 1, a.n[2]);
+        const size_t lds = ((size_t)dag.nslot * 64 * waves + dag.nuni + 1) * dtype_size(dtype);
+        if (dtype == OPF_F64) hipLaunchKernelGGL(sweep_dag_kernel<double>, gd, dim3(64 * waves), lds, st, a, g);
+        else hipLaunchKernelGGL(sweep_dag_kernel<float>, gd, dim3(64 * waves), lds, st, a, g);
+        OPF_HIP(hipGetLastError());
+        return OPF_OK;
     }
     dim3 grid((a.n[0] + 63) / 64, (a.n[1] + 3) / 4, a.n[2]);
     if (dtype == OPF_F64) hipLaunchKernelGGL(sweep_kernel<double>, grid, dim3(64, 4), 0, st, a);
@@ -754,11 +912,11 @@ extern "C" int opf_sweep(const opf_expr_node* nodes, int nnodes, int root, opf_f
         a.out = target;
         a.old = out->data;
         void* dev = nullptr;
-        const std::vector<Insn> sc = structural_code(P);
-        OPF_TRY(upload_program(ctx, sc.data(), sc.size() * sizeof(Insn), &dev, true));
+        DagInfo dag;
+        OPF_TRY(upload_sweep(ctx, structural_code(P), true, &dev, &dag));
         a.code = dev;
         a.ncode = (int)P.code.size();
-        OPF_TRY(launch_sweep(ctx, d.dtype, a, P));
+        OPF_TRY(launch_sweep(ctx, d.dtype, a, P, dag));
         if (inplace) std::swap(out->data, out->spare);
     }
     return launch_ghost_fill(out, out->data);

@@ -74,9 +74,15 @@ int lower_tree(const opf_expr_node* nodes, int nnodes, int root, opf_field* cons
 int lower_tree_set(const opf_expr_node* nodes, int nnodes, int root, opf_field* const* fields, int nfields,
                    const opf_mesh* mesh, const int* unknown_slots, int nunknown, LoweredProgram* out,
                    bool unknown_as_field = false);
+// a sweep program in the interpreter's form (sweep_dag.hpp); nslot = 0: as the stack program
+struct DagInfo {
+    int nload = 0, nuni = 0, nbundle = 0, nslot = 0, result = 0;
+};
+// the interpreter's form of a stack program on the device
+int upload_sweep(opf_ctx* ctx, const std::vector<Insn>& code, bool evictable, void** dev, DagInfo* dag);
 // the sweep of program P over the box [a.s, a.s + a.n) on the context's stream, by the
 // engine the context's jit mode selects (interpreter or the compiled kernel of P)
-int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a, const LoweredProgram& P);
+int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a, const LoweredProgram& P, const DagInfo& dag);
 // the compiled kernel of P (hipRTC, cached) and its launch; form 0 = by grid size,
 // 1 = direct (loads from HBM), 2 = staged in LDS where the program allows
 int jit_launch_sweep(hipStream_t st, const LoweredProgram& P, int dtype, const SweepArgs& a, int form = 0);
