@@ -258,6 +258,14 @@ extern "C" int opf_mesh_create(opf_ctx* ctx, int dim, const int start[3], const 
         for (int i = 1; i < nx - 1; ++i) uni &= (m->hdx[d][i] == m->hdx[d][0]);
         m->uniform[d] = uni;
         m->h[d] = m->hdx[d][0];
+        int e;
+        if (uni && m->h[d] > 0 && std::frexp(m->h[d], &e) == 0.5) {
+            const double h = m->h[d];
+            bool whole = std::fmod(m->hx[d][0], h) == 0.0;
+            for (int i = 1; i < nx; ++i) whole &= m->hx[d][i] - m->hx[d][i - 1] == h;
+            const double far = std::max(std::fabs(m->hx[d][0]), std::fabs(m->hx[d][nx - 1])) / h;
+            if (whole && far < 0x1p50) m->span[d] = far;
+        }
         OPF_HIP(hipMalloc(&m->x_dev[d], nx * sizeof(double)));
         OPF_HIP(hipMalloc(&m->dx_dev[d], (nx - 1) * sizeof(double)));
         OPF_HIP(hipMemcpy(m->x_dev[d], m->hx[d].data(), nx * sizeof(double), hipMemcpyHostToDevice));

@@ -73,39 +73,303 @@ std::string hexkey(uint64_t h) {
     return buf;
 }
 
-// Values a generator knows to be s * h_d, a power-of-two multiple s of the uniform
-// power-of-two spacing h_d of dim d (a dx of that dim, sums of two such, scalings by
-// a power-of-two literal), and literal constants. A division by s * h_d is emitted
-// as the multiplication by 1 / (s * h_d): both round the same real number, so the
-// bits are the reference's.
+// Values a generator knows in terms of the uniform spacing h_d of one dim d: (x_i of that dim, where
+// kx is set) + s * h_d for a small multiple s of 1/4, and literal constants. h_d is a power of two
+// (umask) or any h (cmask: values that are s * h_d for a power of two s); x_i only where every
+// coordinate is a whole multiple of a power-of-two h_d (xmask). All of it is exact, so such a value
+// needs no table and no operation, and a division by one is
+//   s and h_d powers of two: the multiplication by 1 / (s * h_d), which rounds the same real number;
+//   else: const_div (constdiv.hpp) with the reciprocal of s * h_d.
+// The reference's linear interpolation to faces divides by a difference of such values per face, so
+// on these meshes it has no division left: flux form of a variable diffusion at 256^3 FP64, bound by
+// its divisions before and by memory now, 173 -> 109 us (402 MB).
 struct Known {
-    std::vector<signed char> d;  // dim of a known multiple, -1 none
-    std::vector<double> s;       // its multiple
+    std::vector<signed char> d;  // dim of a known value, -1 none
+    std::vector<char> kx;        // 1: x_i + s h
+    std::vector<double> s;
     std::vector<char> lit;       // a literal constant
     std::vector<double> c;       // its value
-    explicit Known(size_t n) : d(n, -1), s(n, 0.0), lit(n, 0), c(n, 0.0) {}
+    int umask, cmask, xmask;
+    Known(size_t n, const SweepArgs& a)
+        : d(n, -1), kx(n, 0), s(n, 0.0), lit(n, 0), c(n, 0.0), umask(a.umask), cmask(a.cmask), xmask(a.xmask) {}
     static bool pow2(double v, int lo, int hi) {
         int e;
         return v > 0 && std::frexp(v, &e) == 0.5 && e - 1 >= lo && e - 1 <= hi;
     }
-    void dx(int id, int dim) { d[id] = (signed char)dim, s[id] = 1.0; }
+    bool has(int mask, int dim) const { return mask >> dim & 1; }
+    void set(int id, int dim, int k, double v) {
+        // a multiple of 1/4 up to 4 h (and not 0, whose sign a later product would need), or of a
+        // general h a power of two, which scales it exactly
+        if (k == 0 && (v == 0 || std::fabs(v) > 4.0 || v * 4 != std::floor(v * 4))) return;
+        if (k == 1 && (!has(xmask, dim) || std::fabs(v) > 64 || v * 4 != std::floor(v * 4))) return;
+        if (k < 0 || k > 1 || (!has(umask, dim) && !pow2(v, -2, 2))) return;
+        d[id] = (signed char)dim, kx[id] = (char)k, s[id] = v;
+    }
+    bool dx(int id, int dim) {
+        if (has(umask | cmask, dim)) set(id, dim, 0, 1.0);
+        return d[id] >= 0;
+    }
+    void x(int id, int dim, int shift) {
+        if (has(xmask, dim)) set(id, dim, 1, shift);
+    }
     void literal(int id, double v) { lit[id] = 1, c[id] = v; }
     // result id of x op y
     void arith(int op, int id, int x, int y) {
-        if (op == I_ADD && d[x] >= 0 && d[x] == d[y] && pow2(s[x] + s[y], -2, 2)) d[id] = d[x], s[id] = s[x] + s[y];
+        if (op == I_ADD && d[x] >= 0 && d[x] == d[y]) set(id, d[x], kx[x] + kx[y], s[x] + s[y]);
+        if (op == I_SUB && d[x] >= 0 && d[x] == d[y] && has(umask, d[x])) set(id, d[x], kx[x] - kx[y], s[x] - s[y]);
         if (op == I_MUL) {
-            if (d[x] >= 0 && lit[y] && pow2(s[x] * c[y], -2, 2)) d[id] = d[x], s[id] = s[x] * c[y];
-            if (d[y] >= 0 && lit[x] && pow2(s[y] * c[x], -2, 2)) d[id] = d[y], s[id] = s[y] * c[x];
+            if (d[x] >= 0 && !kx[x] && lit[y]) set(id, d[x], 0, s[x] * c[y]);
+            if (d[y] >= 0 && !kx[y] && lit[x]) set(id, d[y], 0, s[y] * c[x]);
         }
     }
-    // the multiplication replacing x / y, or an empty string
-    std::string div(int x, int y) const {
-        if (d[y] < 0) return "";
+    // s * h_d as an expression, empty when the value is not one
+    std::string constant(int id) const {
+        if (d[id] < 0 || kx[id]) return "";
         char b[96];
-        snprintf(b, sizeof b, "v%d * ((T)a.rdx[%d] * (T)%a)", x, d[y], 1.0 / s[y]);
+        snprintf(b, sizeof b, "(T)a.hdx[%d] * (T)%a", d[id], s[id]);
         return b;
     }
 };
+
+// A cell's program as straight-line code, values <pre><id>. fast: the divisions FP64 can do through a
+// reciprocal, guarded (lo_, hi_: the bounds of the numerators met, see kGuardSrc); else every one as
+// a division.
+struct CellGen {
+    const LoweredProgram& P;
+    int dtype;
+    bool fast;      // emit guarded divisions
+    bool guarded = false;  // some were
+    bool opaque = false;   // the program can drop a NaN: comparisons, selections, functions
+    CellGen(const LoweredProgram& p, int dt, bool f) : P(p), dtype(dt), fast(f && dt == OPF_F64) {
+        for (const Insn& in : P.code)
+            opaque |= in.op == I_MIN || in.op == I_MAX || in.op == I_GT || in.op == I_LT || in.op == I_GE ||
+                      in.op == I_LE || in.op == I_SEL || in.op == I_FN1 || in.op == I_FN2;
+    }
+    // x / y, or the multiplication or const_div that gives the same bits
+    std::string div(const Known& kn, char pre, int x, int y) {
+        char b[256];
+        const int d = kn.d[y];
+        const double s = kn.s[y];
+        const char* bound = opaque ? "opf_cdivb(lo_, hi_, " : "opf_cdiv(lo_, ";
+        if (d >= 0 && !kn.kx[y] && kn.has(kn.umask, d) && Known::pow2(std::fabs(s), -2, 2)) {
+            snprintf(b, sizeof b, "%c%d * ((T)a.rdx[%d] * (T)%a)", pre, x, d, 1.0 / s);
+            return b;
+        }
+        if (fast && d >= 0 && !kn.kx[y] && kn.has(kn.cmask, d)) {
+            snprintf(b, sizeof b, "%s%c%d, a.hdx[%d] * %a, a.rdx[%d] * %a)", bound, pre, x, d, s, d, 1.0 / s);
+            guarded = true;
+            return b;
+        }
+        const double c = kn.c[y], m = std::fabs(c);
+        if (fast && kn.lit[y] && m >= 0x1p-100 && m <= 0x1p100 && !Known::pow2(m, -200, 200)) {
+            snprintf(b, sizeof b, "%s%c%c%d, %a, %a)", bound, c < 0 ? '-' : ' ', pre, x, m, 1.0 / m);
+            guarded = true;
+            return b;
+        }
+        snprintf(b, sizeof b, "%c%d / %c%d", pre, x, pre, y);
+        return b;
+    }
+    // ld(instruction), tab(instruction): the expressions of a load and a mesh table entry
+    template <typename Ld, typename Tab>
+    int emit(std::string& out, Known& kn, char pre, int base, Ld&& ld, Tab&& tab, int* result) {
+        std::vector<int> st;
+        char line[512];
+        auto pop = [&](int& v) -> bool {
+            if (st.empty()) return false;
+            v = st.back();
+            st.pop_back();
+            return true;
+        };
+        int id = base;
+        for (const Insn& in : P.code) {
+            std::string e;
+            int x, y, z;
+            switch (in.op) {
+                case I_LD: e = ld(in); break;
+                case I_CONST:
+                    if (in.a) {  // launch-time constant: the source does not depend on its value
+                        e = "(T)a.cst[" + std::to_string(in.b) + "]";
+                        break;
+                    }
+                    long long bits;
+                    std::memcpy(&bits, &in.imm, 8);
+                    e = "(T)__longlong_as_double(" + std::to_string(bits) + "LL)";
+                    kn.literal(id, in.imm);
+                    break;
+                case I_DX: e = kn.dx(id, in.a) ? kn.constant(id) : tab(in); break;
+                case I_X:
+                    e = tab(in);
+                    kn.x(id, in.a, in.b);
+                    break;
+                case I_ADD:
+                case I_SUB:
+                case I_MUL:
+                case I_DIV:
+                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
+                    kn.arith(in.op, id, x, y);
+                    e = kn.constant(id);
+                    if (!e.empty()) break;
+                    if (in.op == I_DIV) {
+                        e = div(kn, pre, x, y);
+                        break;
+                    }
+                    snprintf(line, sizeof line, "%c%d %c %c%d", pre, x, in.op == I_ADD ? '+' : in.op == I_SUB ? '-' : '*',
+                             pre, y);
+                    e = line;
+                    break;
+                case I_NEG:
+                case I_ABS:
+                    if (!pop(x)) return OPF_ERR_ARG;
+                    snprintf(line, sizeof line, in.op == I_NEG ? "-%c%d" : "(T)fabs((double)%c%d)", pre, x);
+                    e = line;
+                    break;
+                case I_MIN:  // std::min(a, b) = b < a ? b : a
+                case I_MAX:  // std::max(a, b) = a < b ? b : a
+                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
+                    snprintf(line, sizeof line, "%c%d < %c%d ? %c%d : %c%d", pre, in.op == I_MIN ? y : x, pre,
+                             in.op == I_MIN ? x : y, pre, y, pre, x);
+                    e = line;
+                    break;
+                case I_GT:
+                case I_LT:
+                case I_GE:
+                case I_LE:
+                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
+                    snprintf(line, sizeof line, "%c%d %s %c%d ? (T)1 : (T)0", pre, x,
+                             in.op == I_GT ? ">" : in.op == I_LT ? "<" : in.op == I_GE ? ">=" : "<=", pre, y);
+                    e = line;
+                    break;
+                case I_FN1:
+                    if (!pop(x)) return OPF_ERR_ARG;
+                    snprintf(line, sizeof line, "opf_fn1<T>(%d, %c%d)", in.a, pre, x);
+                    e = line;
+                    break;
+                case I_FN2:
+                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
+                    snprintf(line, sizeof line, "opf_fn2<T>(%d, %c%d, %c%d)", in.a, pre, x, pre, y);
+                    e = line;
+                    break;
+                case I_SEL:
+                    if (!pop(z) || !pop(y) || !pop(x)) return OPF_ERR_ARG;
+                    snprintf(line, sizeof line, "%c%d != (T)0 ? %c%d : %c%d", pre, x, pre, y, pre, z);
+                    e = line;
+                    break;
+                case I_WENO_UP:
+                case I_WENO_DOWN: {
+                    int h, v[6];
+                    if (!pop(h)) return OPF_ERR_ARG;
+                    for (int q = 5; q >= 0; --q)
+                        if (!pop(v[q])) return OPF_ERR_ARG;
+                    const bool quick = fast && !opaque;
+                    e = quick ? "weno_guarded(lo_, nb_" : "weno_kernel<T>(";
+                    for (int q = 0; q < 6; ++q) {
+                        snprintf(line, sizeof line, "%s%c%d", q || quick ? ", " : "", pre, v[q]);
+                        e += line;
+                    }
+                    const int d = kn.d[h];
+                    if (quick && d >= 0 && !kn.kx[h])
+                        snprintf(line, sizeof line, ", a.hdx[%d] * %a, a.rdx[%d] * %a, %s)", d, kn.s[h], d, 1.0 / kn.s[h],
+                                 in.op == I_WENO_UP ? "true" : "false");
+                    else if (quick)
+                        snprintf(line, sizeof line, ", %c%d, 0.0, %s)", pre, h, in.op == I_WENO_UP ? "true" : "false");
+                    else
+                        snprintf(line, sizeof line, ", %c%d, %s)", pre, h, in.op == I_WENO_UP ? "true" : "false");
+                    e += line;
+                    guarded |= quick;
+                } break;
+                default: return OPF_ERR_ARG;
+            }
+            out += "    const T " + std::string(1, pre) + std::to_string(id) + " = " + e + ";\n";
+            st.push_back(id++);
+        }
+        if (st.size() != 1) return OPF_ERR_ARG;
+        *result = st.back();
+        return OPF_OK;
+    }
+};
+
+// The guarded divisions of a generated cell (FP64). opf_cdiv is const_div; it rounds as the division
+// for numerators of 0 or at least 2^-600 by divisors in [2^-102, 2^102], and gives NaN where it
+// overflows or its numerator is not finite. lo_ keeps the least key (magnitude's high word, 0 the
+// largest), hi_ the largest magnitude where a program could drop the NaN; else the cell's value shows
+// it. weno_guarded: weno_kernel with its divisions by h, 3 and 6 as const_div on differences of 0 or
+// at least 2^-600 (so those of its derivatives by 3 and 6 are in range too), rh = 0: h of no known
+// reciprocal, divided by; and its three weights through the reciprocal of their sum, for
+// a_i >= 2^-300 and a sum up to 2^700 (nb_ otherwise). An FP64 division is some 17 issue slots, a
+// const_div 3 and its key 2: WENO53 in two dims at 1000 x 900 cells, of 40 divisions a cell, 29 -> 19 us.
+const char* const kGuardSrc = R"(
+__device__ __forceinline__ unsigned opf_key(double x) {
+    unsigned k; asm("v_lshl_add_u32 %0, %1, 1, -1" : "=v"(k) : "v"(__double2hiint(x))); return k;
+}
+__device__ __forceinline__ double opf_cd(double x, double h, double y) {
+    const double q = x * y; return __builtin_fma(-__builtin_fma(h, q, -x), y, q);
+}
+__device__ __forceinline__ double opf_cdiv(unsigned& lo, double x, double h, double y) {
+    lo = min(lo, opf_key(x)); return opf_cd(x, h, y);
+}
+__device__ __forceinline__ double opf_cdivb(unsigned& lo, int& hi, double x, double h, double y) {
+    lo = min(lo, opf_key(x)); hi = max(hi, __double2hiint(x) & 0x7fffffff); return opf_cd(x, h, y);
+}
+__device__ __forceinline__ double weno_guarded(unsigned& lo, bool& nb, double v0, double v1, double v2, double v3, double v4,
+                                               double v5, double h, double rh, bool up) {
+    double d1 = v1 - v0, d2 = v2 - v1, d3 = v3 - v2, d4 = v4 - v3, d5 = v5 - v4;
+    lo = min(min(min(lo, opf_key(d1)), min(opf_key(d2), opf_key(d3))), min(opf_key(d4), opf_key(d5)));
+    if (rh != 0) { d1 = opf_cd(d1, h, rh); d2 = opf_cd(d2, h, rh); d3 = opf_cd(d3, h, rh); d4 = opf_cd(d4, h, rh); d5 = opf_cd(d5, h, rh); }
+    else { d1 = d1 / h; d2 = d2 / h; d3 = d3 / h; d4 = d4 / h; d5 = d5 / h; nb |= !(__builtin_fabs(h) <= 0x1p100); }
+    if (up) { double t = d1; d1 = d5; d5 = t; t = d2; d2 = d4; d4 = t; }
+    const double c1312 = 13. / 12., y3 = 1. / 3., y6 = 1. / 6.;
+    double ddx1 = opf_cd(d1, 3., y3) - opf_cd(7. * d2, 6., y6) + opf_cd(11. * d3, 6., y6);
+    double ddx2 = opf_cd(-d2, 6., y6) + opf_cd(5. * d3, 6., y6) + opf_cd(d4, 3., y3);
+    double ddx3 = opf_cd(d3, 3., y3) + opf_cd(5. * d4, 6., y6) - opf_cd(d5, 6., y6);
+    double t1 = d1 - 2. * d2 + d3, t2 = d1 - 4. * d2 + 3. * d3;
+    double s1 = c1312 * (t1 * t1) + (t2 * t2) / 4;
+    double t3 = d2 - 2. * d3 + d4, t4 = d2 - d4;
+    double s2 = c1312 * (t3 * t3) + (t4 * t4) / 4.;
+    double t5 = d3 - 2. * d4 + d5, t6 = 3. * d3 - 4. * d4 + d5;
+    double s3 = c1312 * (t5 * t5) + (t6 * t6) / 4.;
+    double m = d1 * d1;
+    double q = d2 * d2; m = m < q ? q : m;
+    q = d3 * d3; m = m < q ? q : m;
+    q = d4 * d4; m = m < q ? q : m;
+    q = d5 * d5; m = m < q ? q : m;
+    const double eps = 1e-6 * m + 1e-99;
+    double e1 = s1 + eps, e2 = s2 + eps, e3 = s3 + eps;
+    double a1 = .1 / (e1 * e1);
+    double a2 = .6 / (e2 * e2);
+    double a3 = .3 / (e3 * e3);
+    const double S = a1 + a2 + a3, y = 1.0 / S;
+    nb |= !(__builtin_fmin(__builtin_fmin(a1, a2), a3) >= 0x1p-300 && S <= 0x1p700);
+    return opf_cd(a1, S, y) * ddx1 + opf_cd(a2, S, y) * ddx2 + opf_cd(a3, S, y) * ddx3;
+}
+)";
+
+// The value of a cell as T <name>: the guarded form where it has one, redone with divisions by the
+// waves that met a value out of its range.
+template <typename Ld, typename Tab>
+int emit_cell(const LoweredProgram& P, int dtype, const SweepArgs& a, int base, Ld&& ld, Tab&& tab,
+              const std::string& name, std::string& s) {
+    int res = 0;
+    std::string body;
+    CellGen fast(P, dtype, true);
+    {
+        Known kn((size_t)base + P.code.size(), a);
+        OPF_TRY(fast.emit(body, kn, 'v', base, ld, tab, &res));
+    }
+    s += "    T " + name + ";\n    {\n";
+    if (fast.guarded) s += "    unsigned lo_ = 0xffffffffu; int hi_ = 0; bool nb_ = false;\n";
+    s += body + "    " + name + " = v" + std::to_string(res) + ";\n";
+    if (fast.guarded) {
+        // 2^-600 as a key, 2^700 as a high word
+        s += "    if (__any(nb_ || lo_ < ((1023u - 600u) << 21) - 1u || hi_ >= (1023 + 700) << 20 || !(fabs(" + name +
+             ") < __builtin_inf()))) {\n";
+        CellGen slow(P, dtype, false);
+        Known kn((size_t)base + P.code.size(), a);
+        OPF_TRY(slow.emit(s, kn, 'w', base, ld, tab, &res));
+        s += "    " + name + " = w" + std::to_string(res) + ";\n    }\n";
+    }
+    s += "    }\n";
+    return OPF_OK;
+}
 
 // the straight-line kernel of program P in precision T, writing out (op) value
 // the block's tile (bx, by, bz) from its hardware id: workgroups are dispatched round-robin
@@ -126,6 +390,7 @@ int gen_source(const LoweredProgram& P, int dtype, int op, int R, const SweepArg
     s += "\n";
     s += kWenoSrc;
     s += kMathSrc;
+    s += kGuardSrc;
     {
         char hdr[2048];
         snprintf(hdr, sizeof hdr,
@@ -171,122 +436,18 @@ int gen_source(const LoweredProgram& P, int dtype, int op, int R, const SweepArg
             s += line;
         }
     }
-    std::vector<int> st;  // stack of value ids
-    std::vector<int> res;  // result value of each of the R cells
     const int NV = (int)P.code.size();
-    Known kn((size_t)R * NV);
-    auto pop = [&](int& v) -> bool {
-        if (st.empty()) return false;
-        v = st.back();
-        st.pop_back();
-        return true;
-    };
     // cell r of the thread's R cells (k + r) uses value ids r * NV + (instruction index)
     for (int r = 0; r < R; ++r) {
-        int nv = r * NV;
-        st.clear();
-        for (const Insn& in : P.code) {
-            const int id = nv;
-            switch (in.op) {
-                case I_LD:
-                    if (r == 0) snprintf(line, sizeof line, "  const T v%d = F%d[%d];\n", id, in.a, in.b);
-                    else  // a constant offset, so loads that cells share are one load
-                        snprintf(line, sizeof line, "  const T v%d = F%d[%lldLL];\n", id, in.a,
-                                 in.b + (long long)r * a.f[in.a].e0 * a.f[in.a].e1);
-                    break;
-                case I_CONST: {
-                    if (in.a) {  // launch-time constant: the source does not depend on its value
-                        snprintf(line, sizeof line, "  const T v%d = (T)a.cst[%d];\n", id, in.b);
-                        break;
-                    }
-                    long long bits;
-                    std::memcpy(&bits, &in.imm, 8);
-                    snprintf(line, sizeof line, "  const T v%d = (T)__longlong_as_double(%lldLL);\n", id, bits);
-                    kn.literal(id, in.imm);
-                } break;
-                case I_DX:
-                    if (a.umask >> in.a & 1) {
-                        snprintf(line, sizeof line, "  const T v%d = (T)a.hdx[%d];\n", id, in.a);
-                        kn.dx(id, in.a);
-                    } else {
-                        snprintf(line, sizeof line, "  const T v%d = DX%d[%d];\n", id, in.a, in.b + (in.a == 2 ? r : 0));
-                    }
-                    break;
-                case I_X:
-                    snprintf(line, sizeof line, "  const T v%d = X%d[%d];\n", id, in.a, in.b + (in.a == 2 ? r : 0));
-                    break;
-                case I_ADD:
-                case I_SUB:
-                case I_MUL:
-                case I_DIV: {
-                    int x, y;
-                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
-                    const char o = in.op == I_ADD ? '+' : in.op == I_SUB ? '-' : in.op == I_MUL ? '*' : '/';
-                    const std::string mul = in.op == I_DIV ? kn.div(x, y) : std::string();
-                    if (!mul.empty())
-                        snprintf(line, sizeof line, "  const T v%d = %s;\n", id, mul.c_str());
-                    else
-                        snprintf(line, sizeof line, "  const T v%d = v%d %c v%d;\n", id, x, o, y);
-                    kn.arith(in.op, id, x, y);
-                } break;
-                case I_NEG: {
-                    int x;
-                    if (!pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "  const T v%d = -v%d;\n", id, x);
-                } break;
-                case I_MIN:
-                case I_MAX:
-                case I_GT:
-                case I_LT:
-                case I_GE:
-                case I_LE: {
-                    int x, y;
-                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
-                    if (in.op == I_MIN)  // std::min(a, b) = b < a ? b : a
-                        snprintf(line, sizeof line, "  const T v%d = v%d < v%d ? v%d : v%d;\n", id, y, x, y, x);
-                    else if (in.op == I_MAX)  // std::max(a, b) = a < b ? b : a
-                        snprintf(line, sizeof line, "  const T v%d = v%d < v%d ? v%d : v%d;\n", id, x, y, y, x);
-                    else
-                        snprintf(line, sizeof line, "  const T v%d = v%d %s v%d ? (T)1 : (T)0;\n", id, x,
-                                 in.op == I_GT ? ">" : in.op == I_LT ? "<" : in.op == I_GE ? ">=" : "<=", y);
-                } break;
-                case I_ABS: {
-                    int x;
-                    if (!pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "  const T v%d = (T)fabs((double)v%d);\n", id, x);
-                } break;
-                case I_FN1: {
-                    int x;
-                    if (!pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "  const T v%d = opf_fn1<T>(%d, v%d);\n", id, in.a, x);
-                } break;
-                case I_FN2: {
-                    int x, y;
-                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "  const T v%d = opf_fn2<T>(%d, v%d, v%d);\n", id, in.a, x, y);
-                } break;
-                case I_SEL: {
-                    int c, t_, f_;
-                    if (!pop(f_) || !pop(t_) || !pop(c)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "  const T v%d = v%d != (T)0 ? v%d : v%d;\n", id, c, t_, f_);
-                } break;
-                case I_WENO_UP:
-                case I_WENO_DOWN: {
-                    int h, v[6];
-                    if (!pop(h)) return OPF_ERR_ARG;
-                    for (int q = 5; q >= 0; --q)
-                        if (!pop(v[q])) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "  const T v%d = weno_kernel<T>(v%d, v%d, v%d, v%d, v%d, v%d, v%d, %s);\n",
-                             id, v[0], v[1], v[2], v[3], v[4], v[5], h, in.op == I_WENO_UP ? "true" : "false");
-                } break;
-                default: return OPF_ERR_ARG;
-            }
-            s += line;
-            st.push_back(id);
-            ++nv;
-        }
-        if (st.size() != 1) return OPF_ERR_ARG;
-        res.push_back(st.back());
+        auto ld = [&](const Insn& in) {  // a constant offset, so loads that cells share are one load
+            return "F" + std::to_string(in.a) + "[" +
+                   (r == 0 ? std::to_string(in.b) : std::to_string(in.b + (long long)r * a.f[in.a].e0 * a.f[in.a].e1) + "LL") +
+                   "]";
+        };
+        auto tab = [&](const Insn& in) {
+            return (in.op == I_DX ? "DX" : "X") + std::to_string(in.a) + "[" + std::to_string(in.b + (in.a == 2 ? r : 0)) + "]";
+        };
+        OPF_TRY(emit_cell(P, dtype, a, r * NV, ld, tab, "res" + std::to_string(r), s));
     }
     // every load of the R cells precedes the first store
     s += "  const long long lo = (i - a.oo[0]) + (long long)a.oe0 * ((j - a.oo[1]) + (long long)a.oe1 * (k - a.oo[2]));\n";
@@ -294,14 +455,13 @@ int gen_source(const LoweredProgram& P, int dtype, int op, int R, const SweepArg
     for (int r = 0; r < R; ++r) {
         char at[48];
         snprintf(at, sizeof at, r ? "lo + %d * OP" : "lo", r);
-        const int v = res[r];
         switch (op) {
-            case OPF_OP_EQ: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = v%d;\n", at, v); break;
-            case OPF_OP_ADD: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] + v%d;\n", at, at, v); break;
-            case OPF_OP_MINUS: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] - v%d;\n", at, at, v); break;
-            case OPF_OP_MUL: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] * v%d;\n", at, at, v); break;
+            case OPF_OP_EQ: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = res%d;\n", at, r); break;
+            case OPF_OP_ADD: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] + res%d;\n", at, at, r); break;
+            case OPF_OP_MINUS: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] - res%d;\n", at, at, r); break;
+            case OPF_OP_MUL: snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] * res%d;\n", at, at, r); break;
             case OPF_OP_DIV:
-                snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] / v%d;\n", at, at, v);
+                snprintf(line, sizeof line, "  ((T*)a.out)[%s] = ((const T*)a.old)[%s] / res%d;\n", at, at, r);
                 break;
             default: return OPF_ERR_ARG;
         }
@@ -360,7 +520,7 @@ bool tile_layout(const LoweredProgram& P, bool plane, int RY, TileField (&tf)[SW
     return true;
 }
 
-int gen_source_tile(const LoweredProgram& P, int dtype, int op, int RY, bool plane, int umask,
+int gen_source_tile(const LoweredProgram& P, int dtype, int op, int RY, bool plane, const SweepArgs& a,
                     const TileField (&tf)[SWEEP_MAX_FIELDS], std::string& s) {
     s.clear();
     s += dtype == OPF_F64 ? "typedef double T;\n" : "typedef float T;\n";
@@ -368,6 +528,7 @@ int gen_source_tile(const LoweredProgram& P, int dtype, int op, int RY, bool pla
     s += "\n";
     s += kWenoSrc;
     s += kMathSrc;
+    s += kGuardSrc;
     const int TY = kTileNTY * RY;
     char line[2048];
     snprintf(line, sizeof line,
@@ -502,136 +663,31 @@ int gen_source_tile(const LoweredProgram& P, int dtype, int op, int RY, bool pla
     }
     if (dxu[2]) s += "    const T* __restrict__ DX2 = (const T*)a.dx[2] + (k - a.morg[2]);\n";
     if (xu[2]) s += "    const T* __restrict__ X2 = (const T*)a.x[2] + (k - a.morg[2]);\n";
-    std::vector<int> st;
-    std::vector<int> res;
     const int NV = (int)P.code.size();
-    Known kn((size_t)RY * NV);
-    auto pop = [&](int& v) -> bool {
-        if (st.empty()) return false;
-        v = st.back();
-        st.pop_back();
-        return true;
-    };
     for (int r = 0; r < RY; ++r) {
-        int nv = r * NV;
-        st.clear();
-        for (const Insn& in : P.code) {
-            const int id = nv;
-            switch (in.op) {
-                case I_LD: {
-                    const TileField& F = tf[in.a];
-                    const int dx = (in.c & 255) - 64, dy = ((in.c >> 8) & 255) - 64, dz = ((in.c >> 16) & 255) - 64;
-                    snprintf(line, sizeof line, "    const T v%d = B%d_%d[%d];\n", id, in.a, dz + 64,
-                             (r + dy) * F.W + dx);
-                } break;
-                case I_CONST: {
-                    if (in.a) {
-                        snprintf(line, sizeof line, "    const T v%d = (T)a.cst[%d];\n", id, in.b);
-                        break;
-                    }
-                    long long bits;
-                    std::memcpy(&bits, &in.imm, 8);
-                    snprintf(line, sizeof line, "    const T v%d = (T)__longlong_as_double(%lldLL);\n", id, bits);
-                    kn.literal(id, in.imm);
-                } break;
-                case I_DX:
-                case I_X: {
-                    if (in.op == I_DX && (umask >> in.a & 1)) {
-                        snprintf(line, sizeof line, "    const T v%d = (T)a.hdx[%d];\n", id, in.a);
-                        kn.dx(id, in.a);
-                        break;
-                    }
-                    const char* tb = in.op == I_DX ? "DX" : "X";
-                    if (in.a == 1) snprintf(line, sizeof line, "    const T v%d = %s1_%d[%d];\n", id, tb, r, in.b);
-                    else snprintf(line, sizeof line, "    const T v%d = %s%d[%d];\n", id, tb, in.a, in.b);
-                } break;
-                case I_ADD:
-                case I_SUB:
-                case I_MUL:
-                case I_DIV: {
-                    int x, y;
-                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
-                    const char o = in.op == I_ADD ? '+' : in.op == I_SUB ? '-' : in.op == I_MUL ? '*' : '/';
-                    const std::string mul = in.op == I_DIV ? kn.div(x, y) : std::string();
-                    if (!mul.empty())
-                        snprintf(line, sizeof line, "    const T v%d = %s;\n", id, mul.c_str());
-                    else
-                        snprintf(line, sizeof line, "    const T v%d = v%d %c v%d;\n", id, x, o, y);
-                    kn.arith(in.op, id, x, y);
-                } break;
-                case I_NEG: {
-                    int x;
-                    if (!pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "    const T v%d = -v%d;\n", id, x);
-                } break;
-                case I_MIN:
-                case I_MAX:
-                case I_GT:
-                case I_LT:
-                case I_GE:
-                case I_LE: {
-                    int x, y;
-                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
-                    if (in.op == I_MIN)  // std::min(a, b) = b < a ? b : a
-                        snprintf(line, sizeof line, "      const T v%d = v%d < v%d ? v%d : v%d;\n", id, y, x, y, x);
-                    else if (in.op == I_MAX)  // std::max(a, b) = a < b ? b : a
-                        snprintf(line, sizeof line, "      const T v%d = v%d < v%d ? v%d : v%d;\n", id, x, y, y, x);
-                    else
-                        snprintf(line, sizeof line, "      const T v%d = v%d %s v%d ? (T)1 : (T)0;\n", id, x,
-                                 in.op == I_GT ? ">" : in.op == I_LT ? "<" : in.op == I_GE ? ">=" : "<=", y);
-                } break;
-                case I_ABS: {
-                    int x;
-                    if (!pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "      const T v%d = (T)fabs((double)v%d);\n", id, x);
-                } break;
-                case I_FN1: {
-                    int x;
-                    if (!pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "      const T v%d = opf_fn1<T>(%d, v%d);\n", id, in.a, x);
-                } break;
-                case I_FN2: {
-                    int x, y;
-                    if (!pop(y) || !pop(x)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "      const T v%d = opf_fn2<T>(%d, v%d, v%d);\n", id, in.a, x, y);
-                } break;
-                case I_SEL: {
-                    int c, t_, f_;
-                    if (!pop(f_) || !pop(t_) || !pop(c)) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line, "      const T v%d = v%d != (T)0 ? v%d : v%d;\n", id, c, t_, f_);
-                } break;
-                case I_WENO_UP:
-                case I_WENO_DOWN: {
-                    int h, v[6];
-                    if (!pop(h)) return OPF_ERR_ARG;
-                    for (int q = 5; q >= 0; --q)
-                        if (!pop(v[q])) return OPF_ERR_ARG;
-                    snprintf(line, sizeof line,
-                             "    const T v%d = weno_kernel<T>(v%d, v%d, v%d, v%d, v%d, v%d, v%d, %s);\n", id, v[0],
-                             v[1], v[2], v[3], v[4], v[5], h, in.op == I_WENO_UP ? "true" : "false");
-                } break;
-                default: return OPF_ERR_ARG;
-            }
-            s += line;
-            st.push_back(id);
-            ++nv;
-        }
-        if (st.size() != 1) return OPF_ERR_ARG;
-        res.push_back(st.back());
+        auto ld = [&](const Insn& in) {
+            const int dx = (in.c & 255) - 64, dy = ((in.c >> 8) & 255) - 64, dz = ((in.c >> 16) & 255) - 64;
+            return "B" + std::to_string(in.a) + "_" + std::to_string(dz + 64) + "[" +
+                   std::to_string((r + dy) * tf[in.a].W + dx) + "]";
+        };
+        auto tab = [&](const Insn& in) {
+            return (in.op == I_DX ? "DX" : "X") + std::to_string(in.a) + (in.a == 1 ? "_" + std::to_string(r) : "") + "[" +
+                   std::to_string(in.b) + "]";
+        };
+        OPF_TRY(emit_cell(P, dtype, a, r * NV, ld, tab, "res" + std::to_string(r), s));
     }
     s += "    if (i < xe) {\n";
     s += "      const long long lo = (i - a.oo[0]) + (long long)a.oe0 * ((jb - a.oo[1]) + (long long)a.oe1 * (k - a.oo[2]));\n";
     for (int r = 0; r < RY; ++r) {
         char at[48];
         snprintf(at, sizeof at, "lo + %d * a.oe0", r);
-        const int v = res[r];
         char val[160];
         switch (op) {
-            case OPF_OP_EQ: snprintf(val, sizeof val, "v%d", v); break;
-            case OPF_OP_ADD: snprintf(val, sizeof val, "((const T*)a.old)[%s] + v%d", at, v); break;
-            case OPF_OP_MINUS: snprintf(val, sizeof val, "((const T*)a.old)[%s] - v%d", at, v); break;
-            case OPF_OP_MUL: snprintf(val, sizeof val, "((const T*)a.old)[%s] * v%d", at, v); break;
-            case OPF_OP_DIV: snprintf(val, sizeof val, "((const T*)a.old)[%s] / v%d", at, v); break;
+            case OPF_OP_EQ: snprintf(val, sizeof val, "res%d", r); break;
+            case OPF_OP_ADD: snprintf(val, sizeof val, "((const T*)a.old)[%s] + res%d", at, r); break;
+            case OPF_OP_MINUS: snprintf(val, sizeof val, "((const T*)a.old)[%s] - res%d", at, r); break;
+            case OPF_OP_MUL: snprintf(val, sizeof val, "((const T*)a.old)[%s] * res%d", at, r); break;
+            case OPF_OP_DIV: snprintf(val, sizeof val, "((const T*)a.old)[%s] / res%d", at, r); break;
             default: return OPF_ERR_ARG;
         }
         snprintf(line, sizeof line, "      if (jb + %d < ye) ((T*)a.out)[%s] = %s;\n", r, at, val);
@@ -831,7 +887,7 @@ uint64_t plan_key(const LoweredProgram& P, int dtype, const SweepArgs& a, int de
         h = fnv1a64(w, sizeof w, h);
         if (!(in.op == I_CONST && in.a)) h = fnv1a64(&in.imm, sizeof in.imm, h);
     }
-    const int q[6] = {dtype, a.op, a.umask, a.n[2] == 1, a.n[2] % 4, dev * 4 + form};
+    const int q[8] = {dtype, a.op, a.umask, a.cmask, a.xmask, a.n[2] == 1, a.n[2] % 4, dev * 4 + form};
     h = fnv1a64(q, sizeof q, h);
     for (const FieldArg& f : a.f) {  // the direct form bakes plane strides into its loads
         const long long ps = (long long)f.e0 * f.e1;
@@ -899,7 +955,7 @@ int jit_launch_sweep(hipStream_t st, const LoweredProgram& P, int dtype, const S
         for (auto& f : tf) nq += f.used ? f.NQ : 0;
         if (lds > (size_t)64 * 1024 || nq > 24 || P.code.size() * RY > (size_t)SWEEP_JIT_MAX_INSNS) continue;
         std::string src;
-        OPF_CHECK(gen_source_tile(P, dtype, a.op, RY, plane, a.umask, tf, src) == OPF_OK, OPF_ERR_ARG,
+        OPF_CHECK(gen_source_tile(P, dtype, a.op, RY, plane, a, tf, src) == OPF_OK, OPF_ERR_ARG,
                   "jit: malformed sweep program");
         uint64_t mk = 0;
         OPF_TRY(function_for_source(src, &fn, &mk));

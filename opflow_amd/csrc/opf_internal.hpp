@@ -89,6 +89,8 @@ struct opf_mesh {
     float* x_f32[3] = {nullptr, nullptr, nullptr};
     bool uniform[3] = {false, false, false};
     double h[3] = {0, 0, 0};
+    // largest |x| / h of a uniform dim whose coordinates are whole multiples of a power-of-two h, else -1
+    double span[3] = {-1, -1, -1};
     double x(int d, int i) const { return hx[d][i - (start[d] - pad)]; }
     double dx(int d, int i) const { return hdx[d][i - (start[d] - pad)]; }
     bool has_node(int d, int i) const {

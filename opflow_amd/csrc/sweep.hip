@@ -745,18 +745,27 @@ std::vector<Insn> structural_code(const LoweredProgram& P) {
 }
 
 void uniform_spacing(const opf_mesh* m, int dtype, SweepArgs& a) {
-    a.umask = 0;
+    a.umask = a.cmask = a.xmask = 0;
     for (int d = 0; d < m->dim; ++d) {
         a.hdx[d] = a.rdx[d] = 0.0;
         int e;
         const double h = m->h[d];
+        if (!m->uniform[d] || !(h > 0)) continue;
+        if (std::frexp(h, &e) != 0.5) {
+            if (dtype != OPF_F64 || !(h >= 0x1p-100 && h <= 0x1p100)) continue;
+            a.cmask |= 1 << d;
+            a.hdx[d] = h;
+            a.rdx[d] = 1.0 / h;
+            continue;
+        }
         // a power of two whose reciprocal is a normal number of the sweep's precision
-        if (!m->uniform[d] || !(h > 0) || std::frexp(h, &e) != 0.5) continue;
         const int lim = dtype == OPF_F64 ? 1016 : 120;  // room for multiples 1/4 .. 4 of h
         if (e - 1 > lim || e - 1 < -lim) continue;
         a.umask |= 1 << d;
         a.hdx[d] = h;
         a.rdx[d] = 1.0 / h;
+        // (x_i + s h) for |s| <= 64 and quarters of h are exact below 2^53 (2^24) of them
+        if (m->span[d] >= 0 && m->span[d] < (dtype == OPF_F64 ? 0x1p40 : 0x1p18)) a.xmask |= 1 << d;
     }
 }
 

@@ -95,9 +95,10 @@ void jit_stats(long long* compiles, long long* loaded, long long* resident);
 int check_bounds(const LoweredProgram& P, opf_field* const* fields, int nfields, const opf_mesh* mesh, const int s[3],
                  const int n[3]);
 int mesh_arrays(const opf_mesh* m, int dtype, const void* x[3], const void* dx[3]);
-// dims of m whose spacing is uniform and a power of two with a normal reciprocal in
-// precision dtype: a.umask, a.hdx, a.rdx (compiled sweeps divide by h as a
-// multiplication by 1 / h, which gives the same bits)
+// dims of m whose spacing is uniform: a power of two with a normal reciprocal in precision
+// dtype (a.umask; compiled sweeps divide by h as a multiplication by 1 / h, which gives the
+// same bits), with all coordinates whole multiples of it (a.xmask), or any h in FP64
+// (a.cmask); a.hdx, a.rdx
 void uniform_spacing(const opf_mesh* m, int dtype, SweepArgs& a);
 
 }  // namespace opf
