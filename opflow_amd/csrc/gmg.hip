@@ -1122,6 +1122,163 @@ __global__ __launch_bounds__(NT) void k2_up(GOp<T> o, const T* __restrict__ x2, 
     }
 }
 
+// ---- the same two launches for variable coefficients. The coefficients of a cell are read once a
+// launch and kept in LDS with its D and w / D (one division a cell instead of one a sweep; a missing
+// neighbour has the coefficient 0, so the sweeps have no boundary cases). The levels of a handled
+// equation are small and bound by launches and their latency: two launches a level replace five.
+// 640 x 400 cells, four such levels (the first 8.3 and 6.3 us, the others 4.6 and 4.5, against five
+// launches of 3 to 5 each): a cycle of them 78 -> 42 us, the solve 2.49 -> 2.14 ms.
+// Tiles of 16 x 16 from 2^16 cells on, 8 x 8 below, as above (32 x 32 would not fit the LDS).
+template <typename T, int TS>
+struct VarTile {
+    static constexpr int W2 = TS + 4, W1 = TS + 2;
+    T b[W2 * W2], wd[W2 * W2], s1[W2 * W2];     // right-hand side, w / D, x1 (x3) on the tile + 2
+    T c[4][W1 * W1], dd[W1 * W1], s2[W1 * W1];  // neighbour coefficients, D, x2 (x4) on the tile + 1
+    // position p of the tile + 2: its cell (false: outside a non-periodic dim)
+    __device__ __forceinline__ static bool cell(const GOp<T>& o, int x0, int y0, int p, int& i, int& j) {
+        return f2_map(x0 - 2 + p % W2, o.n0, o.per[0], i) && f2_map(y0 - 2 + p / W2, o.n1, o.per[1], j);
+    }
+    // b, w / D and, on the tile + 1, the coefficients and D of position p (all 0 outside)
+    __device__ __forceinline__ void stage(const GOp<T>& o, const T* __restrict__ bv, T w, bool ok, int i, int j, int p) {
+        T k[4] = {0, 0, 0, 0}, D = 0, r = 0, wi = 0;
+        if (ok) {
+            const uint32_t t = (uint32_t)i + o.s1 * (uint32_t)j;
+            const int at[2] = {i, j}, n[2] = {o.n0, o.n1};
+            D = o.sg[t];
+            r = bv[t];
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const T a = o.af[d][face_index(d, i + (d == 0 && s), j + (d == 1 && s), 0, o.n0, o.n1)];
+                    const bool in = o.per[d] || (s ? at[d] < n[d] - 1 : at[d] > 0);
+                    D += in ? a : a * o.bfac[d][s];
+                    k[2 * d + s] = in ? a : (T)0;
+                }
+            wi = w / D;
+        }
+        b[p] = r;
+        wd[p] = wi;
+        const int li = p % W2 - 1, lj = p / W2 - 1;
+        if (li >= 0 && li < W1 && lj >= 0 && lj < W1) {
+            const int q = li + W1 * lj;
+            for (int e = 0; e < 4; ++e) c[e][q] = k[e];
+            dd[q] = D;
+        }
+    }
+    // (A v)_c at position q of the tile + 1; v at c with row stride W
+    __device__ __forceinline__ T apply(const T* v, int c0, int W, int q) const {
+        T acc = c[0][q] * v[c0 - 1];
+        acc += c[1][q] * v[c0 + 1];
+        acc += c[2][q] * v[c0 - W];
+        acc += c[3][q] * v[c0 + W];
+        return dd[q] * v[c0] - acc;
+    }
+    // s2 = s1 + w (b - A s1) / D on the tile + 1
+    __device__ __forceinline__ void sweep() {
+        for (int q = threadIdx.x; q < W1 * W1; q += blockDim.x) {
+            const int p = (q / W1 + 1) * W2 + q % W1 + 1;
+            s2[q] = s1[p] + wd[p] * (b[p] - apply(s1, p, W2, q));
+        }
+        __syncthreads();
+    }
+};
+
+template <typename T, int TS, int NT>
+__global__ __launch_bounds__(NT) void k2v_down(GOp<T> o, const T* __restrict__ b, T* __restrict__ x2o,
+                                               T* __restrict__ bc, int c0, int c1, T w, F2Tile ft, Bat bt) {
+    using V = VarTile<T, TS>;
+    static_assert((TS / 2) * (TS / 2) <= NT, "one coarse cell of the tile per thread");
+    __shared__ V v;
+    BAT_SLOT(bt);
+    b += vo;
+    x2o += vo;
+    bc += (long long)slot * ((long long)c0 * c1);
+    for (int tile = (int)xcd_block(blockIdx.x, gridDim.x); tile < ft.tiles; tile += gridDim.x) {
+        const int x0 = (tile % ft.tx) * TS, y0 = (tile / ft.tx) * TS;
+        for (int p = threadIdx.x; p < V::W2 * V::W2; p += blockDim.x) {
+            int i = 0, j = 0;
+            const bool ok = V::cell(o, x0, y0, p, i, j);
+            v.stage(o, b, w, ok, i, j, p);
+            v.s1[p] = v.wd[p] * v.b[p];
+        }
+        __syncthreads();
+        v.sweep();
+        if (threadIdx.x < (TS / 2) * (TS / 2)) {
+            const int ci = threadIdx.x % (TS / 2), cj = threadIdx.x / (TS / 2);
+            T s = 0;
+#pragma unroll
+            for (int dj = 0; dj < 2; ++dj)
+#pragma unroll
+                for (int di = 0; di < 2; ++di) {
+                    const int li = 2 * ci + di, lj = 2 * cj + dj, i = x0 + li, j = y0 + lj;
+                    if (i >= o.n0 || j >= o.n1) continue;
+                    const int q = (lj + 1) * V::W1 + li + 1;
+                    s += v.b[(lj + 2) * V::W2 + li + 2] - v.apply(v.s2, q, V::W1, q);
+                    x2o[(uint32_t)i + o.s1 * (uint32_t)j] = v.s2[q];
+                }
+            const int I = x0 / 2 + ci, J = y0 / 2 + cj;
+            if (I < c0 && J < c1) bc[(uint32_t)I + (uint32_t)c0 * (uint32_t)J] = s * (T)0.25;
+        }
+        __syncthreads();  // the LDS tile is reused
+    }
+}
+
+template <typename T, int TS, int NT, bool DOTS>
+__global__ __launch_bounds__(NT) void k2v_up(GOp<T> o, const T* __restrict__ x2, const T* __restrict__ xc, int c0,
+                                             int c1, const T* __restrict__ b, T* __restrict__ out, T w,
+                                             const T* __restrict__ q, double* __restrict__ part, F2Tile ft, Bat bt) {
+    using V = VarTile<T, TS>;
+    __shared__ V v;
+    BAT_SLOT(bt);
+    x2 += vo;
+    b += vo;
+    out += vo;
+    xc += (long long)slot * ((long long)c0 * c1);
+    if (DOTS) {
+        q += vo;
+        part += (long long)slot * bt.ps;
+    }
+    const int cn[3] = {c0, c1, 1};
+    double d0 = 0, d1 = 0, d2 = 0;
+    for (int tile = (int)xcd_block(blockIdx.x, gridDim.x); tile < ft.tiles; tile += gridDim.x) {
+        const int x0 = (tile % ft.tx) * TS, y0 = (tile / ft.tx) * TS;
+        for (int p = threadIdx.x; p < V::W2 * V::W2; p += blockDim.x) {
+            int i = 0, j = 0;
+            const bool ok = V::cell(o, x0, y0, p, i, j);
+            v.s1[p] = ok ? x2[(uint32_t)i + o.s1 * (uint32_t)j] + prolong_at<T, 2>(o, xc, cn, i, j, 0) : (T)0;
+            v.stage(o, b, w, ok, i, j, p);
+        }
+        __syncthreads();
+        v.sweep();
+        for (int p = threadIdx.x; p < TS * TS; p += blockDim.x) {
+            const int li = p % TS, lj = p / TS, i = x0 + li, j = y0 + lj;
+            if (i >= o.n0 || j >= o.n1) continue;
+            const int c = (lj + 1) * V::W1 + li + 1, p2 = (lj + 2) * V::W2 + li + 2;
+            const T x5 = v.s2[c] + v.wd[p2] * (v.b[p2] - v.apply(v.s2, c, V::W1, c));
+            const uint32_t t = (uint32_t)i + o.s1 * (uint32_t)j;
+            out[t] = x5;
+            if (DOTS) {
+                const double zv = (double)x5;
+                d0 += (double)v.b[p2] * zv;
+                d1 += zv * (double)q[t];
+                d2 += zv;
+            }
+        }
+        __syncthreads();
+    }
+    if (DOTS) {
+        d0 = gmg_block_sum(d0);
+        d1 = gmg_block_sum(d1);
+        d2 = gmg_block_sum(d2);
+        if (threadIdx.x == 0) {
+            part[blockIdx.x] = d0;
+            part[GMG_MAXB + blockIdx.x] = d1;
+            part[2 * GMG_MAXB + blockIdx.x] = d2;
+        }
+    }
+}
+
 // ---- coarse tail: every level of at most GMG_TAIL_N cells in one workgroup per slot.
 // A V-cycle's coarse levels are tiny and launch-bound (a handful of cells per
 // CU); here one 1024-thread workgroup runs their smoothing sweeps, residual
@@ -2006,17 +2163,19 @@ static void ph_vtail(const Hierarchy& H, hipStream_t st, const int* mask, int l0
                                                   st, ta, bt));
 }
 
-// 2-D constant-coefficient V(2,2) levels run as k2_down / k2_up: one block per tile
-// (at most GMG_MAXB, then striding); on the finest level k2_up writes the partials
-// of the three dot products, one per block
-static bool fused2d(const Hierarchy& H) { return H.dim == 2 && !H.var && H.pre == 2 && H.post == 2; }
+// 2-D V(2,2) levels run as k2_down / k2_up (variable coefficients: k2v_*): one block per
+// tile (at most GMG_MAXB, then striding); on the finest level the up half writes the
+// partials of the three dot products, one per block
+static bool fused2d(const Hierarchy& H) { return H.dim == 2 && H.pre == 2 && H.post == 2; }
 // tile side of a level's k2 kernels (threads: 256 for 32 and 16, 64 for 8); measured on
 // the 2048^2 hierarchy: 16 x 16 tiles took the 1024^2 level's pair 26.2 -> 25.1 us and
 // 8 x 8 the 128^2 and 64^2 levels' 8-10 -> 5.5 us each, while a 32^2 level stays in the
 // coarse tail (its 8 x 8 pair costs 11 us, the tail 5 us more than without it)
-static int f2_ts(const GLevelHost& L) { return L.N >= (1LL << 21) ? 32 : L.N >= (1LL << 16) ? 16 : 8; }
-static F2Tile f2tile(const GLevelHost& L) {
-    const int ts = f2_ts(L);
+static int f2_ts(const GLevelHost& L, bool var) {
+    return L.N >= (1LL << 21) && !var ? 32 : L.N >= (1LL << 16) ? 16 : 8;
+}
+static F2Tile f2tile(const GLevelHost& L, bool var) {
+    const int ts = f2_ts(L, var);
     F2Tile ft;
     ft.tx = (L.n[0] + ts - 1) / ts;
     ft.ty = (L.n[1] + ts - 1) / ts;
@@ -2026,7 +2185,7 @@ static F2Tile f2tile(const GLevelHost& L) {
 // partial sums per value that the finest level's V-cycle leaves for the DOT3 finish
 template <typename T>
 static int dot3_parts(const Hierarchy& H) {
-    if (fused2d(H) && H.dev.size() > 1) return std::min(f2tile(H.host[0]).tiles, GMG_MAXB);
+    if (fused2d(H) && H.dev.size() > 1) return std::min(f2tile(H.host[0], H.var).tiles, GMG_MAXB);
     return red_count<T>(H);
 }
 
@@ -2054,10 +2213,10 @@ void ph_vcycle(const Hierarchy& H, hipStream_t st, const int* mask, int l, const
     if (fused2d(H)) {
         // the level in two launches (k2_down / k2_up): x2 kept in the level temp
         const GLevelDev& C = H.dev[l + 1];
-        const F2Tile ft = f2tile(L);
+        const F2Tile ft = f2tile(L, H.var);
         const unsigned G = (unsigned)std::min(ft.tiles, GMG_MAXB);
         const Bat bt = bat(H, mask, N);
-        const int ts = f2_ts(L);
+        const int ts = f2_ts(L, H.var);
         auto by_ts = [&](auto launch) {
             if (ts == 32) launch(std::integral_constant<int, 32>{}, std::integral_constant<int, 256>{});
             else if (ts == 16) launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 256>{});
@@ -2065,19 +2224,30 @@ void ph_vcycle(const Hierarchy& H, hipStream_t st, const int* mask, int l, const
         };
         by_ts([&](auto TS_, auto NT_) {
             constexpr int TS = decltype(TS_)::value, NT = decltype(NT_)::value;
+            if constexpr (TS <= 16)
+                if (H.var) {
+                    hipLaunchKernelGGL((k2v_down<T, TS, NT>), dim3(G, B), dim3(NT), 0, st, o, rhs, (T*)D.t, (T*)C.b,
+                                       C.n[0], C.n[1], w, ft, bt);
+                    return;
+                }
             hipLaunchKernelGGL((k2_down<T, TS, NT>), dim3(G, B), dim3(NT), 0, st, o, rhs, (T*)D.t, (T*)C.b, C.n[0],
                                C.n[1], w, ft, bt);
         });
         ph_vcycle<T>(H, st, mask, l + 1, (const T*)C.b, (T*)C.x);
         by_ts([&](auto TS_, auto NT_) {
             constexpr int TS = decltype(TS_)::value, NT = decltype(NT_)::value;
-            if (dot_q)  // one partial per block (dot3_parts)
-                hipLaunchKernelGGL((k2_up<T, TS, NT, true>), dim3(G, B), dim3(NT), 0, st, o, (const T*)D.t,
-                                   (const T*)C.x, C.n[0], C.n[1], rhs, out, w, dot_q, H.part, ft, bt);
-            else
-                hipLaunchKernelGGL((k2_up<T, TS, NT, false>), dim3(G, B), dim3(NT), 0, st, o, (const T*)D.t,
-                                   (const T*)C.x, C.n[0], C.n[1], rhs, out, w, (const T*)nullptr, (double*)nullptr,
-                                   ft, bt);
+            auto up = [&](auto kernel, const T* q, double* part) {
+                hipLaunchKernelGGL(kernel, dim3(G, B), dim3(NT), 0, st, o, (const T*)D.t, (const T*)C.x, C.n[0], C.n[1],
+                                   rhs, out, w, q, part, ft, bt);
+            };
+            if constexpr (TS <= 16)
+                if (H.var) {
+                    if (dot_q) up(k2v_up<T, TS, NT, true>, dot_q, H.part);
+                    else up(k2v_up<T, TS, NT, false>, (const T*)nullptr, (double*)nullptr);
+                    return;
+                }
+            if (dot_q) up(k2_up<T, TS, NT, true>, dot_q, H.part);  // one partial per block (dot3_parts)
+            else up(k2_up<T, TS, NT, false>, (const T*)nullptr, (double*)nullptr);
         });
         return;
     }
