@@ -1,19 +1,19 @@
 // Dense FP64 inverse of a multigrid hierarchy's coarsest level (at most 1024 cells),
 // assembled and inverted on the device.
 //
-// The inverse is a blocked in-place Gauss-Jordan elimination with 32 x 32 pivot blocks.
-// Per block two launches: k_gj_panel inverts the pivot block (every workgroup for itself:
-// 32 rank-1 steps in registers, the pivot row and column exchanged through LDS, one barrier
-// a step) and forms one 32-column tile of the scaled pivot rows; k_gj_update applies the
-// rank-32 update to the other rows in 64 x 64 tiles held 4 x 4 per thread. The chain of n
-// pivots bounds it, not the 2 n^3 operations: at n = 1000, 32 x (12.5 us panel + 10.1 us
-// update) = 0.72 ms. The diagonal
-// pivots of a symmetric matrix are all positive exactly when it is positive definite, which
-// every level of a Laplacian with a non-negative shift is; a pivot that is not positive
-// sets a flag, and the level is then inverted on the host with row exchanges, as an
+// The inverse is a blocked Gauss-Jordan elimination with 32 x 32 pivot blocks, one launch a
+// block. Every workgroup of k_gj_step owns a 64 x 64 tile: it scales its part of the pivot rows
+// by the inverted pivot block and subtracts (its part of the pivot columns) x (those rows), both on
+// the matrix cores (FP64 16 x 16 x 4), reading one buffer and writing the other, so that no
+// workgroup waits for another; the one that holds the next pivot block then inverts it (32 rank-1
+// steps of one wave, without a barrier). That chain bounds it, not the 2 n^3 operations: n = 1000,
+// 32 launches of 11.3 us, two thirds of it memory; with a panel launch in which every workgroup inverted the pivot block and
+// an update launch on the vector pipes, 12.9 + 10.4 us and a gap more.
+// The diagonal pivots of a symmetric matrix are all positive exactly when it is positive
+// definite, which every level of a Laplacian with a non-negative shift is; a pivot that is not
+// positive sets a flag, and the level is then inverted on the host with row exchanges, as an
 // indefinite operator needs. On a 640 x 400 variable-coefficient equation (coarsest level
-// 40 x 25, rebuilt at every solve) the host elimination took 240 ms of a 252 ms solve; the
-// solve now takes 2.6 ms.
+// 40 x 25, rebuilt at every solve) the host elimination took 240 ms of a 252 ms solve.
 #include <algorithm>
 #include <cmath>
 
@@ -23,7 +23,7 @@ namespace opf {
 namespace {
 
 constexpr int kPB = 32;  // pivot block
-constexpr int kTU = 64;  // update tile
+constexpr int kTU = 64;  // tile of a workgroup
 
 // the coarsest level's operator as the assembly reads it
 struct CoarseOp {
@@ -94,119 +94,209 @@ __device__ __forceinline__ double quick_rcp(double v) {
     return __builtin_fma(__builtin_fma(-v, y, 1.0), y, y);
 }
 
-// pivot block k0: R (kPB x n) = the scaled pivot rows, the inverted pivot block in the
-// pivot's own columns; C (n x kPB) = the pivot columns as they were. One barrier a pivot:
-// the row and column buffers alternate, and a buffer is written again only after the next
-// pivot's barrier.
-__global__ __launch_bounds__(256) void k_gj_panel(const double* __restrict__ A, int n, int k0, double* __restrict__ R,
-                                                  double* __restrict__ C, int* __restrict__ flag) {
-    __shared__ double prow[2][kPB], pcol[2][kPB], P[kPB][kPB + 2], T[kPB][kPB + 2];
-    const int bs = min(kPB, n - k0), j0 = blockIdx.x * kPB;
-    const int t = threadIdx.x, r = t >> 3, g = t & 7, c0 = g * 4;  // this thread: row r, columns c0 .. c0 + 3
+// In-place inverse of the symmetric kPB x kPB matrix M by one workgroup of 256: thread t has columns
+// 4 (t / 32) .. of row t % 32. Four pivots a round: their columns are exchanged through LDS (their
+// rows are the columns, negated for the pivots already taken, as elimination in place leaves a
+// symmetric matrix), every thread inverts their 4 x 4 block by halves and subtracts a rank-4 update.
+// The round's chain of latencies bounds it: with one pivot a round 12 us a block, with four by one
+// wave 6, now 3.5. One barrier a round: the buffers alternate. xch: kXch values. False when a leading
+// minor of a pivot block is not positive.
+constexpr int kXch = 16 * kPB;
+__device__ __forceinline__ bool invert_block(double (*M)[kPB + 2], double* xch) {
+    const int r = threadIdx.x & 31, g = threadIdx.x >> 5;
     double a[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int c = c0 + q;
-        a[q] = r < bs && c < bs ? A[(size_t)(k0 + r) * n + k0 + c] : (r == c ? 1.0 : 0.0);
-        T[r][c] = r < bs && j0 + c < n ? A[(size_t)(k0 + r) * n + j0 + c] : 0.0;
-        if (j0 + r < n) C[(size_t)(j0 + r) * kPB + c] = c < bs ? A[(size_t)(j0 + r) * n + k0 + c] : 0.0;
-    }
-    bool bad = false;
-    for (int m = 0; m < kPB / 4; ++m)
+    for (int w = 0; w < 4; ++w) a[w] = M[r][4 * g + w];
+    bool ok = true;
+#pragma unroll 1
+    for (int m = 0; m < kPB / 4; ++m) {
+        const int p = 4 * m;
+        const bool own = r >= p && r < p + 4;
+        double *col = xch + (m & 1) * 8 * kPB, *rows = col + 4 * kPB;  // col[4 r + k], rows[kPB k + c]
+        if (g == m) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {  // pivot p, held in register q of the threads with g = m
-            const int p = 4 * m + q;
-            double* pr = prow[q & 1];
-            double* pc = pcol[q & 1];
-            if (r == p) {
-#pragma unroll
-                for (int w = 0; w < 4; ++w) pr[c0 + w] = a[w];
+            for (int k = 0; k < 4; ++k) {
+                col[4 * r + k] = a[k];
+                rows[kPB * k + r] = r < p ? -a[k] : a[k];
             }
-            if (g == m) pc[r] = a[q];
-            __syncthreads();
-            const double piv = pr[p], inv = quick_rcp(piv);
-            bad |= !(piv > 0.0) || !isfinite(inv);
-            const bool own = r == p;
-            const double f = own ? -inv : pc[r] * inv;  // the pivot's row is scaled: a' = a / piv
-#pragma unroll
-            for (int w = 0; w < 4; ++w) a[w] = __builtin_fma(-f, pr[c0 + w], own ? 0.0 : a[w]);
-            if (g == m) a[q] = own ? inv : -f;
         }
-    if (bad && t == 0 && blockIdx.x == 0) *flag = 1;
-    if (j0 == k0) {
+        __syncthreads();
+        // V = the inverse of [[P, Q], [Q^T, S]] (2 x 2 blocks, P and S symmetric)
+        const double* b = col + 4 * p;
+        const double p0 = b[0], p1 = b[4], p2 = b[5], q0 = b[8], q1 = b[12], q2 = b[9], q3 = b[13];
+        const double dp = p0 * p2 - p1 * p1, ip = quick_rcp(dp);
+        const double i0 = p2 * ip, i1 = -p1 * ip, i2 = p0 * ip;                     // P^-1
+        const double u0 = i0 * q0 + i1 * q2, u1 = i0 * q1 + i1 * q3;                // U = P^-1 Q
+        const double u2 = i1 * q0 + i2 * q2, u3 = i1 * q1 + i2 * q3;
+        const double s0 = b[10] - (q0 * u0 + q2 * u2), s1 = b[14] - (q1 * u0 + q3 * u2);
+        const double s2 = b[15] - (q1 * u1 + q3 * u3);                              // S - Q^T U
+        const double ds = s0 * s2 - s1 * s1, is = quick_rcp(ds);
+        const double j0 = s2 * is, j1 = -s1 * is, j2 = s0 * is;
+        ok &= p0 > 0.0 && dp > 0.0 && s0 > 0.0 && ds > 0.0 && isfinite(ip) && isfinite(is);
+        const double v0 = -(u0 * j0 + u1 * j1), v1 = -(u0 * j1 + u1 * j2);          // -U (..)^-1
+        const double v2 = -(u2 * j0 + u3 * j1), v3 = -(u2 * j1 + u3 * j2);
+        const double w0 = i0 - (v0 * u0 + v1 * u1), w1 = i1 - (v0 * u2 + v1 * u3), w2 = i2 - (v2 * u2 + v3 * u3);
+        // a row of the block becomes V times the pivot rows: its factors are those of -1 in its place
+        double c[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (j0 + c0 + q < n) R[(size_t)r * n + j0 + c0 + q] = a[q];
-        return;
+        for (int k = 0; k < 4; ++k) c[k] = own ? (r == p + k ? -1.0 : 0.0) : col[4 * r + k];
+        const double f[4] = {c[0] * w0 + c[1] * w1 + c[2] * v0 + c[3] * v1, c[0] * w1 + c[1] * w2 + c[2] * v2 + c[3] * v3,
+                             c[0] * v0 + c[1] * v2 + c[2] * j0 + c[3] * j1, c[0] * v1 + c[1] * v3 + c[2] * j1 + c[3] * j2};
+        const double keep = own ? 0.0 : 1.0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            double n = keep * a[w];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) n = __builtin_fma(-f[k], rows[kPB * k + 4 * g + w], n);
+            a[w] = g == m ? -f[w] : n;
+        }
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) P[r][c0 + q] = a[q];
     __syncthreads();
-    double s[4] = {0, 0, 0, 0};
-#pragma unroll 8
-    for (int m = 0; m < kPB; ++m) {
-        const double pm = P[r][m];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] = __builtin_fma(pm, T[m][c0 + q], s[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        if (j0 + c0 + q < n) R[(size_t)r * n + j0 + c0 + q] = s[q];
+    for (int w = 0; w < 4; ++w) M[r][4 * g + w] = a[w];
+    __syncthreads();
+    return ok;
 }
 
-// rows of the pivot block become R; every other row loses (its pivot columns) x R, with
-// its pivot columns taken as zero first. The tile's own entries are loaded first, so that
-// they arrive while the panels are staged.
-__global__ __launch_bounds__(256) void k_gj_update(double* __restrict__ A, int n, int k0, const double* __restrict__ R,
-                                                   const double* __restrict__ C) {
-    __shared__ double sc[kPB][kTU + 2], sr[kPB][kTU + 2];
-    const int bs = min(kPB, n - k0), i0 = blockIdx.y * kTU, j0 = blockIdx.x * kTU, t = threadIdx.x;
-    const int ti = (t >> 4) * 4, tj = t & 15;  // rows ti .. ti + 3, columns tj + 16 y
-    double acc[4][4];
+// the first pivot block's inverse
+__global__ __launch_bounds__(256) void k_gj_first(const double* __restrict__ A, int n, double* __restrict__ D,
+                                                  int* __restrict__ flag) {
+    __shared__ double M[kPB][kPB + 2];
+    __shared__ __attribute__((aligned(16))) double xch[kXch];
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int y = 0; y < 4; ++y) {
-            const int i = min(i0 + ti + x, n - 1), j = min(j0 + tj + 16 * y, n - 1);
-            acc[x][y] = A[(size_t)i * n + j];
-        }
-#pragma unroll
-    for (int w = 0; w < kPB * kTU / 256; ++w) {
-        const int e = t + 256 * w;
-        const int ci = e / kPB, cm = e % kPB;  // C is kPB wide
-        sc[cm][ci] = i0 + ci < n ? C[(size_t)(i0 + ci) * kPB + cm] : 0.0;
-        const int rm = e / kTU, rj = e % kTU;
-        sr[rm][rj] = rm < bs && j0 + rj < n ? R[(size_t)rm * n + j0 + rj] : 0.0;
-    }
-#pragma unroll
-    for (int y = 0; y < 4; ++y) {
-        const int j = j0 + tj + 16 * y;
-        const bool zero = j >= k0 && j < k0 + bs;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) acc[x][y] = zero ? 0.0 : acc[x][y];
+    for (int u = 0; u < kPB * kPB / 256; ++u) {
+        const int e = threadIdx.x + 256 * u, r = e / kPB, c = e % kPB;
+        const double v = A[(size_t)min(r, n - 1) * n + min(c, n - 1)];
+        M[r][c] = r < n && c < n ? v : (r == c ? 1.0 : 0.0);
     }
     __syncthreads();
-#pragma unroll 4
-    for (int m = 0; m < kPB; ++m) {
-        double u[4], v[4];
+    if (!invert_block(M, xch) && threadIdx.x == 0) *flag = 1;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) u[q] = -sc[m][ti + q], v[q] = sr[m][tj + 16 * q];
+    for (int u = 0; u < kPB * kPB / 256; ++u) {
+        const int e = threadIdx.x + 256 * u;
+        D[e] = M[e / kPB][e % kPB];
+    }
+}
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+// v_mfma_f64_16x16x4: lane l brings row (column) l % 16 of the factors at depth l / 16 and holds
+// column l % 16, rows l / 16 + 4 q of the product.
+// The next pivot block's inverse, by the first workgroup of a step, which forms the block for itself
+// instead of waiting for its tile: the block less (its pivot columns) x (scaled pivot rows).
+__device__ __forceinline__ void next_block(const double* __restrict__ A, int n, int k0, const double* __restrict__ D,
+                                           double* __restrict__ Dn, int* __restrict__ flag, double (*sc)[kTU + 2],
+                                           double (*sr)[kTU + 2], double (*sd)[kPB + 2], double* xch) {
+    const int k1 = k0 + kPB, t = threadIdx.x, w = t >> 6, lane = t & 63, lo = lane & 15, hi = lane >> 4;
+    const int x = 16 * (w >> 1), y = 16 * (w & 1);  // this wave's quarter of the block
+    auto at = [&](int i, int j) { return A[(size_t)min(i, n - 1) * n + min(j, n - 1)]; };
+    f64x4 acc, s = {0, 0, 0, 0};
 #pragma unroll
-        for (int x = 0; x < 4; ++x)
-#pragma unroll
-            for (int y = 0; y < 4; ++y) acc[x][y] = __builtin_fma(u[x], v[y], acc[x][y]);
+    for (int q = 0; q < 4; ++q) {
+        const int i = k1 + x + hi + 4 * q, j = k1 + y + lo;
+        const double v = at(i, j);
+        acc[q] = i < n && j < n ? v : (i == j ? 1.0 : 0.0);
     }
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-        const int i = i0 + ti + x;
-        if (i >= n) continue;
-        const bool prow = i >= k0 && i < k0 + bs;
+    for (int u = 0; u < kPB * kPB / 256; ++u) {  // k1 < n: the pivot block at k0 is whole
+        const int e = t + 256 * u, r = e / kPB, c = e % kPB;
+        const double cv = at(k1 + r, k0 + c), rv = at(k0 + r, k1 + c);
+        sc[c][r] = k1 + r < n ? -cv : 0.0;
+        sr[r][c] = k1 + c < n ? rv : 0.0;
+        sd[c][r] = D[e];
+    }
+    __syncthreads();
 #pragma unroll
-        for (int y = 0; y < 4; ++y) {
-            const int j = j0 + tj + 16 * y;
-            if (j < n) A[(size_t)i * n + j] = prow ? sr[i - k0][tj + 16 * y] : acc[x][y];
+    for (int m = 0; m < kPB; m += 4)
+        s = __builtin_amdgcn_mfma_f64_16x16x4f64(sd[m + hi][x + lo], sr[m + hi][y + lo], s, 0, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sr[x + hi + 4 * q][y + lo] = s[q];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kPB; m += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sc[m + hi][x + lo], sr[m + hi][y + lo], acc, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sd[x + hi + 4 * q][y + lo] = acc[q];
+    __syncthreads();
+    if (!invert_block(sd, xch) && t == 0) *flag = 1;
+#pragma unroll
+    for (int u = 0; u < kPB * kPB / 256; ++u) {
+        const int e = t + 256 * u;
+        Dn[e] = sd[e / kPB][e % kPB];
+    }
+}
+
+// Pivot block k0 with inverse D: B = A after its elimination (workgroups 1 ..: a tile each), Dn =
+// the inverse of the next pivot block (workgroup 0).
+__global__ __launch_bounds__(256) void k_gj_step(const double* __restrict__ A, double* __restrict__ B, int n, int k0,
+                                                 const double* __restrict__ D, double* __restrict__ Dn,
+                                                 int* __restrict__ flag) {
+    __shared__ double sc[kPB][kTU + 2];   // -(pivot columns), by depth
+    __shared__ double sr[kPB][kTU + 2];   // pivot rows, then scaled
+    __shared__ double sd[kPB][kPB + 2];   // D transposed
+    __shared__ __attribute__((aligned(16))) double xch[kXch];
+    if (blockIdx.x == 0) {
+        if (k0 + kPB < n) next_block(A, n, k0, D, Dn, flag, sc, sr, sd, xch);
+        return;
+    }
+    const int tiles = (n + kTU - 1) / kTU, tile = blockIdx.x - 1;
+    const int bs = min(kPB, n - k0), i0 = tile / tiles * kTU, j0 = tile % tiles * kTU, t = threadIdx.x;
+    const int w = t >> 6, lane = t & 63, lo = lane & 15, hi = lane >> 4;
+    f64x4 acc[4];  // rows i0 + 16 w + hi + 4 q, columns j0 + 16 y + lo: the pivot's columns from zero
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = i0 + 16 * w + hi + 4 * q, j = j0 + 16 * y + lo;
+            const double v = A[(size_t)min(i, n - 1) * n + min(j, n - 1)];
+            acc[y][q] = i < n && j < n && !(j >= k0 && j < k0 + bs) ? v : 0.0;
         }
+#pragma unroll
+    for (int u = 0; u < kPB * kTU / 256; ++u) {
+        const int e = t + 256 * u;
+        const int ci = e / kPB, cm = e % kPB;
+        const double c = A[(size_t)min(i0 + ci, n - 1) * n + min(k0 + cm, n - 1)];
+        sc[cm][ci] = i0 + ci < n && cm < bs ? -c : 0.0;
+        const int rm = e / kTU, rj = e % kTU, j = j0 + rj;
+        const double r = A[(size_t)min(k0 + rm, n - 1) * n + min(j, n - 1)];
+        // the pivot's own columns become its inverse: D times the identity
+        sr[rm][rj] = j >= k0 && j < k0 + kPB ? (rm == j - k0 && rm < bs ? 1.0 : 0.0) : rm < bs && j < n ? r : 0.0;
     }
+#pragma unroll
+    for (int u = 0; u < kPB * kPB / 256; ++u) {
+        const int e = t + 256 * u;
+        sd[e % kPB][e / kPB] = D[e];
+    }
+    __syncthreads();
+    {  // wave w scales columns 16 w .. of the pivot rows
+        f64x4 s[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+        for (int m = 0; m < kPB; m += 4) {
+            const double b = sr[m + hi][16 * w + lo];
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+                s[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(sd[m + hi][16 * x + lo], b, s[x], 0, 0, 0);
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sr[16 * x + hi + 4 * q][16 * w + lo] = s[x][q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kPB; m += 4) {
+        const double a = sc[m + hi][16 * w + lo];
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+            acc[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, sr[m + hi][16 * y + lo], acc[y], 0, 0, 0);
+    }
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = i0 + 16 * w + hi + 4 * q, j = j0 + 16 * y + lo;
+            if (i < n && j < n) B[(size_t)i * n + j] = i >= k0 && i < k0 + bs ? sr[i - k0][16 * y + lo] : acc[y][q];
+        }
 }
 
 // Gauss-Jordan inverse with partial pivoting (host)
@@ -260,36 +350,38 @@ int coarse_inverse_dev(hipStream_t st, Hierarchy& H) {
     o.var = L.var;
     o.sigma = L.sigma;
     o.sg = D.sg64;
-    // scratch kept with the hierarchy: R, C, the shift and the flag
-    const size_t panel = (size_t)kPB * n;
+    // scratch kept with the hierarchy: the second buffer, two pivot blocks, the shift and the flag
+    const size_t nn = (size_t)n * n, work = nn + 2 * kPB * kPB + 2;
     if (!H.cinv) {
-        OPF_HIP(hipMalloc((void**)&H.cinv, sizeof(double) * n * n));
-        OPF_HIP(hipMalloc((void**)&H.cwork, sizeof(double) * (2 * panel + 2)));
+        OPF_HIP(hipMalloc((void**)&H.cinv, sizeof(double) * nn));
+        OPF_HIP(hipMalloc((void**)&H.cwork, sizeof(double) * work));
         H.cN = n;
-        H.bytes += sizeof(double) * ((size_t)n * n + 2 * panel + 2);
+        H.bytes += sizeof(double) * (nn + work);
     }
-    double *R = H.cwork, *C = R + panel, *dm = C + panel;
+    double *D0 = H.cwork + nn, *dm = D0 + 2 * kPB * kPB;
     int* flag = (int*)(dm + 1);
+    // the buffers alternate from one pivot block to the next and end on cinv
+    const int blocks = (n + kPB - 1) / kPB;
+    double* buf[2] = {blocks & 1 ? H.cwork : H.cinv, blocks & 1 ? H.cinv : H.cwork};
     auto assemble = [&] {
         if (H.singular) hipLaunchKernelGGL(k_coarse_shift, dim3(1), dim3(1024), 0, st, o, dm);
-        hipLaunchKernelGGL(k_coarse_fill, dim3(n), dim3(256), 0, st, o, H.singular ? (const double*)dm : nullptr, H.cinv);
+        hipLaunchKernelGGL(k_coarse_fill, dim3(n), dim3(256), 0, st, o, H.singular ? (const double*)dm : nullptr, buf[0]);
     };
     int bad = 0;
     OPF_HIP(hipMemsetAsync(flag, 0, sizeof(int), st));
     assemble();
-    const unsigned panels = (unsigned)((n + kPB - 1) / kPB), tiles = (unsigned)((n + kTU - 1) / kTU);
-    for (int k0 = 0; k0 < n; k0 += kPB) {
-        hipLaunchKernelGGL(k_gj_panel, dim3(panels), dim3(256), 0, st, (const double*)H.cinv, n, k0, R, C, flag);
-        hipLaunchKernelGGL(k_gj_update, dim3(tiles, tiles), dim3(256), 0, st, H.cinv, n, k0, (const double*)R,
-                           (const double*)C);
-    }
+    const unsigned tiles = (unsigned)((n + kTU - 1) / kTU);
+    hipLaunchKernelGGL(k_gj_first, dim3(1), dim3(256), 0, st, (const double*)buf[0], n, D0, flag);
+    for (int q = 0; q < blocks; ++q)
+        hipLaunchKernelGGL(k_gj_step, dim3(tiles * tiles + 1), dim3(256), 0, st, (const double*)buf[q & 1], buf[~q & 1], n,
+                           q * kPB, (const double*)(D0 + (q & 1) * kPB * kPB), D0 + (~q & 1) * kPB * kPB, flag);
     OPF_HIP(hipGetLastError());
     OPF_HIP(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, st));
     OPF_HIP(hipStreamSynchronize(st));
     if (!bad) return OPF_OK;
     std::vector<double> A((size_t)n * n), inv;
     assemble();
-    OPF_HIP(hipMemcpyAsync(A.data(), H.cinv, sizeof(double) * A.size(), hipMemcpyDeviceToHost, st));
+    OPF_HIP(hipMemcpyAsync(A.data(), buf[0], sizeof(double) * A.size(), hipMemcpyDeviceToHost, st));
     OPF_HIP(hipStreamSynchronize(st));
     OPF_CHECK(invert_pivoting(A, n, inv), OPF_ERR_ARG, "gmg: singular coarsest operator");
     OPF_HIP(hipMemcpyAsync(H.cinv, inv.data(), sizeof(double) * inv.size(), hipMemcpyHostToDevice, st));
