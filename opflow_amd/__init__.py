@@ -196,6 +196,10 @@ _FN2 = ["pow", "fmod", "remainder", "fdim", "hypot", "atan2", "copysign", "nexta
 _FN_SMOOTH_DELTA, _FN_SMOOTH_HEAVISIDE = 32, 33
 
 
+# nodes of two operands and no value: most of an expression
+_BINARY = frozenset((_N_ADD, _N_SUB, _N_MUL, _N_DIV))
+
+
 def _wrap(v):
     if isinstance(v, Expr):
         return v
@@ -237,21 +241,25 @@ class Expr:
         slot_of = {}
 
         def visit(e):
-            if id(e) in memo:
-                return memo[id(e)]
-            if e.kind == _N_UNKNOWN:  # a set's StencilField placeholder: a = the target's index
+            known = memo.get(id(e))
+            if known is not None:
+                return known
+            kind = e.kind
+            if kind in _BINARY:
+                node = (kind, visit(e.a), visit(e.b), e.dim, 0.0)
+            elif kind == _N_UNKNOWN:  # a set's StencilField placeholder: a = the target's index
                 node = (_N_UNKNOWN, int(e.a), 0, 0, 0.0)
-            elif e.kind == _N_FIELD and unknown is not None and e.field is unknown:
+            elif kind == _N_FIELD and unknown is not None and e.field is unknown:
                 node = (_N_UNKNOWN, 0, 0, 0, 0.0)
-            elif e.kind == _N_FIELD:
+            elif kind == _N_FIELD:
                 key = id(e.field)
                 if key not in slot_of:
                     slot_of[key] = len(fields)
                     fields.append(e.field)
                 node = (_N_FIELD, slot_of[key], 0, 0, 0.0)
-            elif e.kind == _N_CONST:
+            elif kind == _N_CONST:
                 node = (_N_CONST, 0, 0, 0, e.value)
-            elif e.kind == _N_CONV:  # the weights follow the argument as consecutive CONST nodes
+            elif kind == _N_CONV:  # the weights follow the argument as consecutive CONST nodes
                 ia = visit(e.a)
                 ib = len(nodes)
                 for w in e.value:
@@ -260,11 +268,11 @@ class Expr:
             else:
                 ia = visit(e.a)
                 ib = visit(e.b) if e.b is not None else 0
-                dim = visit(e.c) if e.kind == _N_COND else e.dim
-                node = (e.kind, ia, ib, dim, float(e.value) if e.kind in (_N_FLUXLIM, _N_FUNC1) else 0.0)
+                dim = visit(e.c) if kind == _N_COND else e.dim
+                node = (kind, ia, ib, dim, float(e.value) if kind in (_N_FLUXLIM, _N_FUNC1) else 0.0)
+            memo[id(e)] = at = len(nodes)
             nodes.append(node)
-            memo[id(e)] = len(nodes) - 1
-            return memo[id(e)]
+            return at
 
         root = visit(self)
         return nodes, fields, root
@@ -289,10 +297,7 @@ class Equation:
 
 
 def _node_array(nodes):
-    arr = (L.ExprNode * len(nodes))()
-    for i, (k, a, b, d, v) in enumerate(nodes):
-        arr[i].kind, arr[i].a, arr[i].b, arr[i].dim, arr[i].value = k, a, b, d, v
-    return arr
+    return (L.ExprNode * len(nodes))(*nodes)  # (kind, a, b, dim, value), the structure's order
 
 
 # operator kernels (FDMOperators/*.hpp, Interpolator/D1Linear.hpp)

@@ -129,18 +129,22 @@ extern "C" int opf_ctx_set_jit(opf_ctx* c, int mode) {
 }
 
 namespace opf {
-static uint64_t fnv1a(const void* p, size_t n) {
+// key of a program's bytes, eight at a time (a sweep program has kilobytes and is looked up at
+// every sweep); entries are told apart by their bytes
+static uint64_t program_hash(const void* p, size_t n) {
     const unsigned char* b = (const unsigned char*)p;
-    uint64_t h = 1469598103934665603ull;
-    for (size_t i = 0; i < n; ++i) {
-        h ^= b[i];
-        h *= 1099511628211ull;
+    uint64_t h = 1469598103934665603ull ^ (uint64_t)n;
+    for (size_t i = 0; i < n; i += 8) {
+        uint64_t w = 0;
+        std::memcpy(&w, b + i, std::min<size_t>(8, n - i));
+        h = (h ^ w) * 0x9e3779b97f4a7c15ull;
+        h ^= h >> 32;
     }
-    return h ^ (uint64_t)n;
+    return h;
 }
 
 int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool evictable, ProgImage image, int* meta) {
-    uint64_t h = fnv1a(bytes, n);
+    uint64_t h = program_hash(bytes, n);
     for (auto& p : ctx->progs)
         if (p.hash == h && p.bytes == n && p.evictable == evictable && p.image == image &&
             std::memcmp(p.host.data(), bytes, n) == 0) {

@@ -881,12 +881,22 @@ struct Plan {
 std::unordered_map<uint64_t, Plan> g_plans;
 
 uint64_t plan_key(const LoweredProgram& P, int dtype, const SweepArgs& a, int dev, int form) {
-    uint64_t h = 1469598103934665603ULL;
+    // two words of 64 bits at a time, from two states: a program has hundreds of instructions and its
+    // key is formed at every sweep (10 us of bytewise hashing for a flux-form expression)
+    uint64_t h = 1469598103934665603ULL, g = 0x2545f4914f6cdd1dULL;
+    auto mix = [](uint64_t& s, uint64_t w) {
+        s = (s ^ w) * 0x9e3779b97f4a7c15ULL;
+        s ^= s >> 32;
+    };
     for (const Insn& in : P.code) {
-        const int w[4] = {in.op, in.a, in.b, in.c};
-        h = fnv1a64(w, sizeof w, h);
-        if (!(in.op == I_CONST && in.a)) h = fnv1a64(&in.imm, sizeof in.imm, h);
+        mix(h, (uint64_t)(uint32_t)in.op << 32 | (uint32_t)in.a);
+        mix(g, (uint64_t)(uint32_t)in.b << 32 | (uint32_t)in.c);
+        if (in.op != I_CONST || in.a) continue;
+        uint64_t bits;
+        std::memcpy(&bits, &in.imm, 8);
+        mix(h, bits);
     }
+    mix(h, g);
     const int q[8] = {dtype, a.op, a.umask, a.cmask, a.xmask, a.n[2] == 1, a.n[2] % 4, dev * 4 + form};
     h = fnv1a64(q, sizeof q, h);
     for (const FieldArg& f : a.f) {  // the direct form bakes plane strides into its loads

@@ -484,6 +484,7 @@ int lower_tree_set(const opf_expr_node* nodes, int nnodes, int root, opf_field* 
     L.nunknown = nunknown;
     L.unknown_as_field = unknown_as_field;
     L.init();
+    L.code.reserve(256);
     int rc = L.compute_locs();
     OPF_CHECK(rc == OPF_OK, rc, "lowering: malformed tree (children must precede parents, valid field slots)");
     L.emit(root, 0, 0, 0);
@@ -491,8 +492,8 @@ int lower_tree_set(const opf_expr_node* nodes, int nnodes, int root, opf_field* 
     OPF_CHECK(L.maxdepth <= SWEEP_MAX_DEPTH, OPF_ERR_UNSUPPORTED, "expression needs stack depth %d > %d",
               L.maxdepth, SWEEP_MAX_DEPTH);
     OPF_CHECK(L.code.size() < 100000, OPF_ERR_UNSUPPORTED, "expression too large after inlining");
-    out->code = L.code;
-    out->consts = L.consts;
+    out->code = std::move(L.code);
+    out->consts = std::move(L.consts);
     out->maxdepth = L.maxdepth;
     for (int f = 0; f < SWEEP_MAX_FIELDS; ++f)
         for (int d = 0; d < 3; ++d) {
@@ -785,7 +786,7 @@ int upload_sweep(opf_ctx* ctx, const std::vector<Insn>& code, bool evictable, vo
     return OPF_OK;
 }
 
-int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProgram& P, const DagInfo& dag) {
+int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProgram& P, DagInfo dag) {
     hipStream_t st = ctx->stream;
     SweepArgs a = a0;
     OPF_CHECK(P.consts.size() <= (size_t)SWEEP_MAX_CONSTS, OPF_ERR_ARG, "sweep: %zu constant slots",
@@ -801,6 +802,12 @@ int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProg
         // runs the same program on the interpreter (same bits); argument errors stand
         if (rc != OPF_ERR_HIP) return rc;
         (void)hipGetLastError();
+    }
+    if (!a.code) {
+        void* dev = nullptr;
+        OPF_TRY(upload_sweep(ctx, structural_code(P), true, &dev, &dag));
+        a.code = dev;
+        a.ncode = (int)P.code.size();
     }
     if (dag.nslot > 0 && (long long)a.n[0] * a.n[1] < (1LL << 31)) {
         DagArgs g{};
@@ -920,12 +927,7 @@ extern "C" int opf_sweep(const opf_expr_node* nodes, int nnodes, int root, opf_f
         }
         a.out = target;
         a.old = out->data;
-        void* dev = nullptr;
-        DagInfo dag;
-        OPF_TRY(upload_sweep(ctx, structural_code(P), true, &dev, &dag));
-        a.code = dev;
-        a.ncode = (int)P.code.size();
-        OPF_TRY(launch_sweep(ctx, d.dtype, a, P, dag));
+        OPF_TRY(launch_sweep(ctx, d.dtype, a, P));
         if (inplace) std::swap(out->data, out->spare);
     }
     return launch_ghost_fill(out, out->data);

@@ -81,8 +81,9 @@ struct DagInfo {
 // the interpreter's form of a stack program on the device
 int upload_sweep(opf_ctx* ctx, const std::vector<Insn>& code, bool evictable, void** dev, DagInfo* dag);
 // the sweep of program P over the box [a.s, a.s + a.n) on the context's stream, by the
-// engine the context's jit mode selects (interpreter or the compiled kernel of P)
-int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a, const LoweredProgram& P, const DagInfo& dag);
+// engine the context's jit mode selects (interpreter or the compiled kernel of P); a.code: P in the
+// interpreter's form on the device with its dag, or null: uploaded here when the interpreter runs it
+int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a, const LoweredProgram& P, DagInfo dag = {});
 // the compiled kernel of P (hipRTC, cached) and its launch; form 0 = by grid size,
 // 1 = direct (loads from HBM), 2 = staged in LDS where the program allows
 int jit_launch_sweep(hipStream_t st, const LoweredProgram& P, int dtype, const SweepArgs& a, int form = 0);
