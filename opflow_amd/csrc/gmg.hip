@@ -1279,6 +1279,189 @@ __global__ __launch_bounds__(NT) void k2v_up(GOp<T> o, const T* __restrict__ x2,
     }
 }
 
+// ---- the same two launches for small 3-D levels with constant coefficients: cubes of 8 x 8 x 8 cells,
+// a workgroup of 512 each, one cell a thread. Levels between the streaming passes and the coarse tail
+// are bound by launches: they took six of 4 to 5 us (two smoothing sweeps in one, restriction,
+// prolongation, two sweeps), now two of 5.3 and 6.7: 192 x 160 x 128 mixed 2.53 -> 2.45 ms. A missing neighbour
+// is a 0 in LDS, so only D and w / D depend on the boundary.
+constexpr long long K3_MAX = 1 << 18;  // cells of a level: beyond, reading the halos of 12^3 for 8^3 costs more
+constexpr int K3_TS = 8, K3_W1 = K3_TS + 2, K3_W2 = K3_TS + 4, K3_NT = 512;
+
+// the cell of position (x, y, z), in bounds in any case: wrapped on a periodic dim, else clamped and
+// false outside
+template <typename T>
+__device__ __forceinline__ bool k3_cell(const GOp<T>& o, int x, int y, int z, int (&c)[3]) {
+    const bool a = f2_map(x, o.n0, o.per[0], c[0] = x), b = f2_map(y, o.n1, o.per[1], c[1] = y);
+    const bool d = f2_map(z, o.n2, o.per[2], c[2] = z);
+    c[0] = min(max(c[0], 0), o.n0 - 1);
+    c[1] = min(max(c[1], 0), o.n1 - 1);
+    c[2] = min(max(c[2], 0), o.n2 - 1);
+    return a && b && d;
+}
+// D and w / D of a cell
+template <typename T>
+__device__ __forceinline__ void k3_diag(const GOp<T>& o, const int (&c)[3], T w, T& D, T& wd) {
+    const int n[3] = {o.n0, o.n1, o.n2};
+    bool edge = false;
+    D = o.dint;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (o.per[d]) continue;
+        if (c[d] == 0) D += o.a[d] * (o.bfac[d][0] - (T)1), edge = true;
+        if (c[d] == n[d] - 1) D += o.a[d] * (o.bfac[d][1] - (T)1), edge = true;
+    }
+    wd = o.wdi;
+    if (edge) wd = w / D;
+}
+template <typename T, int W>
+__device__ __forceinline__ T k3_apply(const GOp<T>& o, T D, const T* v, int p) {
+    T acc = o.a[0] * v[p - 1];
+    acc += o.a[0] * v[p + 1];
+    acc += o.a[1] * v[p - W];
+    acc += o.a[1] * v[p + W];
+    acc += o.a[2] * v[p - W * W];
+    acc += o.a[2] * v[p + W * W];
+    return D * v[p] - acc;
+}
+__device__ __forceinline__ uint32_t k3_lin(uint32_t s1, uint32_t s2, const int (&c)[3]) {
+    return (uint32_t)c[0] + s1 * (uint32_t)c[1] + s2 * (uint32_t)c[2];
+}
+struct K3Tile {
+    int tx, ty;
+};
+// one sweep on the tile + 1: to = from + w (b - A from) / D; b with stride WB from position pb
+template <typename T, int WB>
+__device__ __forceinline__ void k3_sweep(const GOp<T>& o, T w, int x0, int y0, int z0, const T* from, const T* b, T* to) {
+#pragma unroll
+    for (int q = threadIdx.x; q < K3_W1 * K3_W1 * K3_W1; q += K3_NT) {
+        const int lx = q % K3_W1, ly = q / K3_W1 % K3_W1, lz = q / (K3_W1 * K3_W1);
+        const int p = (lx + 1) + K3_W2 * (ly + 1) + K3_W2 * K3_W2 * (lz + 1);
+        const int pb = WB == K3_W2 ? p : q;
+        int c[3];
+        T D, wd, v = 0;
+        if (k3_cell(o, x0 - 1 + lx, y0 - 1 + ly, z0 - 1 + lz, c)) {
+            k3_diag(o, c, w, D, wd);
+            v = from[p] + wd * (b[pb] - k3_apply<T, K3_W2>(o, D, from, p));
+        }
+        to[q] = v;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(K3_NT) void k3_down(GOp<T> o, const T* __restrict__ b, T* __restrict__ x2o,
+                                                 T* __restrict__ bc, int c0, int c1, int c2, T w, K3Tile kt, Bat bt) {
+    __shared__ T sb[K3_W2 * K3_W2 * K3_W2], s1[K3_W2 * K3_W2 * K3_W2], s2[K3_W1 * K3_W1 * K3_W1];
+    BAT_SLOT(bt);
+    b += vo;
+    x2o += vo;
+    bc += (long long)slot * ((long long)c0 * c1 * c2);
+    const int t = threadIdx.x, tile = blockIdx.x;
+    const int x0 = tile % kt.tx * K3_TS, y0 = tile / kt.tx % kt.ty * K3_TS, z0 = tile / (kt.tx * kt.ty) * K3_TS;
+#pragma unroll
+    for (int p = t; p < K3_W2 * K3_W2 * K3_W2; p += K3_NT) {
+        int c[3];
+        const bool ok = k3_cell(o, x0 - 2 + p % K3_W2, y0 - 2 + p / K3_W2 % K3_W2, z0 - 2 + p / (K3_W2 * K3_W2), c);
+        const T bv = b[k3_lin(o.s1, o.s2, c)];
+        T D, wd;
+        k3_diag(o, c, w, D, wd);
+        sb[p] = ok ? bv : (T)0;
+        s1[p] = ok ? wd * bv : (T)0;
+    }
+    __syncthreads();
+    k3_sweep<T, K3_W2>(o, w, x0, y0, z0, s1, sb, s2);
+    __syncthreads();
+    const int lx = t % K3_TS, ly = t / K3_TS % K3_TS, lz = t / (K3_TS * K3_TS);
+    const int c[3] = {x0 + lx, y0 + ly, z0 + lz};
+    T r = 0;
+    if (c[0] < o.n0 && c[1] < o.n1 && c[2] < o.n2) {
+        const int q = (lx + 1) + K3_W1 * (ly + 1) + K3_W1 * K3_W1 * (lz + 1);
+        T D, wd;
+        k3_diag(o, c, w, D, wd);
+        r = sb[(lx + 2) + K3_W2 * (ly + 2) + K3_W2 * K3_W2 * (lz + 2)] - k3_apply<T, K3_W1>(o, D, s2, q);
+        x2o[k3_lin(o.s1, o.s2, c)] = s2[q];
+    }
+    s1[t] = r;  // free since the sweep
+    __syncthreads();
+    if (t < 64) {  // a coarse cell: the mean of its children's residuals
+        const int ci = t & 3, cj = t >> 2 & 3, ck = t >> 4;
+        T s = 0;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) s += s1[2 * ci + (m & 1) + K3_TS * (2 * cj + (m >> 1 & 1)) + K3_TS * K3_TS * (2 * ck + (m >> 2))];
+        const int I = x0 / 2 + ci, J = y0 / 2 + cj, K = z0 / 2 + ck;
+        if (I < c0 && J < c1 && K < c2) bc[(uint32_t)I + (uint32_t)c0 * ((uint32_t)J + (uint32_t)c1 * K)] = s * (T)0.125;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(K3_NT) void k3_up(GOp<T> o, const T* __restrict__ x2, const T* __restrict__ xc, int c0,
+                                               int c1, int c2, const T* __restrict__ b, T* __restrict__ out, T w,
+                                               K3Tile kt, Bat bt) {
+    constexpr int N2 = K3_W2 * K3_W2 * K3_W2, NP = (N2 + K3_NT - 1) / K3_NT;
+    __shared__ T s3[N2], sb[K3_W1 * K3_W1 * K3_W1], s4[K3_W1 * K3_W1 * K3_W1], sc[K3_TS * K3_TS * K3_TS];
+    BAT_SLOT(bt);
+    x2 += vo;
+    b += vo;
+    out += vo;
+    xc += (long long)slot * ((long long)c0 * c1 * c2);
+    const int t = threadIdx.x, tile = blockIdx.x;
+    const int x0 = tile % kt.tx * K3_TS, y0 = tile / kt.tx % kt.ty * K3_TS, z0 = tile / (kt.tx * kt.ty) * K3_TS;
+    T xv[NP];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+        const int p = min(t + u * K3_NT, N2 - 1);
+        int c[3];
+        const bool ok = k3_cell(o, x0 - 2 + p % K3_W2, y0 - 2 + p / K3_W2 % K3_W2, z0 - 2 + p / (K3_W2 * K3_W2), c);
+        const T v = x2[k3_lin(o.s1, o.s2, c)];
+        xv[u] = ok ? v : (T)0;
+    }
+#pragma unroll
+    for (int q = t; q < K3_W1 * K3_W1 * K3_W1; q += K3_NT) {
+        int c[3];
+        const bool ok = k3_cell(o, x0 - 1 + q % K3_W1, y0 - 1 + q / K3_W1 % K3_W1, z0 - 1 + q / (K3_W1 * K3_W1), c);
+        const T v = b[k3_lin(o.s1, o.s2, c)];
+        sb[q] = ok ? v : (T)0;
+    }
+    {  // the coarse cells under the tile + 2, one more on each side; ghosts folded as k_prolong does
+        const int n[3] = {c0, c1, c2}, at[3] = {x0 / 2 - 2 + (t & 7), y0 / 2 - 2 + (t >> 3 & 7), z0 / 2 - 2 + (t >> 6)};
+        int g[3];
+        T fac = 1;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (!f2_map(at[d], n[d], o.per[d], g[d] = at[d])) fac *= (T)1 - o.bfac[d][at[d] < 0 ? 0 : 1];
+            g[d] = min(max(g[d], 0), n[d] - 1);
+        }
+        sc[t] = fac * xc[(uint32_t)g[0] + (uint32_t)c0 * ((uint32_t)g[1] + (uint32_t)c1 * g[2])];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {  // x3 = x2 + P x_c on the tile + 2
+        const int p = t + u * K3_NT;
+        if (p >= N2) continue;
+        const int l[3] = {p % K3_W2, p / K3_W2 % K3_W2, p / (K3_W2 * K3_W2)}, st[3] = {1, 8, 64};
+        int at = 0, oth[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) at += ((l[d] >> 1) + 1) * st[d], oth[d] = (l[d] & 1) ? st[d] : -st[d];
+        T s = 0;
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+            s += (T)((m & 1 ? .25 : .75) * (m & 2 ? .25 : .75) * (m & 4 ? .25 : .75)) *
+                 sc[at + (m & 1 ? oth[0] : 0) + (m & 2 ? oth[1] : 0) + (m & 4 ? oth[2] : 0)];
+        int c[3];
+        const bool ok = k3_cell(o, x0 - 2 + l[0], y0 - 2 + l[1], z0 - 2 + l[2], c);
+        s3[p] = ok ? xv[u] + s : (T)0;
+    }
+    __syncthreads();
+    k3_sweep<T, K3_W1>(o, w, x0, y0, z0, s3, sb, s4);
+    __syncthreads();
+    const int lx = t % K3_TS, ly = t / K3_TS % K3_TS, lz = t / (K3_TS * K3_TS);
+    const int c[3] = {x0 + lx, y0 + ly, z0 + lz};
+    if (c[0] >= o.n0 || c[1] >= o.n1 || c[2] >= o.n2) return;
+    const int q = (lx + 1) + K3_W1 * (ly + 1) + K3_W1 * K3_W1 * (lz + 1);
+    T D, wd;
+    k3_diag(o, c, w, D, wd);
+    out[k3_lin(o.s1, o.s2, c)] = s4[q] + wd * (sb[q] - k3_apply<T, K3_W1>(o, D, s4, q));
+}
+
 // ---- coarse tail: every level of at most GMG_TAIL_N cells in one workgroup per slot.
 // A V-cycle's coarse levels are tiny and launch-bound (a handful of cells per
 // CU); here one 1024-thread workgroup runs their smoothing sweeps, residual
@@ -1808,6 +1991,10 @@ static bool use_zp(const Hierarchy& H, int l) {
     return H.dim == 3 && !H.var && L.n[0] >= 64 && L.n[1] >= 16 && L.n[2] >= 8 && L.N >= (1 << 18) &&
            zp_grid<double>(L).blocks <= GMG_MAXB && zp_grid<float>(L).blocks <= GMG_MAXB;
 }
+// V(2,2) levels below the finest that the streaming passes do not take run as k3_down / k3_up
+static bool use_k3(const Hierarchy& H, int l) {
+    return H.dim == 3 && !H.var && H.pre == 2 && H.post == 2 && l >= 1 && !use_zp(H, l) && H.host[l].N <= K3_MAX;
+}
 // the fused restriction also needs even extents (children pair up inside a tile and a chunk)
 static bool use_zp_restrict(const Hierarchy& H, int l) {
     const GLevelHost& L = H.host[l];
@@ -2301,6 +2488,18 @@ void ph_vcycle(const Hierarchy& H, hipStream_t st, const int* mask, int l, const
             if (dot_q) up(k2_up<T, TS, NT, true>, dot_q, H.part);  // one partial per block (dot3_parts)
             else up(k2_up<T, TS, NT, false>, (const T*)nullptr, (double*)nullptr);
         });
+        return;
+    }
+    if (use_k3(H, l)) {
+        const GLevelDev& C = H.dev[l + 1];
+        const K3Tile kt{(L.n[0] + K3_TS - 1) / K3_TS, (L.n[1] + K3_TS - 1) / K3_TS};
+        const unsigned G = (unsigned)(kt.tx * kt.ty * ((L.n[2] + K3_TS - 1) / K3_TS));
+        const Bat bt = bat(H, mask, N);
+        hipLaunchKernelGGL(k3_down<T>, dim3(G, B), dim3(K3_NT), 0, st, o, rhs, (T*)D.t, (T*)C.b, C.n[0], C.n[1], C.n[2],
+                           w, kt, bt);
+        ph_vcycle<T>(H, st, mask, l + 1, (const T*)C.b, (T*)C.x);
+        hipLaunchKernelGGL(k3_up<T>, dim3(G, B), dim3(K3_NT), 0, st, o, (const T*)D.t, (const T*)C.x, C.n[0], C.n[1],
+                           C.n[2], rhs, out, w, kt, bt);
         return;
     }
     // Jacobi sweeps ping-pong between `out` and the level temp; start on the
