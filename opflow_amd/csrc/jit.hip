@@ -3,7 +3,7 @@
 // The stack program of a sweep (lower_tree) becomes straight-line HIP source:
 // one named value per instruction, every field and mesh array addressed once
 // per cell, the operations and their order exactly those of the interpreter
-// (sweep_kernel), so results have the same bits. It plays the role of the
+// (sweep_dag_kernel), so results have the same bits. It plays the role of the
 // reference's compile-time expression templates (Expression.hpp:51-65), at
 // run time: the source is compiled for gfx950 with hipRTC (-O3, no FMA
 // contraction, no packed FP32), loaded as a module and cached in the process

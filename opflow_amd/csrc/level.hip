@@ -5,8 +5,7 @@
 // cell itself, slot 1 + 2d + s: its neighbour on side s of dim d, x-fastest over
 // the target's assignable range). Nothing of them is copied to the host: the face
 // coefficients, the per-cell shift, the symmetry and uniformity tests and every
-// coarse level are kernels; the host reads back one small record per level build
-// and the coarsest level (at most 1024 cells) for its dense inverse.
+// coarse level are kernels; the host reads back one small record per level build.
 #include <algorithm>
 #include <cmath>
 
