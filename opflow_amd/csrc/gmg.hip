@@ -721,34 +721,36 @@ __global__ __launch_bounds__(256) void k_prolong(T* __restrict__ xf, const T* __
 }
 
 // (P x_c) at fine cell (i, j, k): the (bi/tri)linear weights of k_prolong's
-// general path, boundary ghosts folded (alpha = 1 - bfac), periodic wrap
+// general path, boundary ghosts folded (alpha = 1 - bfac), periodic wrap; per dim
+// the two coarse cells and weights first, then one straight sum
 template <typename T, int DIM>
-__device__ __forceinline__ T prolong_at(const GOp<T>& o, const T* __restrict__ xc, const int cn[3], int i, int j,
-                                        int k) {
-    const int f[3] = {i, j, k};
-    int par[3], oth[3];
-    for (int d = 0; d < 3; ++d) {
-        par[d] = f[d] >> 1;
-        oth[d] = (f[d] & 1) ? par[d] + 1 : par[d] - 1;
+__device__ __forceinline__ T prolong_at(const GOp<T>& o, const T* xc, const int cn[3], int i, int j, int k) {
+    const int f[3] = {i, j, k}, st[3] = {1, cn[0], cn[0] * cn[1]};
+    int at[3][2];
+    T wt[3][2];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        const int par = f[d] >> 1;
+        int oth = (f[d] & 1) ? par + 1 : par - 1;
+        T fac = 1;
+        if (oth < 0 || oth >= cn[d]) {
+            if (o.per[d]) oth = oth < 0 ? oth + cn[d] : oth - cn[d];
+            else {
+                fac = (T)1 - (oth < 0 ? o.bfac[d][0] : o.bfac[d][1]);
+                oth = par;
+            }
+        }
+        at[d][0] = par * st[d], at[d][1] = oth * st[d];
+        wt[d][0] = (T)0.75, wt[d][1] = (T)0.25 * fac;
     }
     T s = 0;
+#pragma unroll
     for (int m = 0; m < (1 << DIM); ++m) {
-        T wgt = 1, fac = 1;
-        int q[3] = {0, 0, 0};
-        for (int d = 0; d < DIM; ++d) {
-            const bool use_oth = (m >> d) & 1;
-            wgt *= use_oth ? (T)0.25 : (T)0.75;
-            int c = use_oth ? oth[d] : par[d];
-            if (c < 0 || c >= cn[d]) {
-                if (o.per[d]) c = c < 0 ? c + cn[d] : c - cn[d];
-                else {
-                    fac *= (T)1 - o.bfac[d][c < 0 ? 0 : 1];
-                    c = par[d];
-                }
-            }
-            q[d] = c;
-        }
-        s += wgt * fac * xc[(uint32_t)q[0] + (uint32_t)cn[0] * ((uint32_t)q[1] + (uint32_t)cn[1] * q[2])];
+        T wgt = 1;
+        int p = 0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) wgt *= wt[d][(m >> d) & 1], p += at[d][(m >> d) & 1];
+        s += wgt * xc[p];
     }
     return s;
 }
@@ -854,57 +856,43 @@ __device__ __forceinline__ bool f2_map(int g, int n, int per, int& w) {
     return true;
 }
 
-// D and (A v)_c at cell (i, j) of a constant-coefficient 2-D level, the neighbours of v
-// read at LDS offsets +-1 / +-W from c (apply_op's order and boundary folding)
+// D and w / D of a cell of a constant-coefficient 2-D level. A missing neighbour is a 0 in LDS, so
+// nothing else depends on the boundary: the tests of every neighbour in every sweep had made the
+// tiles along the boundary, which a small level's launch waits for, the slowest (FP64 us a launch:
+// k2_down 16 x 16 7.3 -> 6.5, 8 x 8 5.1 -> 4.4; k2_up with prolong_at's straight sum 5.0 -> 4.6).
 template <typename T>
-__device__ __forceinline__ T f2_apply(const GOp<T>& o, int i, int j, const T* v, int c, int W, T& D) {
-    T acc = 0;
-    D = o.sigma;
-    const int cc[2] = {i, j}, nn[2] = {o.n0, o.n1}, st[2] = {1, W};
+__device__ __forceinline__ void f2_diag(const GOp<T>& o, T w, int i, int j, T& D, T& wd) {
+    const int c[2] = {i, j}, n[2] = {o.n0, o.n1};
+    bool edge = false;
+    D = o.dint;
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
-        if (cc[d] > 0 || o.per[d]) {
-            D += o.a[d];
-            acc += o.a[d] * v[c - st[d]];
-        } else {
-            D += o.a[d] * o.bfac[d][0];
-        }
-        if (cc[d] < nn[d] - 1 || o.per[d]) {
-            D += o.a[d];
-            acc += o.a[d] * v[c + st[d]];
-        } else {
-            D += o.a[d] * o.bfac[d][1];
-        }
+        if (o.per[d]) continue;
+        if (c[d] == 0) D += o.a[d] * (o.bfac[d][0] - (T)1), edge = true;
+        if (c[d] == n[d] - 1) D += o.a[d] * (o.bfac[d][1] - (T)1), edge = true;
     }
-    return D * v[c] - acc;
-}
-
-// w r / D at cell (i, j): off the boundary as o.wdi r (the interior scaling of the
-// per-level kernels: no division on the cells of a wave that touches no boundary)
-template <typename T>
-__device__ __forceinline__ T f2_corr(const GOp<T>& o, int i, int j, T r, T D, T w) {
-    if (i > 0 && i < o.n0 - 1 && j > 0 && j < o.n1 - 1) return o.wdi * r;
-    return w * r / D;
+    wd = o.wdi;
+    if (edge) wd = w / D;
 }
 
 // A tile whose region with halo 2 lies inside the level and whose cells are all off
 // the boundary: no wrapped or missing neighbour, D = dint everywhere. Such tiles take
-// the straight-line path (f2_apply_in, prolong_in, o.wdi), which gives the general
+// the straight-line path (D = dint, prolong_in, o.wdi), which gives the general
 // path's bits for those cells; tiles along the boundary take the general path.
 template <typename T, int TS>
 __device__ __forceinline__ bool f2_inner(const GOp<T>& o, int x0, int y0) {
     return x0 >= 3 && y0 >= 3 && x0 + TS + 3 <= o.n0 && y0 + TS + 3 <= o.n1;
 }
 
-// (A v)_c of an interior cell (f2_apply's order, D = dint)
+// (A v)_c of a cell with diagonal D
 template <typename T>
-__device__ __forceinline__ T f2_apply_in(const GOp<T>& o, const T* v, int c, int W) {
+__device__ __forceinline__ T f2_apply(const GOp<T>& o, T D, const T* v, int c, int W) {
     T acc = 0;
     acc += o.a[0] * v[c - 1];
     acc += o.a[0] * v[c + 1];
     acc += o.a[1] * v[c - W];
     acc += o.a[1] * v[c + W];
-    return o.dint * v[c] - acc;
+    return D * v[c] - acc;
 }
 
 // (P x_c) at fine cell (i, j) whose four coarse cells lie inside the coarse level
@@ -923,8 +911,8 @@ __device__ __forceinline__ T prolong_in(const T* __restrict__ xc, int c0, int i,
 // one TS x TS tile of k2_down (IN: f2_inner holds for the tile)
 template <typename T, int TS, bool IN>
 __device__ __forceinline__ void k2_down_tile(const GOp<T>& o, const T* __restrict__ b, T* __restrict__ x2o,
-                                             T* __restrict__ bc, int c0, int c1, T w, int x0, int y0, T* sb, T* s1,
-                                             T* s2) {
+                                             T* __restrict__ bc, int c0, int c1, T w, int x0, int y0,
+                                             T* sb, T* s1, T* s2) {
     constexpr int W2 = TS + 4, W1 = TS + 2;
     // b and x1 = w b / D on the tile + 2
     for (int p = threadIdx.x; p < W2 * W2; p += blockDim.x) {
@@ -939,7 +927,9 @@ __device__ __forceinline__ void k2_down_tile(const GOp<T>& o, const T* __restric
         T bv = 0, x1 = 0;
         if (ok) {
             bv = b[(uint32_t)i + o.s1 * (uint32_t)j];
-            x1 = IN ? o.wdi * bv : f2_corr<T>(o, i, j, bv, diag_const<T, 2>(o, i, j, 0), w);
+            T D, wd = o.wdi;
+            if (!IN) f2_diag(o, w, i, j, D, wd);
+            x1 = wd * bv;
         }
         sb[p] = bv;
         s1[p] = x1;
@@ -950,13 +940,13 @@ __device__ __forceinline__ void k2_down_tile(const GOp<T>& o, const T* __restric
         const int li = p % W1, lj = p / W1, c = (lj + 1) * W2 + li + 1;
         T x2 = 0;
         if (IN) {
-            x2 = s1[c] + o.wdi * (sb[c] - f2_apply_in<T>(o, s1, c, W2));
+            x2 = s1[c] + o.wdi * (sb[c] - f2_apply<T>(o, o.dint, s1, c, W2));
         } else {
             int i, j;
             if (f2_map(x0 - 1 + li, o.n0, o.per[0], i) && f2_map(y0 - 1 + lj, o.n1, o.per[1], j)) {
-                T D;
-                const T ax = f2_apply<T>(o, i, j, s1, c, W2, D);
-                x2 = s1[c] + f2_corr<T>(o, i, j, sb[c] - ax, D, w);
+                T D, wd;
+                f2_diag(o, w, i, j, D, wd);
+                x2 = s1[c] + wd * (sb[c] - f2_apply<T>(o, D, s1, c, W2));
             }
         }
         s2[p] = x2;
@@ -974,14 +964,9 @@ __device__ __forceinline__ void k2_down_tile(const GOp<T>& o, const T* __restric
                 const int li = 2 * ci + di, lj = 2 * cj + dj, i = x0 + li, j = y0 + lj;
                 if (IN || (i < o.n0 && j < o.n1)) {
                     const int c = (lj + 1) * W1 + li + 1;
-                    T ax;
-                    if (IN) {
-                        ax = f2_apply_in<T>(o, s2, c, W1);
-                    } else {
-                        T D;
-                        ax = f2_apply<T>(o, i, j, s2, c, W1, D);
-                    }
-                    s += sb[(lj + 2) * W2 + li + 2] - ax;
+                    T D = o.dint, wd;
+                    if (!IN) f2_diag(o, w, i, j, D, wd);
+                    s += sb[(lj + 2) * W2 + li + 2] - f2_apply<T>(o, D, s2, c, W1);
                     x2o[(uint32_t)i + o.s1 * (uint32_t)j] = s2[c];
                 } else {
                     s += (T)0;
@@ -1013,8 +998,8 @@ __global__ __launch_bounds__(NT) void k2_down(GOp<T> o, const T* __restrict__ b,
 // one TS x TS tile of k2_up (IN: f2_inner holds for the tile)
 template <typename T, int TS, bool DOTS, bool IN>
 __device__ __forceinline__ void k2_up_tile(const GOp<T>& o, const T* __restrict__ x2, const T* __restrict__ xc,
-                                           int c0, int c1, const T* __restrict__ b, T* __restrict__ out, T w,
-                                           const T* __restrict__ q, int x0, int y0, T* s3, T* sb, T* s4, double& d0,
+                                           int c0, int c1, const T* __restrict__ b, T* __restrict__ out,
+                                           T w, const T* __restrict__ q, int x0, int y0, T* s3, T* sb, T* s4, double& d0,
                                            double& d1, double& d2) {
     constexpr int W2 = TS + 4, W1 = TS + 2;
     const int cn[3] = {c0, c1, 1};
@@ -1049,13 +1034,13 @@ __device__ __forceinline__ void k2_up_tile(const GOp<T>& o, const T* __restrict_
         const int li = p % W1, lj = p / W1, c = (lj + 1) * W2 + li + 1;
         T x4 = 0;
         if (IN) {
-            x4 = s3[c] + o.wdi * (sb[p] - f2_apply_in<T>(o, s3, c, W2));
+            x4 = s3[c] + o.wdi * (sb[p] - f2_apply<T>(o, o.dint, s3, c, W2));
         } else {
             int i, j;
             if (f2_map(x0 - 1 + li, o.n0, o.per[0], i) && f2_map(y0 - 1 + lj, o.n1, o.per[1], j)) {
-                T D;
-                const T ax = f2_apply<T>(o, i, j, s3, c, W2, D);
-                x4 = s3[c] + f2_corr<T>(o, i, j, sb[p] - ax, D, w);
+                T D, wd;
+                f2_diag(o, w, i, j, D, wd);
+                x4 = s3[c] + wd * (sb[p] - f2_apply<T>(o, D, s3, c, W2));
             }
         }
         s4[p] = x4;
@@ -1067,14 +1052,9 @@ __device__ __forceinline__ void k2_up_tile(const GOp<T>& o, const T* __restrict_
         if (!IN && (i >= o.n0 || j >= o.n1)) continue;
         const int c = (lj + 1) * W1 + li + 1;
         const T bv = sb[c];
-        T x5;
-        if (IN) {
-            x5 = s4[c] + o.wdi * (bv - f2_apply_in<T>(o, s4, c, W1));
-        } else {
-            T D;
-            const T ax = f2_apply<T>(o, i, j, s4, c, W1, D);
-            x5 = s4[c] + f2_corr<T>(o, i, j, bv - ax, D, w);
-        }
+        T D = o.dint, wd = o.wdi;
+        if (!IN) f2_diag(o, w, i, j, D, wd);
+        const T x5 = s4[c] + wd * (bv - f2_apply<T>(o, D, s4, c, W1));
         const uint32_t t = (uint32_t)i + o.s1 * (uint32_t)j;
         out[t] = x5;
         if (DOTS) {
@@ -1537,39 +1517,6 @@ struct TailCell {
     }
 };
 
-// (P x_c) at cell i of a level (the weights of k_prolong's general path)
-template <typename T, int DIM>
-__device__ __forceinline__ T tail_prolong(const GOp<T>& o, const int i[3], const T* xc, const GOp<T>& oc) {
-    const int cn[3] = {oc.n0, oc.n1, oc.n2}, st[3] = {1, oc.n0, oc.n0 * oc.n1};
-    int at[3][2];
-    T wt[3][2];
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-        const int par = i[d] >> 1;
-        int oth = (i[d] & 1) ? par + 1 : par - 1;
-        T fac = 1;
-        if (oth < 0 || oth >= cn[d]) {
-            if (o.per[d]) oth = oth < 0 ? oth + cn[d] : oth - cn[d];
-            else {
-                fac = (T)1 - (oth < 0 ? o.bfac[d][0] : o.bfac[d][1]);
-                oth = par;
-            }
-        }
-        at[d][0] = par * st[d], at[d][1] = oth * st[d];
-        wt[d][0] = (T)0.75, wt[d][1] = (T)0.25 * fac;
-    }
-    T s = 0;
-#pragma unroll
-    for (int m = 0; m < (1 << DIM); ++m) {
-        T wgt = 1;
-        int p = 0;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) wgt *= wt[d][(m >> d) & 1], p += at[d][(m >> d) & 1];
-        s += wgt * xc[p];
-    }
-    return s;
-}
-
 template <typename T, bool VAR, int DIM>
 __global__ __launch_bounds__(GMG_TAIL_NT) void k_vtail(TailArgs<T> ta, Bat bt) {
     __shared__ T lds[3 * GMG_TAIL_CELLS];
@@ -1653,7 +1600,9 @@ __global__ __launch_bounds__(GMG_TAIL_NT) void k_vtail(TailArgs<T> ta, Bat bt) {
         const TailCell<T, VAR, DIM> k(L.o, t, live, ta.w);
         const T b = live ? Bv(L)[t] : (T)0;
         const T* kept = (ta.pre & 1) ? X(L) : Tv(L);
-        T x = live ? kept[t] + tail_prolong<T, DIM>(L.o, k.i, X(ta.lv[l + 1]), ta.lv[l + 1].o) : (T)0;
+        const GOp<T>& oc = ta.lv[l + 1].o;
+        const int cn[3] = {oc.n0, oc.n1, oc.n2};
+        T x = live ? kept[t] + prolong_at<T, DIM>(L.o, X(ta.lv[l + 1]), cn, k.i[0], k.i[1], k.i[2]) : (T)0;
         // the last sweep reads the second buffer, so that x can take its place at once
         T *cur = (ta.post & 1) ? Tv(L) : X(L), *nxt = (ta.post & 1) ? X(L) : Tv(L);
         for (int m = 0; m < ta.post; ++m) {
