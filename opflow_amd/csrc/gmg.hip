@@ -1691,6 +1691,11 @@ __global__ __launch_bounds__(1024) void k_finish(const double* __restrict__ part
             // after the update's true residual: stop a slot that meets tol (or hit the cap /
             // broke down); else adapt the update threshold to the drift of the recurrence
             const double rr = v[0];
+            // At the residual that rounding allows, replacing r by b - A x while the direction is kept
+            // makes beta arbitrary, and x was seen to leave the solution over a hundred such
+            // iterations (1792 x 1024 FP64 to a tolerance of 1e-10 where 1.2e-10 is reached): a
+            // residual that did not fall starts the directions anew, which never raises the error.
+            if (!(rr < 0.25 * s[S_RREF])) s[S_FRESH] = 1.0;
             s[S_RR] = rr;
             s[S_RREF] = rr;
             if (rr <= s[S_TGT] || s[S_ITS] >= (double)maxit || !isfinite(rr)) {
@@ -1710,11 +1715,13 @@ __global__ __launch_bounds__(1024) void k_finish(const double* __restrict__ part
             s[S_RZ] = v[0];
             s[S_ZMEAN] = singular ? v[2] * invN : 0.0;
             s[S_BETA] = 0.0;
+            s[S_FRESH] = 0.0;
             break;
         case FIN_DOT3: {
             double zq = v[1];
             s[S_ZQ] = zq;
-            s[S_BETA] = s[S_RZ] != 0.0 ? -s[S_ALPHA] * zq / s[S_RZ] : 0.0;
+            s[S_BETA] = s[S_RZ] != 0.0 && s[S_FRESH] == 0.0 ? -s[S_ALPHA] * zq / s[S_RZ] : 0.0;
+            s[S_FRESH] = 0.0;
             s[S_RZ] = v[0];
             s[S_ZMEAN] = singular ? v[2] * invN : 0.0;
         } break;
