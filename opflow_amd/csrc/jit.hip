@@ -55,6 +55,9 @@ const char* const kMathSrc =
 const char* const kPadArgsSrc =
 #include "pad_args.inc"
     ;
+const char* const kGuardSrc =
+#include "guard_device.inc"
+    ;
 #undef OPF_SHARED_SRC
 
 const char* const kOpts[] = {"--offload-arch=gfx950", "-O3", "-ffp-contract=off", "-Xclang", "-target-feature",
@@ -132,7 +135,7 @@ struct Known {
 };
 
 // A cell's program as straight-line code, values <pre><id>. fast: the divisions FP64 can do through a
-// reciprocal, guarded (lo_, hi_: the bounds of the numerators met, see kGuardSrc); else every one as
+// reciprocal, guarded (lo_, hi_: the bounds of the numerators met, guard_device.inc); else every one as
 // a division.
 struct CellGen {
     const LoweredProgram& P;
@@ -288,58 +291,11 @@ struct CellGen {
     }
 };
 
-// The guarded divisions of a generated cell (FP64). opf_cdiv is const_div; it rounds as the division
-// for numerators of 0 or at least 2^-600 by divisors in [2^-102, 2^102], and gives NaN where it
-// overflows or its numerator is not finite. lo_ keeps the least key (magnitude's high word, 0 the
-// largest), hi_ the largest magnitude where a program could drop the NaN; else the cell's value shows
-// it. weno_guarded: weno_kernel with its divisions by h, 3 and 6 as const_div on differences of 0 or
-// at least 2^-600 (so those of its derivatives by 3 and 6 are in range too), rh = 0: h of no known
-// reciprocal, divided by; and its three weights through the reciprocal of their sum, for
-// a_i >= 2^-300 and a sum up to 2^700 (nb_ otherwise). An FP64 division is some 17 issue slots, a
-// const_div 3 and its key 2: WENO53 in two dims at 1000 x 900 cells, of 40 divisions a cell, 29 -> 19 us.
-const char* const kGuardSrc = R"(
-__device__ __forceinline__ unsigned opf_key(double x) {
-    unsigned k; asm("v_lshl_add_u32 %0, %1, 1, -1" : "=v"(k) : "v"(__double2hiint(x))); return k;
-}
-__device__ __forceinline__ double opf_cd(double x, double h, double y) {
-    const double q = x * y; return __builtin_fma(-__builtin_fma(h, q, -x), y, q);
-}
-__device__ __forceinline__ double opf_cdiv(unsigned& lo, double x, double h, double y) {
-    lo = min(lo, opf_key(x)); return opf_cd(x, h, y);
-}
-__device__ __forceinline__ double opf_cdivb(unsigned& lo, int& hi, double x, double h, double y) {
-    lo = min(lo, opf_key(x)); hi = max(hi, __double2hiint(x) & 0x7fffffff); return opf_cd(x, h, y);
-}
-__device__ __forceinline__ double weno_guarded(unsigned& lo, bool& nb, double v0, double v1, double v2, double v3, double v4,
-                                               double v5, double h, double rh, bool up) {
-    double d1 = v1 - v0, d2 = v2 - v1, d3 = v3 - v2, d4 = v4 - v3, d5 = v5 - v4;
-    lo = min(min(min(lo, opf_key(d1)), min(opf_key(d2), opf_key(d3))), min(opf_key(d4), opf_key(d5)));
-    if (rh != 0) { d1 = opf_cd(d1, h, rh); d2 = opf_cd(d2, h, rh); d3 = opf_cd(d3, h, rh); d4 = opf_cd(d4, h, rh); d5 = opf_cd(d5, h, rh); }
-    else { d1 = d1 / h; d2 = d2 / h; d3 = d3 / h; d4 = d4 / h; d5 = d5 / h; nb |= !(__builtin_fabs(h) <= 0x1p100); }
-    if (up) { double t = d1; d1 = d5; d5 = t; t = d2; d2 = d4; d4 = t; }
-    const double c1312 = 13. / 12., y3 = 1. / 3., y6 = 1. / 6.;
-    double ddx1 = opf_cd(d1, 3., y3) - opf_cd(7. * d2, 6., y6) + opf_cd(11. * d3, 6., y6);
-    double ddx2 = opf_cd(-d2, 6., y6) + opf_cd(5. * d3, 6., y6) + opf_cd(d4, 3., y3);
-    double ddx3 = opf_cd(d3, 3., y3) + opf_cd(5. * d4, 6., y6) - opf_cd(d5, 6., y6);
-    double t1 = d1 - 2. * d2 + d3, t2 = d1 - 4. * d2 + 3. * d3;
-    double s1 = c1312 * (t1 * t1) + (t2 * t2) / 4;
-    double t3 = d2 - 2. * d3 + d4, t4 = d2 - d4;
-    double s2 = c1312 * (t3 * t3) + (t4 * t4) / 4.;
-    double t5 = d3 - 2. * d4 + d5, t6 = 3. * d3 - 4. * d4 + d5;
-    double s3 = c1312 * (t5 * t5) + (t6 * t6) / 4.;
-    double m = d1 * d1;
-    double q = d2 * d2; m = m < q ? q : m;
-    q = d3 * d3; m = m < q ? q : m;
-    q = d4 * d4; m = m < q ? q : m;
-    q = d5 * d5; m = m < q ? q : m;
-    const double eps = 1e-6 * m + 1e-99;
-    double e1 = s1 + eps, e2 = s2 + eps, e3 = s3 + eps;
-    double a1 = .1 / (e1 * e1);
-    double a2 = .6 / (e2 * e2);
-    double a3 = .3 / (e3 * e3);
-    const double S = a1 + a2 + a3, y = 1.0 / S;
-    nb |= !(__builtin_fmin(__builtin_fmin(a1, a2), a3) >= 0x1p-300 && S <= 0x1p700);
-    return opf_cd(a1, S, y) * ddx1 + opf_cd(a2, S, y) * ddx2 + opf_cd(a3, S, y) * ddx3;
+// The guarded divisions of a generated cell (guard_device.inc). An FP64 division is some 17 issue slots, a
+// const_div 3 and its key 3: WENO53 in two dims at 1000 x 900 cells, of 40 divisions a cell, 29 -> 19 us.
+const char* const kKeySrc = R"(
+__device__ __forceinline__ unsigned opf_key_bits(int v) {
+    unsigned k; asm("v_lshl_add_u32 %0, %1, 1, -1" : "=v"(k) : "v"(v)); return k;
 }
 )";
 
@@ -359,8 +315,8 @@ int emit_cell(const LoweredProgram& P, int dtype, const SweepArgs& a, int base, 
     if (fast.guarded) s += "    unsigned lo_ = 0xffffffffu; int hi_ = 0; bool nb_ = false;\n";
     s += body + "    " + name + " = v" + std::to_string(res) + ";\n";
     if (fast.guarded) {
-        // 2^-600 as a key, 2^700 as a high word
-        s += "    if (__any(nb_ || lo_ < ((1023u - 600u) << 21) - 1u || hi_ >= (1023 + 700) << 20 || !(fabs(" + name +
+        // 2^700 as a high word
+        s += "    if (__any(nb_ || opf_low(lo_) || hi_ >= (1023 + 700) << 20 || !(fabs(" + name +
              ") < __builtin_inf()))) {\n";
         CellGen slow(P, dtype, false);
         Known kn((size_t)base + P.code.size(), a);
@@ -390,6 +346,7 @@ int gen_source(const LoweredProgram& P, int dtype, int op, int R, const SweepArg
     s += "\n";
     s += kWenoSrc;
     s += kMathSrc;
+    s += kKeySrc;
     s += kGuardSrc;
     {
         char hdr[2048];
@@ -528,6 +485,7 @@ int gen_source_tile(const LoweredProgram& P, int dtype, int op, int RY, bool pla
     s += "\n";
     s += kWenoSrc;
     s += kMathSrc;
+    s += kKeySrc;
     s += kGuardSrc;
     const int TY = kTileNTY * RY;
     char line[2048];
