@@ -44,9 +44,11 @@ OPF_CD_HD float const_div(float x, const ConstDivisor& c) { return (float)((doub
 //   least 2^-602, a difference of two quotients 0 or at least 2^-654 -- far above the 2^-969 below
 //   which the residual would not be exact -- and with |coef| >= 2^-100 the new value is 0 or at least
 //   2^-908, so its magnitude shows in the high word, where the next step's test looks for it.
-//   FP32, T = min(100, 103 + l, 80 + 2 l) for spacings up to 2^-l: a difference is 0 or at least
-//   2^-(T + 23), so its quotient at least 2^-126; a difference of two quotients is 0 or at least
-//   2^-(T + 46) / h, and its quotient at least 2^-126 again: nothing is subnormal.
+//   FP32, T = min(100, 101 + l, 78 + 2 l) for spacings up to 2^-l: a difference is 0 or at least
+//   2^-(T + 25) (a ghost between a wall value and a cell has one or two bits below its cell), so its
+//   quotient at least 2^-126; a difference of two quotients is 0 or at least 2^-(T + 48) / h, and its
+//   quotient at least 2^-126 again: nothing is subnormal.
+// A ghost made from a zero is its side's constant, so the constants are 0 or in the range too.
 // div_key orders the magnitudes (the high words, in FP64) so that 0 is the largest: a minimum over
 // cells below the key of 2^-T means that a nonzero value is smaller.
 constexpr unsigned kDivLow = ((1023u - 500u) << 21) - 1u;
@@ -68,18 +70,28 @@ __device__ __forceinline__ bool div_unsafe(double v) {
 }
 #endif
 
-// the least key of a value in the range of spacings h[0 .. dim - 1]
-inline unsigned div_low(const double* h, int dim, bool f64) {
-    if (f64) return kDivLow;
+// T of FP32 for spacings h[0 .. dim - 1]
+inline int div_exp32(const double* h, int dim) {
     int l = 1000, e;
     for (int d = 0; d < dim; ++d) {
         std::frexp(h[d], &e);  // h < 2^e
         if (-e < l) l = -e;
     }
     int t = 100;
-    if (103 + l < t) t = 103 + l;
-    if (80 + 2 * l < t) t = 80 + 2 * l;
+    if (101 + l < t) t = 101 + l;
+    if (78 + 2 * l < t) t = 78 + 2 * l;
+    return t;
+}
+// the least key of a value in the range of spacings h[0 .. dim - 1]
+inline unsigned div_low(const double* h, int dim, bool f64) {
+    if (f64) return kDivLow;
+    const int t = div_exp32(h, dim);
     return t < -100 ? 0xffffffffu : ((unsigned)(127 - t) << 24) - 1u;
+}
+// a side's constant: the wall's value, or what a slope adds to the cell's
+inline bool div_side(double c, const double* h, int dim, bool f64) {
+    c = std::fabs(c);
+    return c == 0.0 || (f64 ? c >= 0x1p-400 && c <= 0x1p400 : c >= std::ldexp(1.0, -div_exp32(h, dim)));
 }
 
 // the host's side of the range: spacing, coefficient and growth of `steps` steps in `dim` dims

@@ -778,10 +778,9 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
         for (int q = 0; q < d.dim; ++q) {
             a.cd[q].h = (double)a.hh[q];
             a.cd[q].y = 1.0 / a.cd[q].h;
-            for (int s = 0; s < 2; ++s) {  // a boundary's constant is 0 or well inside the range
+            for (int s = 0; s < 2; ++s) {
                 const GhostRule& r = gi.rule[q][s][0];
-                const double c = std::fabs(r.type == 1 ? r.c2 / r.c3 : r.type == 2 ? r.c1 : 0.0);
-                ok &= !f64 || c == 0.0 || (c >= 0x1p-400 && c <= 0x1p400);
+                ok &= div_side(r.type == 1 ? r.c2 / r.c3 : r.type == 2 ? r.c1 : 0.0, m->h, d.dim, f64);
             }
         }
         a.divide = !ok;
