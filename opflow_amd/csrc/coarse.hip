@@ -352,11 +352,11 @@ int coarse_inverse_dev(hipStream_t st, Hierarchy& H) {
     o.sg = D.sg64;
     // scratch kept with the hierarchy: the second buffer, two pivot blocks, the shift and the flag
     const size_t nn = (size_t)n * n, work = nn + 2 * kPB * kPB + 2;
-    if (!H.cinv) {
-        OPF_HIP(hipMalloc((void**)&H.cinv, sizeof(double) * nn));
-        OPF_HIP(hipMalloc((void**)&H.cwork, sizeof(double) * work));
-        H.cN = n;
-        H.bytes += sizeof(double) * (nn + work);
+    H.cN = n;
+    for (auto [buf, count] : {std::pair{&H.cinv, nn}, std::pair{&H.cwork, work}}) {
+        if (*buf) continue;
+        OPF_HIP(hipMalloc((void**)buf, sizeof(double) * count));
+        H.bytes += sizeof(double) * count;
     }
     double *D0 = H.cwork + nn, *dm = D0 + 2 * kPB * kPB;
     int* flag = (int*)(dm + 1);

@@ -2169,7 +2169,9 @@ int gmg_build(opf_ctx* ctx, Hierarchy& H, const GLevelHost& fine, const int per[
         }
     }
     OPF_TRY(coarse_inverse_dev(ctx->stream, H));
-    return hier_vectors(H);
+    OPF_TRY(hier_vectors(H));
+    H.complete = true;
+    return OPF_OK;
 }
 
 int gmg_build_dev(opf_ctx* ctx, Hierarchy& H, const DevLevel& fine, const int per[3], const double alpha[3][2],
@@ -2184,7 +2186,7 @@ int gmg_build_dev(opf_ctx* ctx, Hierarchy& H, const DevLevel& fine, const int pe
     F.var = fine.var;
     F.sigma = fine.sigma;
     // an existing hierarchy of the same layout keeps its buffers (and graph)
-    bool same = !H.dev.empty() && H.var == fine.var && H.precision == precision && H.B == std::max(1, slots);
+    bool same = H.complete && !H.dev.empty() && H.var == fine.var && H.precision == precision && H.B == std::max(1, slots);
     for (int d = 0; d < 3 && same; ++d)
         same &= H.host[0].n[d] == fine.n[d] && H.per[d] == per[d] && H.alpha[d][0] == alpha[d][0] &&
                 H.alpha[d][1] == alpha[d][1];
@@ -2201,6 +2203,7 @@ int gmg_build_dev(opf_ctx* ctx, Hierarchy& H, const DevLevel& fine, const int pe
         for (int d = 0; d < 3; ++d) same &= H.host[0].a[d] == fine.a[d];
         if (same) return OPF_OK;  // constant mode: the same operator
     }
+    H.complete = false;
     if (!same) {
         const int pre = H.pre, post = H.post;
         if (!H.dev.empty()) gmg_free(H);
@@ -2248,7 +2251,9 @@ int gmg_build_dev(opf_ctx* ctx, Hierarchy& H, const DevLevel& fine, const int pe
             to_f32_dev(st, D.N, D.sg64, D.sg32);
         }
     OPF_HIP(hipGetLastError());
-    return coarse_inverse_dev(st, H);
+    OPF_TRY(coarse_inverse_dev(st, H));
+    H.complete = true;
+    return OPF_OK;
 }
 
 void gmg_free(Hierarchy& H) {

@@ -87,6 +87,7 @@ struct Hierarchy {
     int precision = OPF_PREC_FP64;  // V-cycle / inner-Krylov precision
     double omega = 0.8;
     int pre = 2, post = 2;
+    bool complete = false;  // the last build ended well: only then may a rebuild keep the buffers
     std::vector<GLevelHost> host;
     std::vector<GLevelDev> dev;
     // coarsest dense inverse (FP64) and the scratch of its computation
