@@ -333,6 +333,16 @@ bool invert_pivoting(std::vector<double>& A, int n, std::vector<double>& inv) {
 
 }  // namespace
 
+// the second buffer, two pivot blocks, the shift and the flag
+static size_t scratch_count(int n) { return (size_t)n * n + 2 * kPB * kPB + 2; }
+
+void coarse_scratch_free(Hierarchy& H) {
+    if (!H.cwork) return;
+    hipFree(H.cwork);
+    H.cwork = nullptr;
+    H.bytes -= sizeof(double) * scratch_count(H.cN);
+}
+
 int coarse_inverse_dev(hipStream_t st, Hierarchy& H) {
     const GLevelHost& L = H.host.back();
     const GLevelDev& D = H.dev.back();
@@ -350,10 +360,9 @@ int coarse_inverse_dev(hipStream_t st, Hierarchy& H) {
     o.var = L.var;
     o.sigma = L.sigma;
     o.sg = D.sg64;
-    // scratch kept with the hierarchy: the second buffer, two pivot blocks, the shift and the flag
-    const size_t nn = (size_t)n * n, work = nn + 2 * kPB * kPB + 2;
+    const size_t nn = (size_t)n * n;
     H.cN = n;
-    for (auto [buf, count] : {std::pair{&H.cinv, nn}, std::pair{&H.cwork, work}}) {
+    for (auto [buf, count] : {std::pair{&H.cinv, nn}, std::pair{&H.cwork, scratch_count(n)}}) {
         if (*buf) continue;
         OPF_HIP(hipMalloc((void**)buf, sizeof(double) * count));
         H.bytes += sizeof(double) * count;

@@ -2002,6 +2002,17 @@ static long long face_count(const int n[3], int d) {
     return (long long)(n[0] + (d == 0)) * (n[1] + (d == 1)) * (n[2] + (d == 2));
 }
 
+// whether a level of n cells has a coarser one
+static bool can_coarsen(int dim, const int n[3]) {
+    long long N = 1;
+    bool can = true;
+    for (int d = 0; d < dim; ++d) {
+        N *= n[d];
+        can &= n[d] % 2 == 0 && n[d] >= 4;
+    }
+    return can && N > 64;
+}
+
 // the next coarser level's shape and constant-mode coefficients; its variable-mode
 // arrays too when `arrays` (host master copy)
 static void coarsen(const Hierarchy& H, const GLevelHost& F, GLevelHost& C, bool arrays = true) {
@@ -2079,9 +2090,7 @@ static int hier_levels(Hierarchy& H, const GLevelHost& fine, const int per[3], c
     H.host.push_back(fine);
     for (;;) {
         const GLevelHost& F = H.host.back();
-        bool can = F.N > 64;
-        for (int d = 0; d < H.dim; ++d) can &= (F.n[d] % 2 == 0) && F.n[d] >= 4;
-        if (!can) break;
+        if (!can_coarsen(H.dim, F.n)) break;
         GLevelHost C;
         coarsen(H, F, C, arrays);
         H.host.push_back(C);
@@ -2169,6 +2178,7 @@ int gmg_build(opf_ctx* ctx, Hierarchy& H, const GLevelHost& fine, const int per[
         }
     }
     OPF_TRY(coarse_inverse_dev(ctx->stream, H));
+    coarse_scratch_free(H);  // the operator stays: its inverse is not formed again
     OPF_TRY(hier_vectors(H));
     H.complete = true;
     return OPF_OK;
@@ -2893,14 +2903,25 @@ static int poisson_level(const opf_poisson_desc* d, GLevelHost& L, int per[3], d
     return OPF_OK;
 }
 
-extern "C" size_t opf_gmg_footprint(const opf_poisson_desc* d, int precision) {
-    if (!d) return 0;
+size_t opf::hier_footprint(const opf_poisson_desc* d, int precision, int slots) {
     long long N = 1;
-    for (int q = 0; q < d->dim; ++q) N *= d->n[q];
+    int n[3] = {1, 1, 1};
+    for (int q = 0; q < d->dim; ++q) N *= n[q] = d->n[q];
     size_t ts = precision == OPF_PREC_MIXED ? 4 : 8;
     double lv = d->dim == 3 ? 8.0 / 7.0 : 4.0 / 3.0;
-    // 3 vectors per level (x, b, t) + 5/6 Krylov vectors + FP64 residual
-    return (size_t)(N * ts * (3 * lv + 6) + N * 8) + (1 << 20);
+    // 3 vectors per level (x, b, t) + 5/6 Krylov vectors + FP64 residual; 1 MiB a slot for its partial
+    // sums and small arrays, the rest of which the coarsest inverse has
+    const size_t slot = (size_t)(N * ts * (3 * lv + 6) + N * 8) + (1 << 20);
+    while (can_coarsen(d->dim, n))
+        for (int q = 0; q < d->dim; ++q) n[q] /= 2;
+    const size_t cells = std::min<size_t>((size_t)n[0] * n[1] * n[2], 1024), inverse = sizeof(double) * cells * cells;
+    const size_t room = (size_t)slots * ((1 << 20) - sizeof(double) * (GMG_PSTRIDE + 64));
+    // and while the inverse is formed, before the vectors are there, its scratch
+    return std::max(slots * slot + (inverse > room ? inverse - room : 0), 2 * inverse + (1 << 16));
+}
+
+extern "C" size_t opf_gmg_footprint(const opf_poisson_desc* d, int precision) {
+    return d ? hier_footprint(d, precision, 1) : 0;
 }
 
 extern "C" int opf_gmg_create(opf_ctx* ctx, const opf_poisson_desc* d, int precision, opf_gmg** out) {

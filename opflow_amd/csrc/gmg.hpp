@@ -90,7 +90,8 @@ struct Hierarchy {
     bool complete = false;  // the last build ended well: only then may a rebuild keep the buffers
     std::vector<GLevelHost> host;
     std::vector<GLevelDev> dev;
-    // coarsest dense inverse (FP64) and the scratch of its computation
+    // coarsest dense inverse (FP64) and the scratch of its computation (kept in variable mode, where
+    // a rebuild needs it)
     double* cinv = nullptr;
     double* cwork = nullptr;
     int cN = 0;
@@ -146,8 +147,11 @@ void coarsen_dev(hipStream_t st, int dim, const int fn[3], const double* const f
                  const int cn[3], double* const caf[3], double* csg);
 void to_f32_dev(hipStream_t st, long long n, const double* src, float* dst);
 // H.cinv = the dense inverse of the coarsest level from its device coefficients
-// (coarse.hip); ends with a wait for st
+// (coarse.hip); ends with a wait for st. Its scratch (H.cwork) stays until it is freed.
 int coarse_inverse_dev(hipStream_t st, Hierarchy& H);
+void coarse_scratch_free(Hierarchy& H);
+// bytes that a hierarchy of d with that many slots takes at most
+size_t hier_footprint(const opf_poisson_desc* d, int precision, int slots);
 int read_scal(const Hierarchy& H, hipStream_t st);
 // Krylov solve with reliable updates, batched over the slots of H (vectors slot-major).
 // The Krylov vectors and the V-cycle are in precision T; x64 / b64 are the FP64

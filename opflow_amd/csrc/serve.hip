@@ -108,7 +108,7 @@ int slots_for(const opf_srv& s, long long N) {
 }
 
 size_t group_bytes(const opf_poisson_desc& d, int precision, int B, long long N) {
-    return opf_gmg_footprint(&d, precision) * (size_t)B + (size_t)B * N * 16 + 4096;
+    return hier_footprint(&d, precision, B) + (size_t)B * N * 16 + 4096;
 }
 
 void free_group(Group* g) {

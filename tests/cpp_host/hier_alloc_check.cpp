@@ -1,47 +1,12 @@
 // A multigrid hierarchy whose build runs out of device memory, then builds again (no GPU: this program
-// stands in for the HIP calls of the library, memory from the host and kernels as nothing). At every
+// stands in for the HIP calls of the library). At every
 // allocation in turn: the failing build reports it, the next one leaves a hierarchy with all of its
 // buffers, and freeing it leaves none behind.
 #include <cstdio>
-#include <cstdlib>
-#include <cstring>
-#include <set>
 
 #include "gmg.hpp"
+#include "hip_standins.hpp"
 #include "opf_internal.hpp"
-
-static std::set<void*> live;
-static long long calls = 0, fail_at = -1;
-static hipError_t take(void** p, size_t n) {
-    if (calls++ == fail_at) return hipErrorOutOfMemory;
-    live.insert(*p = std::calloc(n, 1));
-    return hipSuccess;
-}
-static hipError_t give(void* p) {
-    if (p && !live.erase(p)) return hipErrorInvalidValue;
-    std::free(p);
-    return hipSuccess;
-}
-extern "C" {
-hipError_t hipMalloc(void** p, size_t n) { return take(p, n); }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return take(p, n); }
-hipError_t hipFree(void* p) { return give(p); }
-hipError_t hipHostFree(void* p) { return give(p); }
-hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memcpy(d, s, n), hipSuccess; }
-hipError_t hipMemset(void* d, int v, size_t n) { return std::memset(d, v, n), hipSuccess; }
-hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
-hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* m, hipStream_t* s) {
-    *g = *b = dim3(1);
-    *m = 0;
-    *s = nullptr;
-    return hipSuccess;
-}
-}
 
 using namespace opf;
 
