@@ -150,11 +150,11 @@ int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool e
             std::memcmp(p.host.data(), bytes, n) == 0) {
             p.used = ++ctx->prog_tick;
             *dev = p.dev;
-            if (meta) std::copy(p.meta, p.meta + 5, meta);
+            if (meta) std::copy(p.meta, p.meta + 7, meta);
             return OPF_OK;
         }
     std::vector<unsigned char> made;
-    int m[5] = {0, 0, 0, 0, 0};
+    int m[7] = {};
     if (image) image(bytes, n, made, m);
     if (evictable) {
         size_t ne = 0;
@@ -177,8 +177,8 @@ int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool e
     const unsigned char* b = (const unsigned char*)bytes;
     ctx->progs.push_back({h, d, n, ++ctx->prog_tick, evictable, std::vector<unsigned char>(b, b + n)});
     ctx->progs.back().image = image;
-    std::copy(m, m + 5, ctx->progs.back().meta);
-    if (meta) std::copy(m, m + 5, meta);
+    std::copy(m, m + 7, ctx->progs.back().meta);
+    if (meta) std::copy(m, m + 7, meta);
     ++ctx->prog_uploads;
     *dev = d;
     return OPF_OK;

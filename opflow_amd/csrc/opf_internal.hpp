@@ -63,8 +63,8 @@ struct opf_ctx {
         bool evictable;
         std::vector<unsigned char> host;
         // how the device's copy was made from the bytes (null: it is them), what its maker says of it
-        void (*image)(const void*, size_t, std::vector<unsigned char>&, int[5]) = nullptr;
-        int meta[5] = {0, 0, 0, 0, 0};
+        void (*image)(const void*, size_t, std::vector<unsigned char>&, int[7]) = nullptr;
+        int meta[7] = {};
     };
     static constexpr size_t kMaxPrograms = 1024;
     std::vector<ProgEntry> progs;
@@ -127,7 +127,7 @@ int gen_bumps_grid_dev(hipStream_t st, int dim, const int n[3], uint64_t seed, i
 // so the cache may free it later, after a drain of the context's stream
 // image (optional) makes the device's form of the bytes, when they are uploaded, and what a launch
 // needs to know of it (meta)
-using ProgImage = void (*)(const void* bytes, size_t n, std::vector<unsigned char>& out, int meta[5]);
+using ProgImage = void (*)(const void* bytes, size_t n, std::vector<unsigned char>& out, int meta[7]);
 int upload_program(opf_ctx* ctx, const void* bytes, size_t n, void** dev, bool evictable = false,
                    ProgImage image = nullptr, int* meta = nullptr);
 

@@ -637,7 +637,8 @@ struct DagArgs {
 // row). Bound by a wave's own latencies where a CU has few of them, by LDS and instruction issue
 // elsewhere. us per sweep with its ghost fill, stack program -> bundles: QUICK transport 96 x 80 cells
 // FP64 85 -> 29 (77 -> 20 the kernel), 24 x 20 85 -> 28, 500^2 163 -> 79, 1500^2 1005 -> 538; FTCS
-// 96 x 80 22 -> 16, 1500^2 208 -> 95; WENO 500^2 22 -> 19; u 2 + 1, 1500^2 28 -> 24 (FP32 19 -> 20).
+// 96 x 80 22 -> 16, 1500^2 208 -> 95; WENO 500^2 22 -> 19; u 2 + 1, 1500^2 28 -> 24 (FP32
+// 19 -> 22: such launches run the stack program, see launch_sweep).
 template <typename T>
 __global__ __launch_bounds__(256) void sweep_dag_kernel(SweepArgs a, DagArgs g) {
     extern __shared__ __attribute__((aligned(16))) char dag_lds[];
@@ -771,18 +772,19 @@ void uniform_spacing(const opf_mesh* m, int dtype, SweepArgs& a) {
 }
 
 int upload_sweep(opf_ctx* ctx, const std::vector<Insn>& code, bool evictable, void** dev, DagInfo* dag) {
-    const ProgImage image = [](const void* bytes, size_t n, std::vector<unsigned char>& out, int meta[5]) {
+    const ProgImage image = [](const void* bytes, size_t n, std::vector<unsigned char>& out, int meta[7]) {
         DagInfo d;
         const Insn* c = (const Insn*)bytes;
         if (!DagBuilder().build(c, n / sizeof(Insn), out, d)) {
             d = DagInfo{};
             out.assign((const unsigned char*)bytes, (const unsigned char*)bytes + n);
         }
-        meta[0] = d.nload, meta[1] = d.nuni, meta[2] = d.nbundle, meta[3] = d.nslot, meta[4] = d.result;
+        const int m[7] = {d.nload, d.nuni, d.nbundle, d.nslot, d.result, d.cost, d.stack};
+        std::copy(m, m + 7, meta);
     };
-    int m[5];
+    int m[7];
     OPF_TRY(upload_program(ctx, code.data(), code.size() * sizeof(Insn), dev, evictable, image, m));
-    *dag = {m[0], m[1], m[2], m[3], m[4]};
+    *dag = {m[0], m[1], m[2], m[3], m[4], m[5], m[6]};
     return OPF_OK;
 }
 
@@ -809,7 +811,14 @@ int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProg
         a.code = dev;
         a.ncode = (int)P.code.size();
     }
-    if (dag.nslot > 0 && (long long)a.n[0] * a.n[1] < (1LL << 31)) {
+    // FP32 with waves enough to hide their latencies: an instruction of the stack program takes half a
+    // bundle of one operation, a quarter of one of several, so it runs the programs that the bundles do
+    // not shorten by as much. 256^3 cells, us, bundles / stack: u w + 1.5 (5 instructions, 2 bundles) 149 /
+    // 106, d/dx (9, 4) 198 / 154; d2/dx2 (33, 8) 412 / 448, the heat step (71, 11) 604 / 912. The line
+    // in cells: 512^2 even, 700^2 d/dx 13.5 / 11.5. FP64, where an operand of the stack is twice the
+    // LDS: bundles always (u w + 1.5 200 / 248).
+    const bool dense = dtype == OPF_F32 && cells >= 24LL * 64 * ctx->cus;
+    if (dag.nslot > 0 && (long long)a.n[0] * a.n[1] < (1LL << 31) && !(dense && 2 * dag.cost + 4 >= a.ncode)) {
         DagArgs g{};
         g.n0 = FastDiv((uint32_t)a.n[0]);
         for (int f = 0; f < SWEEP_MAX_FIELDS; ++f) {
@@ -833,6 +842,7 @@ int launch_sweep(opf_ctx* ctx, int dtype, const SweepArgs& a0, const LoweredProg
         OPF_HIP(hipGetLastError());
         return OPF_OK;
     }
+    a.code = (const char*)a.code + dag.stack;
     dim3 grid((a.n[0] + 63) / 64, (a.n[1] + 3) / 4, a.n[2]);
     if (dtype == OPF_F64) hipLaunchKernelGGL(sweep_kernel<double>, grid, dim3(64, 4), 0, st, a);
     else hipLaunchKernelGGL(sweep_kernel<float>, grid, dim3(64, 4), 0, st, a);

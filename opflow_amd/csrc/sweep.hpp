@@ -74,9 +74,10 @@ int lower_tree(const opf_expr_node* nodes, int nnodes, int root, opf_field* cons
 int lower_tree_set(const opf_expr_node* nodes, int nnodes, int root, opf_field* const* fields, int nfields,
                    const opf_mesh* mesh, const int* unknown_slots, int nunknown, LoweredProgram* out,
                    bool unknown_as_field = false);
-// a sweep program in the interpreter's form (sweep_dag.hpp); nslot = 0: as the stack program
+// a sweep program in the interpreter's form (sweep_dag.hpp); nslot = 0: as the stack program. cost: the
+// bundles, one of several operations counted twice; stack: the bytes before the stack program
 struct DagInfo {
-    int nload = 0, nuni = 0, nbundle = 0, nslot = 0, result = 0;
+    int nload = 0, nuni = 0, nbundle = 0, nslot = 0, result = 0, cost = 0, stack = 0;
 };
 // the interpreter's form of a stack program on the device
 int upload_sweep(opf_ctx* ctx, const std::vector<Insn>& code, bool evictable, void** dev, DagInfo* dag);

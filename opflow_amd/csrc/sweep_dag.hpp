@@ -20,7 +20,7 @@ namespace opf {
 constexpr int DAG_W = 4;
 constexpr int DAG_LOADS = 16;      // loads in flight
 // Values a lane keeps at a time (LDS); a program that needs more runs as a stack program. 96 hold
-// every expression of the examples, at 48 KB a wave in FP64.
+// every expression of the examples, at 48 KB a wave in FP64. The image ends with the stack program.
 constexpr int DAG_MAX_SLOTS = 96;
 constexpr int DAG_MAX_UNI = 96;    // constants (one copy a wave)
 
@@ -200,6 +200,7 @@ struct DagBuilder {
         info.nbundle = (int)bundles.size();
         info.nslot = std::max(nslot, 1);
         info.result = word[root];
+        for (const DagBundle& b : bundles) info.cost += b.count > 1 ? 2 : 1;
         loads.resize(dag_loads(info.nload), loads.empty() ? DagLoad{} : loads[0]);  // a last group repeats one
         bundles.push_back(DagBundle{});  // read ahead of the last one
         out.clear();
@@ -209,6 +210,8 @@ struct DagBuilder {
         put(bundles.data(), bundles.size() * sizeof(DagBundle));
         put(loads.data(), loads.size() * sizeof(DagLoad));
         put(unis.data(), unis.size() * sizeof(DagUni));
+        info.stack = (int)out.size();
+        put(code, n * sizeof(Insn));
         return true;
     }
 };
