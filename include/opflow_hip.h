@@ -256,8 +256,9 @@ int opf_sweep(const opf_expr_node* nodes, int nnodes, int root, opf_field* const
 int opf_ftcs(opf_field* u, double coef, int nsteps);
 /* Same update with the temporal-blocking choice made by the caller:
  * tblock = 1 runs one launch per step; tblock = 0 lets the library fuse steps
- * inside one launch where it can (2-D: 4 to 24 steps per launch by grid size, any BC, all of
- * up to 128 when one workgroup holds the grid; 3-D: 3 steps per launch, the ghosts of non-periodic sides rebuilt inside the launch),
+ * inside one launch where it can (2-D: 2 to 62 steps by grid size, all of up to 128 when one
+ * workgroup holds the grid, any BC, the steps spread evenly over the launches; 3-D: 3 steps per
+ * launch, the ghosts of non-periodic sides rebuilt inside the launch; opf_ftcs_plan tells),
  * which is what opf_ftcs does. Results are bit-identical either way.       */
 int opf_ftcs_blocked(opf_field* u, double coef, int nsteps, int tblock);
 /* Launch plan of opf_ftcs_blocked(u, ., nsteps, tblock) without running it:

@@ -264,7 +264,7 @@ __device__ __forceinline__ void strip_ghost_plane(const SideRule<T>* side, const
 // 2 with const_div, over the share of the region that is tile), the barrier and the launch the
 // small ones. Against LDS tiles of the values (32 x 32, 4 steps; 8 x 8, 5 steps): 256^2 Dirichlet
 // 1.61 -> 0.75 us a step, 1500 x 1100 with const_div 12.3 -> 4.5 (0.13 -> 0.37 T cell-updates/s),
-// 4096^2 periodic 42 -> 10.1 (0.40 -> 1.66 T/s).
+// 4096^2 periodic 42 -> 11.0 (0.40 -> 1.53 T/s).
 template <typename T, int MODE, int XW, int RW, int NW>
 __global__ __launch_bounds__(64 * NW) void ftcs2d_strip_kernel(const T* __restrict__ in, T* __restrict__ out,
                                                                FtcsArgs<T> a, int nt, int tx, int ty) {
@@ -644,24 +644,36 @@ __global__ __launch_bounds__(64 * NW) void ftcs3d_strip_kernel(const T* __restri
 
 // Launches of the 2-D kernel: the region (cells in x per lane, rows per wave, waves), the steps per
 // launch and the tile that is left of the region. Per step a launch costs
-//   S2_LAUNCH / nt + max(alone, tiles / CUs * shared)
+//   S2_LAUNCH / nt + max(alone, tiles / CUs * shared + traffic / nt)
 // with the measured time of one step of one workgroup when it has a CU to itself (alone: the
 // barrier and the waves' latency) and when several share one (shared: instruction issue), about
-// 1.8 times that with const_div. More steps a launch save launches and lose tile. FP64, us per
-// step: 256^2 periodic 64 x 32 region with 12 steps 0.65 (64 x 64, 24 steps: 0.71); 700^2 64 x 64,
-// 10 steps 2.0 (64 x 32, 6: 2.1); 4096^2 128 x 64, 10 steps 10.1 (64 x 64: 14.0, 64 x 32: 19.8).
-// With const_div the 128 x 64 region holds too few waves (117 registers): 2000^2 7.7 against 7.3.
+// 1.8 times that with const_div, and the regions read and tiles written at the rate of the last-level
+// cache or of memory, where both time levels are past the L2s (on a grid within them shared has it).
+// More steps a launch save launches and traffic and lose tile. FP64, us per step: 256^2 64 x 32 region
+// with 12 steps 0.80 (64 x 64, 20 steps: 1.00); 700^2, const_div, 64 x 64, 10 steps 1.89 (64 x 32, 6:
+// 1.99); 4096^2 periodic 128 x 64, 10 steps 10.0 (64 x 64, 8: 12.5). With const_div the 128 x 64 region
+// holds too few waves (117 registers): 2000^2 7.7 against 7.3.
+// What the rule takes, without the traffic -> with it, and the best of a sweep over regions and 2 to 24
+// steps: 4096^2 FP64 17.4 -> 11.0, best 10.0; 8192^2 125.7 -> 42.6, 40.8; 16384^2 510 -> 170, 161; 8192^2
+// FP32 64.7 -> 28.4, 25.9; const_div 3000^2 16.3 -> 12.1, 12.1; 8000^2 112 -> 82, 82.
 constexpr int S2_XW[3] = {1, 1, 2}, S2_RW[3] = {4, 8, 8}, S2_NW[3] = {8, 8, 8};
 constexpr double S2_ALONE[3] = {0.33, 0.55, 1.3}, S2_SHARED[3] = {0.31, 0.49, 0.74}, S2_LAUNCH = 4.2;
+constexpr double S2_L2 = 32 << 20, S2_LLC = 256 << 20;  // bytes
+constexpr double S2_LLC_RATE = 9.6e6, S2_HBM_RATE = 5.6e6;  // bytes a us, measured on these launches
+constexpr double S2_F32 = 0.65;  // shared of FP32, where the traffic is counted apart
 constexpr int S2_MOST = 128;  // steps a launch takes at most (the range const_div is given, div_range)
 struct Strip2d {
     int cfg = 0;
     int nt = 1, tx = 1, ty = 1;  // steps, tile
 };
 
-Strip2d strip_plan(const int n[3], const int per[3], int nsteps, int tblock, bool div, int cus) {
+// vsize: bytes of a value
+Strip2d strip_plan(const int n[3], const int per[3], int nsteps, int tblock, bool div, int cus, size_t vsize) {
     Strip2d best;
     double cost = 0;
+    const double level = (double)n[0] * n[1] * vsize;
+    const bool past = 2 * level > S2_L2;
+    const double rate = 2 * level <= S2_LLC ? S2_LLC_RATE : S2_HBM_RATE, issue = vsize == 4 ? S2_F32 : 1.0;
     for (int c = 0; c < (div ? 2 : 3); ++c) {
         const int wx = 64 * S2_XW[c], wy = S2_RW[c] * S2_NW[c];
         const bool allx = !per[0] && n[0] + 2 <= wx, ally = !per[1] && n[1] + 3 <= wy;  // no halo in that dim
@@ -670,8 +682,9 @@ Strip2d strip_plan(const int n[3], const int per[3], int nsteps, int tblock, boo
         for (int nt = tblock == 1 ? 1 : std::min(2, most);;) {
             const int tx = allx ? n[0] : wx - 2 * nt, ty = ally ? n[1] : wy - 2 * nt;
             const double tiles = (double)((n[0] + tx - 1) / tx) * ((n[1] + ty - 1) / ty);
-            const double t = S2_LAUNCH / nt +
-                             (div ? 1.8 : 1.0) * std::max(S2_ALONE[c], tiles / cus * S2_SHARED[c]);
+            const double f = div ? 1.8 : 1.0, shared = f * tiles / cus * S2_SHARED[c];
+            const double busy = past ? shared * issue + (tiles * wx * wy * vsize + level) / (rate * nt) : shared;
+            const double t = S2_LAUNCH / nt + std::max(f * S2_ALONE[c], busy);
             if (cost == 0 || t < cost) {
                 cost = t;
                 best.cfg = c;
@@ -829,7 +842,7 @@ int ftcs_t(opf_field* f, double coef, int nsteps, int tblock, void* ext_spare = 
         }
         nxt = f->spare;
     }
-    const Strip2d p2 = d.dim == 2 ? strip_plan(a.n, a.per, nsteps, tblock, !pow2, f->ctx->cus) : Strip2d{};
+    const Strip2d p2 = d.dim == 2 ? strip_plan(a.n, a.per, nsteps, tblock, !pow2, f->ctx->cus, sizeof(T)) : Strip2d{};
     bool ghosts_stale = false;  // the 3-D blocked kernel writes interior cells only
     for (int it = 0; it < nsteps;) {
         const T* in = (const T*)cur;
@@ -935,7 +948,7 @@ extern "C" int opf_ftcs_plan(const opf_field* u, int nsteps, int tblock, int* la
     *max_steps = 0;
     bool pow2 = true;
     for (int q = 0; q < d.dim; ++q) pow2 &= is_pow2(u->mesh->h[q]);
-    const int nt = d.dim == 2 && nsteps > 0 ? strip_plan(n, per, nsteps, tblock, !pow2, u->ctx->cus).nt : 0;
+    const int nt = d.dim == 2 && nsteps > 0 ? strip_plan(n, per, nsteps, tblock, !pow2, u->ctx->cus, dtype_size(d.dtype)).nt : 0;
     for (int it = 0; it < nsteps;) {
         const int k = d.dim == 2 ? std::min(nt, nsteps - it)
                                  : launch_steps3(nsteps - it, tblock);
