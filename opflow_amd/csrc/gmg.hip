@@ -1694,7 +1694,11 @@ __global__ __launch_bounds__(1024) void k_finish(const double* __restrict__ part
             // At the residual that rounding allows, replacing r by b - A x while the direction is kept
             // makes beta arbitrary, and x was seen to leave the solution over a hundred such
             // iterations (1792 x 1024 FP64 to a tolerance of 1e-10 where 1.2e-10 is reached): a
-            // residual that did not fall starts the directions anew, which never raises the error.
+            // residual that is not half of the last update's starts the directions anew. Updates come
+            // when the recurrence fell by 10 or more, or to the tolerance, so such a residual is one
+            // whose recurrence had lost it; a solve that converges slowly keeps its directions: of 300
+            // (spacings 1 : 50, coefficients over 1e6, 5 to 400 iterations) one had another count, 368
+            // where the direction kept ran to the cap of 400.
             if (!(rr < 0.25 * s[S_RREF])) s[S_FRESH] = 1.0;
             s[S_RR] = rr;
             s[S_RREF] = rr;

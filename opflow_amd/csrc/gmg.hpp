@@ -191,7 +191,7 @@ enum {
     S_MEAN,  // scratch mean (singular projections)
     S_RREC,  // recurrence residual^2 when the last update was decided
     S_DLT2,  // current update threshold: update when rr < S_DLT2 * S_RREF
-    S_FRESH,  // 1: the next direction starts from z alone (a true residual that did not fall)
+    S_FRESH,  // 1: the next direction starts from z alone (a true residual above half of the last update's)
     S_N
 };
 static_assert(S_N <= GMG_SSTRIDE, "scalars per slot");
