@@ -652,7 +652,7 @@ __global__ __launch_bounds__(64 * NW) void ftcs3d_strip_kernel(const T* __restri
 // More steps a launch save launches and traffic and lose tile. FP64, us per step: 256^2 64 x 32 region
 // with 12 steps 0.80 (64 x 64, 20 steps: 1.00); 700^2, const_div, 64 x 64, 10 steps 1.89 (64 x 32, 6:
 // 1.99); 4096^2 periodic 128 x 64, 10 steps 10.0 (64 x 64, 8: 12.5). With const_div the 128 x 64 region
-// holds too few waves (117 registers): 2000^2 7.7 against 7.3.
+// holds too few waves (117 registers): 2000^2, 4 steps, 7.7 against 7.3.
 // What the rule takes, without the traffic -> with it, and the best of a sweep over regions and 2 to 24
 // steps: 4096^2 FP64 17.4 -> 11.0, best 10.0; 8192^2 125.7 -> 42.6, 40.8; 16384^2 510 -> 170, 161; 8192^2
 // FP32 64.7 -> 28.4, 25.9; const_div 3000^2 16.3 -> 12.1, 12.1; 8000^2 112 -> 82, 82.
